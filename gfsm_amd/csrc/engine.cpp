@@ -298,10 +298,12 @@ Status upload_graph(Ctx &ctx, const HostGraph &g, DevGraph *&out)
 
 Status plan_for(const HostGraph &data, const HostGraph &query, const gfsm_match_opts &o, Plan &plan)
 {
-    if (!(o.flags & GFSM_ORDER_COST)) return plan_query(query, plan);
-    if (o.root_lo || o.root_hi)
+    const bool by_cost = o.flags & GFSM_ORDER_COST;
+    if (by_cost && (o.root_lo || o.root_hi))
         return Status::err(GFSM_ERR_ARG, "root windows refer to the reference order's root; not with GFSM_ORDER_COST");
-    return plan_query(query, plan, &data);
+    Status st = plan_query(query, plan, by_cost ? &data : nullptr);
+    if (st.good()) set_injectivity(data, plan);
+    return st;
 }
 
 const uint2 *dense_segments_cached(DevGraph &dg, uint32_t rel)

@@ -160,6 +160,17 @@ bool layout_ok(const HostGraph &g)
     return !bad;
 }
 
+bool any_loop(const HostGraph &g)
+{
+    std::atomic<bool> loops{false};
+    parallel_for(g.V, [&](uint64_t b, uint64_t e) {
+        for (uint64_t x = b; x < e; x++)
+            for (uint32_t p = g.dir[g.dir_ptr[x]].beg; p < g.dir[g.dir_ptr[x + 1]].beg; p++)
+                if (g.nbr[p] == x) loops = true;
+    });
+    return loops;
+}
+
 }  // namespace
 
 Status save_bin(const HostGraph &g, const char *path)
@@ -223,6 +234,7 @@ Status load_bin(const char *path, HostGraph *&out)
     if (!ok) return Status::err(GFSM_ERR_INVALID_DATA, "truncated graph image");
     if (payload_checksum(*g) != h.checksum) return Status::err(GFSM_ERR_INVALID_DATA, "graph image checksum mismatch");
     if (!layout_ok(*g)) return Status::err(GFSM_ERR_INVALID_DATA, "graph image layout is inconsistent");
+    g->has_loops = any_loop(*g);
     out = g.release();
     return Status::ok();
 }

@@ -55,6 +55,7 @@ struct HostGraph {
     std::vector<uint64_t> rel_off;
     std::vector<uint32_t> rel_vtx, rel_beg, rel_cnt;
     uint32_t max_degree = 0;
+    bool has_loops = true;  // some entry x -> x (whatever its relation)
     uint64_t nent() const { return nbr.size(); }
     uint64_t ndir() const { return dir.empty() ? 0 : dir.size() - 1; }
 
@@ -106,6 +107,8 @@ struct Plan {
     std::vector<uint32_t> header, requirements;  // reference layout (HnGPU.cuh:41-58)
     QueryPlanDev dev;                       // what the kernels read
 };
+// Fill the plan's injectivity masks (DepthPlanDev::inj) for a data graph.
+void set_injectivity(const HostGraph &data, Plan &plan);
 // The reference's matching order, or with `by_cost` (a data graph) the
 // order chosen from its relation statistics.
 Status plan_query(const HostGraph &query, Plan &out, const HostGraph *by_cost = nullptr);

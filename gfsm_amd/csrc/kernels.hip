@@ -604,12 +604,12 @@ DEV uint32_t pick_row_or(RP rows, uint32_t row, uint32_t c, uint32_t d, uint32_t
 // `dyn` is the dynamic LDS: the node-start bitmap, the per-position generator
 // base and a pool of pool_words words that stages, per frontier node of the
 // tile, the checked ancestor segments, the next generator segment and the
-// placed vertices, as far as they fit.  LAST_COUNT adds its embeddings and
-// digest to the thread's accumulators; the other kinds write their output.
+// placed vertices, as far as they fit.  `inj` is the depth's injectivity mask
+// (a scalar).  LAST_COUNT adds its embeddings and digest to the thread's accumulators; the other kinds write their output.
 template <uint32_t KIND, uint32_t I, class DP, class CP>
 DEV void expand_tile(const DevGraphView &g, const DP &dp, CP col, CP dcol,
                      const StepIO &io, uint64_t lt, uint64_t gt, uint64_t gt0, const ScanWS &ws, uint32_t ep,
-                     uint32_t pool_words, TileShared<I> &sh, unsigned char *dyn, uint64_t &acc_cnt,
+                     uint32_t inj, uint32_t pool_words, TileShared<I> &sh, unsigned char *dyn, uint64_t &acc_cnt,
                      uint64_t &acc_h0, uint64_t &acc_h1, bool tickets = true)
 {
     constexpr uint32_t T = kTile, TC = kTile * I, NW = TC / 64;
@@ -839,9 +839,11 @@ DEV void expand_tile(const DevGraphView &g, const DP &dp, CP col, CP dcol,
     // pointer that could be either would turn the LDS reads into flat loads,
     // which take the vector-memory path.
     auto tail = [&](auto rows) {
-        // Phase 2: injectivity against the node's placed vertices, one placed
-        // column at a time for all items, so I reads are in flight together.
-        for (uint32_t kk = 0; kk < d; kk++) {
+        // Phase 2: injectivity against the placed vertices a candidate of this
+        // depth can coincide with, one placed column at a time for all items,
+        // so I reads are in flight together.
+        for (uint32_t im = inj; im; im &= im - 1) {
+            const uint32_t kk = (uint32_t)__builtin_ctz(im);
             uint32_t pv[I];
 #pragma unroll
             for (uint32_t k = 0; k < I; k++) pv[k] = rows[jj[k] * d + kk];
@@ -1094,7 +1096,7 @@ __global__ __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(4))) void
         for (TileDeal dl; dl.tile() < a.io.ntiles; dl.next()) {
             const uint64_t t = dl.tile();
             __syncthreads();  // the previous tile's readers of the tile LDS are done
-            expand_tile<KIND, I>(a.g, a.dp, a.col, a.dcol, a.io, t, t, 0, a.ws, ep, a.pool_words, sh, smem, acc_cnt,
+            expand_tile<KIND, I>(a.g, a.dp, a.col, a.dcol, a.io, t, t, 0, a.ws, ep, a.dp.inj, a.pool_words, sh, smem, acc_cnt,
                                  acc_h0, acc_h1, false);
         }
     } else {
@@ -1102,7 +1104,7 @@ __global__ __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(4))) void
         for (;;) {
             const uint64_t t = tickets_take(&sh.next);
             if (t >= a.io.ntiles) break;
-            expand_tile<KIND, I>(a.g, a.dp, a.col, a.dcol, a.io, t, t, 0, a.ws, ep, a.pool_words, sh, smem, acc_cnt,
+            expand_tile<KIND, I>(a.g, a.dp, a.col, a.dcol, a.io, t, t, 0, a.ws, ep, a.dp.inj, a.pool_words, sh, smem, acc_cnt,
                                  acc_h0, acc_h1);
         }
     }
@@ -1123,7 +1125,7 @@ __global__ __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(8))) void
     for (TileDeal dl; dl.tile() < a.io.ntiles; dl.next()) {  // dealt by XCD, as for LAST_COUNT
         const uint64_t t = dl.tile();
         __syncthreads();
-        expand_tile<EXPAND_LAST_BARE, I>(a.g, a.dp, a.col, a.dcol, a.io, t, t, 0, a.ws, ep, a.pool_words, sh, smem,
+        expand_tile<EXPAND_LAST_BARE, I>(a.g, a.dp, a.col, a.dcol, a.io, t, t, 0, a.ws, ep, a.dp.inj, a.pool_words, sh, smem,
                                          acc_cnt, acc_h0, acc_h1, false);
     }
     flush_sums(acc_cnt, 0, 0, a.io.tot, sh.red);
@@ -1558,13 +1560,15 @@ __global__ __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(4))) void
             // 256-query batch 36.3 against 39.3 ms)
             uint64_t c = 0, h0 = 0, h1 = 0;
             const StepIO io = uniform_copy(B.io);
+            const uint32_t inj = (uint32_t)__builtin_amdgcn_readfirstlane((int)plan->depth[B.d].inj);
             expand_tile<EXPAND_MID, I>(cfg.g, plan->depth[B.d], plan->col, plan->dcol, io, t - t0, t, t0, cfg.ws,
-                                       ep, cfg.pool_words, sh, smem, c, h0, h1);
+                                       ep, inj, cfg.pool_words, sh, smem, c, h0, h1);
         } else {
             uint64_t c = 0, h0 = 0, h1 = 0;
             const StepIO io = uniform_copy(B.io);
+            const uint32_t inj = (uint32_t)__builtin_amdgcn_readfirstlane((int)plan->depth[B.d].inj);
             expand_tile<EXPAND_LAST_COUNT, I>(cfg.g, plan->depth[B.d], plan->col, plan->dcol, io, t - t0, t, t0,
-                                              cfg.ws, ep, cfg.pool_words, sh, smem, c, h0, h1);
+                                              cfg.ws, ep, inj, cfg.pool_words, sh, smem, c, h0, h1);
             flush_sums(c, h0, h1, io.tot, sh.red);
         }
     }

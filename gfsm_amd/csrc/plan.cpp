@@ -75,6 +75,39 @@ void project_levels(const HostGraph &data, const Plan &plan, uint64_t nroots, ui
     }
 }
 
+// Which placed vertices a candidate can coincide with:
+//   * labelled mode: a vertex placed at depth k >= 1 came from a segment of
+//     that depth's generator relation, whose target label it carries (the
+//     root: the source label of the depth-1 generator relation), so a
+//     candidate with another label differs from it;
+//   * a data graph without self loops: a candidate is an entry of the segment
+//     of its generator's ancestor and of every checked ancestor, so equal to
+//     none of them (a candidate that is, fails that check anyway).
+// The candidate test reads one LDS word per candidate and compared column, and
+// at 4 to 16 labels most columns drop out (measured, start against now: labelled
+// random graph of 200,000 vertices, 7-vertex count, 7.93 -> 7.55 ms; nine capped
+// 8-vertex queries on a power-law graph, 5.69 -> 5.37 ms; unlabelled grids, where
+// only the loop rule helps, -0.3% to -2.5%).
+void set_injectivity(const HostGraph &data, Plan &plan)
+{
+    const bool by_label = data.mode == GFSM_MODE_VLABEL;
+    uint32_t label[GFSM_MAXQ] = {};
+    for (uint32_t k = 0; by_label && k < plan.q; k++)
+        label[k] = k ? (plan.dev.depth[k].gen_rel >> 10) & 0x7FFu : plan.dev.root_rel >> 21;
+    for (uint32_t d = 1; d < plan.q; d++) {
+        DepthPlanDev &dp = plan.dev.depth[d];
+        uint32_t m = 0;
+        for (uint32_t k = 0; k < d; k++)
+            if (!by_label || label[k] == label[d]) m |= 1u << k;
+        if (!data.has_loops) {
+            m &= ~(1u << (d - dp.gen_dist));
+            for (uint32_t r = 0; r < dp.nchk; r++)
+                if (dp.chk_dist[r]) m &= ~(1u << (d - dp.chk_dist[r]));
+        }
+        dp.inj = m;
+    }
+}
+
 Status plan_query(const HostGraph &qg, Plan &out, const HostGraph *by_cost)
 {
     out = Plan{};

@@ -20,8 +20,13 @@ struct DepthPlanDev {
     uint32_t nchk;
     uint32_t nxt_dist;
     uint32_t nxt_rel;
+    // Placed columns a candidate of this depth has to be compared with for
+    // injectivity (bit k: the vertex placed at depth k); the others differ from
+    // every candidate by construction (see set_injectivity).
+    uint32_t inj;
     uint32_t chk_dist[GFSM_MAXCHK];
     uint32_t chk_rel[GFSM_MAXCHK];
+    uint32_t pad;
     // Dense segment tables ({begin, end} per data vertex, see DevGraph) of
     // nxt_rel and of the first four chk_rel, filled in per run where one
     // exists; null: the segment hash table.
