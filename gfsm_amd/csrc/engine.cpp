@@ -50,8 +50,8 @@ Status Lane::init(uint64_t max_tiles, bool tile_index)
     HIP_TRY(hipMemset(tot_d, 0, sizeof(Totals)));
     HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&tot_h), sizeof(Totals), hipHostMallocDefault));
     std::memset(tot_h, 0, sizeof(Totals));
-    HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&kc_h), 2 * sizeof(uint64_t), hipHostMallocCoherent));
-    kc_h[0] = kc_h[1] = 0;
+    HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&kc_h), 4 * sizeof(uint64_t), hipHostMallocCoherent));
+    std::memset(kc_h, 0, 4 * sizeof(uint64_t));
     for (int i = 0; i < 2; i++) HIP_TRY(hipEventCreate(&ev[i]));
     return Status::ok();
 }
@@ -238,9 +238,9 @@ Status ensure_arena(Arena &a, uint64_t bytes)
 Status ensure_arena(Ctx &ctx, uint64_t bytes) { return ensure_arena(ctx.arena, bytes); }
 
 template <class T>
-static Status dev_copy(T *&dst, const std::vector<T> &src, size_t &bytes)
+static Status dev_copy(T *&dst, const std::vector<T> &src, size_t &bytes, size_t pad = 0)
 {
-    size_t b = std::max<size_t>(src.size(), 1) * sizeof(T);
+    size_t b = std::max<size_t>(src.size() + pad, 1) * sizeof(T);
     HIP_TRY(hipMalloc(&dst, b));
     if (!src.empty()) HIP_TRY(hipMemcpy(dst, src.data(), src.size() * sizeof(T), hipMemcpyHostToDevice));
     bytes += b;
@@ -264,7 +264,7 @@ Status upload_graph(Ctx &ctx, const HostGraph &g, DevGraph *&out)
         dir_flat[2 * i] = g.dir[i].rel;
         dir_flat[2 * i + 1] = g.dir[i].beg;
     }
-    Status st = dev_copy(dg->nbr, g.nbr, dg->bytes);
+    Status st = dev_copy(dg->nbr, g.nbr, dg->bytes, kNbrPad);
     if (st.good()) st = dev_copy(dg->dir_ptr, g.dir_ptr, dg->bytes);
     if (st.good()) st = dev_copy(dg->dir, dir_flat, dg->bytes);
     if (st.good()) st = dev_copy(dg->rel_vtx, g.rel_vtx, dg->bytes);
@@ -415,6 +415,8 @@ struct Runner {
     Result &res;
     uint32_t q = 0;
     bool rows_mode = false, digest = false, prof = false;
+    bool tail = false;          // depth q-2 counts the last depth's embeddings (EXPAND_TAIL)
+    uint64_t tail_count = 0;    // embeddings counted by capped tail steps
     uint32_t *vec[GFSM_MAXQ] = {}, *gbeg[GFSM_MAXQ] = {};
     uint64_t *off[GFSM_MAXQ] = {};
     uint64_t cap[GFSM_MAXQ] = {};
@@ -455,7 +457,7 @@ struct Runner {
     // (Only when the next generator is an older ancestor, not the new vertex.)
     uint32_t need_nxt(uint32_t kind, uint32_t d) const
     {
-        return (kind == EXPAND_MID && plan.dev.depth[d].nxt_dist > 1) ? 1u : 0u;
+        return ((kind == EXPAND_MID || kind == EXPAND_TAIL) && plan.dev.depth[d].nxt_dist > 1) ? 1u : 0u;
     }
 
     // Candidates per thread for one expand launch: forced, else tuned.
@@ -487,6 +489,7 @@ struct Runner {
         rows_mode = flags & (GFSM_ROWS | GFSM_SORTED);
         digest = (flags & GFSM_DIGEST) && !rows_mode;  // rows mode: digest from the host rows
         prof = flags & GFSM_PROFILE;
+        tail = (lane.kc_h && lane.tile_node) && !rows_mode && !digest && q >= 3 && plan.dev.depth[q - 1].nchk == 0;
         grid_cap = std::max<uint32_t>(ctx.num_cus, 1) * ctx.tune.wgs_per_cu;
         const uint64_t min_nodes = 8 * kTile;  // a level must hold one launch tile's survivors
         uint64_t row_bytes = 0;
@@ -508,6 +511,7 @@ struct Runner {
             chunk[k + 1] = std::min<uint64_t>(c, launch_limit());
         }
         chunk[q - 1] = launch_limit();
+        if (tail) chunk[q - 2] = launch_limit();  // writes no level
         char *p = nullptr;
         if (fixed) {
             if (total > fixed->bytes)
@@ -703,16 +707,20 @@ struct Runner {
         // registers under 64 for eight waves per SIMD).
         const bool bare = last && !rows_mode && !digest && plan.dev.depth[d].nchk == 0 &&
                           !(forced_items > kBareItems);
-        const uint32_t kind =
+        const bool at_tail = tail && d + 2 == q;
+        const uint32_t inner_kind =
             last ? (rows_mode ? EXPAND_LAST_ROWS : (bare ? EXPAND_LAST_BARE : EXPAND_LAST_COUNT)) : EXPAND_MID;
         const uint64_t tile_limit = launch_limit();
-        const uint32_t items =
-            bare ? std::min(pick_items(EXPAND_LAST_COUNT, d), bare_items(g1 - g0, S_prev, d)) : pick_items(kind, d);
+        const uint32_t items = bare ? std::min(pick_items(EXPAND_LAST_COUNT, d), bare_items(g1 - g0, S_prev, d))
+                                    : pick_items(inner_kind, d);
         const uint32_t pool_words = bare ? std::min(ctx.tune.pool_words, kBarePoolWords) : ctx.tune.pool_words;
         const uint32_t grid_mul = bare ? 2 : 1;  // twice the resident workgroups
         const uint64_t tc = (uint64_t)kTile * items;
+        const bool capped = max_depth_cand || max_cand;  // then lane.kc_h and lane.tile_node are there
+        uint64_t untailed = g0;  // candidates before it take the two steps (a cap ends inside them)
         bool first = true;
         for (uint64_t c = g0; c < g1;) {
+            const uint32_t kind = at_tail && c >= untailed ? (uint32_t)EXPAND_TAIL : inner_kind;
             uint64_t e = std::min(g1, c + std::max<uint64_t>(tc, std::min(chunk[d], tile_limit)));
             if (max_depth_cand) {
                 // Deterministic cap: depth d tests only its first max_depth_cand
@@ -721,6 +729,8 @@ struct Runner {
                 if (depth_done[d] >= max_depth_cand) return Status::err(GFSM_ERR_CAP, "per-depth candidate cap reached");
                 e = std::min(e, c + (max_depth_cand - depth_done[d]));
             }
+            if (at_tail && kind == EXPAND_MID)  // writes the level, up to the range's end
+                e = std::min(e, std::min(untailed, c + std::max<uint64_t>(tc, cap[d])));
             ExpandArgs a{};
             a.items = items;
             a.pool_words = pool_words;
@@ -730,7 +740,13 @@ struct Runner {
             std::memcpy(a.dcol, plan.dev.dcol, sizeof(a.dcol));
             StepIO &io = a.io;
             io.need_nxt = need_nxt(kind, d);
-            if (kind == EXPAND_MID)
+            if (kind == EXPAND_TAIL) {
+                a.linj = plan.dev.depth[d + 1].inj;
+                a.tail_sums = lane.tile_node;
+                a.room = max_depth_cand ? max_depth_cand - std::min(max_depth_cand, depth_done[d + 1]) : ~0ull;
+                if (max_cand) a.room = std::min(a.room, max_cand - std::min(max_cand, cand_total + (e - c)));
+            }
+            if (kind == EXPAND_MID || kind == EXPAND_TAIL)
                 a.dp.nxt_seg = dense(plan.dev.depth[d].nxt_rel, e - c);
             for (uint32_t r = 0; r < std::min<uint32_t>(plan.dev.depth[d].nchk, kDenseChk); r++)
                 a.dp.chk_seg[r] = dense(plan.dev.depth[d].chk_rel[r], e - c);
@@ -744,7 +760,7 @@ struct Runner {
             io.S_prev = S_prev;
             io.g_begin = c;
             io.g_end = e;
-            if (!last) {
+            if (kind == EXPAND_MID) {
                 io.out_vec = vec[d];
                 io.out_off = off[d];
                 io.out_gbeg = gbeg[d];
@@ -754,7 +770,9 @@ struct Runner {
                 io.cap = rows_cap;
             }
             io.tot = lane.tot_d;
-            io.host_kc = (kind == EXPAND_MID || kind == EXPAND_LAST_ROWS) ? arm_step_totals() : nullptr;
+            io.host_kc = (kind == EXPAND_MID || kind == EXPAND_LAST_ROWS || (kind == EXPAND_TAIL && capped))
+                             ? arm_step_totals()
+                             : nullptr;
             io.ntiles = (e - c + tc - 1) / tc;
             a.ws = lane.ws;
             // Launch-shape checks: the workspace holds every tile, the frontier
@@ -788,6 +806,32 @@ struct Runner {
             Status st = kend(true);
             if (!st.good()) return st;
             if (kind == EXPAND_LAST_COUNT || kind == EXPAND_LAST_BARE) {
+                res.stats.cand[d] += e - c;
+                depth_done[d] += e - c;
+                c = e;
+                continue;
+            }
+            if (kind == EXPAND_TAIL) {
+                if (capped) {
+                    st = sync_step_totals(io.host_kc, true);
+                    if (!st.good()) return st;
+                    const volatile uint64_t *w = reinterpret_cast<const volatile uint64_t *>(io.host_kc);
+                    const uint64_t kept = w[0], cnt = w[1], emb = w[2], tiles = w[3];
+                    if (tiles < io.ntiles) {
+                        // The cap's last candidate falls in tile `tiles`: that tile
+                        // is expanded level by level, which stops there.
+                        const uint64_t to = c + tiles * tc;
+                        untailed = std::min(e, to + tc);
+                        cand_total -= e - to;
+                        e = to;
+                    }
+                    if (max_depth_cand && e > c) chunk[d] = capped_chunk(d, e - c, cnt, tile_limit, tc);
+                    cand_total += cnt;
+                    tail_count += emb;
+                    res.stats.level[d] += kept;
+                    res.stats.cand[d + 1] += cnt;
+                    depth_done[d + 1] += cnt;
+                }
                 res.stats.cand[d] += e - c;
                 depth_done[d] += e - c;
                 c = e;
@@ -1043,7 +1087,11 @@ Status run_match(Ctx &ctx, const HostGraph &data, const DevGraph &dg, const Plan
         }
         if (o.flags & GFSM_SORTED) sort_rows(res.rows, q);
     } else {
-        res.count = L.tot_h->count;
+        res.count = L.tot_h->count + run.tail_count;
+        if (run.tail && !o.max_depth_cand && !o.max_cand) {
+            res.stats.level[q - 2] = L.tot_h->tail_keep;
+            res.stats.cand[q - 1] = L.tot_h->tail_cand;
+        }
         res.stats.level[q - 1] = res.count;
         res.digest[0] = L.tot_h->dg0;
         res.digest[1] = L.tot_h->dg1;

@@ -50,7 +50,8 @@ struct Totals {
     uint64_t cnt;     // candidates of the next depth
     uint64_t count;   // last level, count-only: embeddings
     uint64_t dg0, dg1;// digest sums
-    uint64_t pad[3];
+    uint64_t tail_keep, tail_cand; // tail steps: nodes kept, candidates of the last depth (sums)
+    uint64_t pad;
 };
 
 enum ExpandKind : uint32_t {
@@ -59,6 +60,8 @@ enum ExpandKind : uint32_t {
     EXPAND_LAST_ROWS = 2,  // last depth: write rows in original ids (and digest)
     EXPAND_LAST_BARE = 3,  // last depth, count only, no checks and no digest: a lean kernel
                            // that fits twice the resident workgroups of the others
+    EXPAND_TAIL = 4,       // depth q-2 of a count whose last depth has no checks: the survivors'
+                           // children are counted from their segments, no level is written
 };
 constexpr uint32_t kBarePoolWords = 2048;  // LDS pool of the lean last-depth kernel
 
@@ -90,8 +93,10 @@ struct StepIO {
     const uint64_t *tile_node; // [2*ntiles] first and last frontier node of each tile (k_tile_index),
                                // or null: each tile searches in_off itself
     uint64_t *host_kc;         // or null: fine-grained host words that also receive {keep, cnt},
-                               // so the host reads a step's totals without a copy
+                               // so the host reads a step's totals without a copy (a capped
+                               // EXPAND_TAIL: see ExpandArgs::room)
 };
+constexpr uint32_t kNbrPad = 4;     // words allocated past nbr's end (four-word loads of a segment's end)
 constexpr uint32_t kDenseChk = 4;  // checked relations per depth with a dense-table slot (DepthPlanDev)
 
 // Root step: the candidates of depth 0 (a slice of the relation index).
@@ -118,6 +123,14 @@ struct ExpandArgs {
     ScanWS ws;
     uint32_t items;            // candidates per thread: 1, 2, 4 or 8 (tile = 256 * items)
     uint32_t pool_words;       // LDS words for per-node staging (checked segments, rows)
+    uint32_t linj;             // EXPAND_TAIL: injectivity mask of the last depth
+    uint32_t pad;
+    // EXPAND_TAIL under a cap (io.host_kc set): last-depth candidates left.  The
+    // step counts its first tiles whose candidates fit and tells the host {nodes
+    // kept, candidates, embeddings, tiles} of those; nothing goes to io.tot.
+    uint64_t room;
+    uint64_t *tail_sums;       // [2*ntiles] the tiles' {embeddings, kept and candidates}; may be
+                               // io.tile_node's array (a tile reads its entries before it writes them)
 };
 
 struct RootArgs {

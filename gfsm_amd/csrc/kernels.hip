@@ -47,6 +47,7 @@ DEV gptr_t<T> gp(T *p)
 
 constexpr uint32_t kWaves = kTile / 64;
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));  // one 16-byte store
+typedef uint32_t u32x4_w __attribute__((ext_vector_type(4), aligned(4)));  // ... or load of four words, word-aligned
 constexpr uint32_t kNodeLk = 4;  // node-setup lookups a thread keeps in flight
 constexpr uint32_t kStageLd = 8; // row words a thread loads before storing them to LDS
 
@@ -421,6 +422,33 @@ DEV void flush_sums(uint64_t cnt, uint64_t h0, uint64_t h1, Totals *tot_ptr, uin
     }
 }
 
+// The same for a tail step: embeddings, nodes kept and candidates of the last depth.
+DEV void flush_tail(uint64_t cnt, uint64_t kept, uint64_t cand, Totals *tot_ptr, uint64_t (*s_red)[kWaves])
+{
+    const uint32_t lane = lane_id(), wave = threadIdx.x >> 6;
+    cnt = wave_sum64(cnt);
+    kept = wave_sum64(kept);
+    cand = wave_sum64(cand);
+    if (lane == 0) {
+        s_red[0][wave] = cnt;
+        s_red[1][wave] = kept;
+        s_red[2][wave] = cand;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint64_t c = 0, a = 0, b = 0;
+        for (uint32_t w = 0; w < kWaves; w++) {
+            c += s_red[0][w];
+            a += s_red[1][w];
+            b += s_red[2][w];
+        }
+        const auto tot = gp(tot_ptr);
+        if (c) __hip_atomic_fetch_add(&tot->count, c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (a) __hip_atomic_fetch_add(&tot->tail_keep, a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (b) __hip_atomic_fetch_add(&tot->tail_cand, b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+}
+
 // One per-node lookup of a tile's staging (a checked ancestor's segment or
 // the next generator's): the row column whose vertex is looked up (~0u: none,
 // the check is the candidate's own), its relation and its dense table.
@@ -451,6 +479,27 @@ DEV void publish_kc(uint64_t *kc, uint64_t keep, uint64_t cnt)
 {
     __hip_atomic_store(kc + 1, cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     __hip_atomic_store(kc, keep, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// One tile's sums of a capped tail step: a tile keeps at most 2,048 nodes, of
+// fewer than 2^26 candidates each.
+constexpr uint32_t kTailKeptShift = 48;
+DEV void tail_tile_sums(uint64_t *sums, uint64_t t, uint64_t cnt, uint64_t kept, uint64_t cand,
+                        uint64_t (*s_red)[kWaves])
+{
+    const uint32_t lane = lane_id(), wave = threadIdx.x >> 6;
+    cnt = wave_sum64(cnt);
+    cand = wave_sum64(kept << kTailKeptShift | cand);
+    if (lane == 0) {
+        s_red[0][wave] = cnt;
+        s_red[1][wave] = cand;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        uint64_t v = 0;
+        for (uint32_t w = 0; w < kWaves; w++) v += s_red[threadIdx.x][w];
+        gp(sums)[2 * t + threadIdx.x] = v;
+    }
 }
 
 // Root tile `lt` of a root step (global tile gt, the step's scan starting at
@@ -588,16 +637,124 @@ DEV uint64_t frontier_search(P off, uint64_t S, uint64_t key, uint32_t sub)
     return lo;
 }
 
-// Column c of the node row at `row` (c < d), or `own` (the candidate itself)
-// when c == d.  The row word is read for every lane, at column 0 where it is
-// not wanted, and the value is selected afterwards: a select between the two
-// sources' addresses would put the candidates' register array in scratch
-// memory and make every such read a flat load.
-template <class RP>
-DEV uint32_t pick_row_or(RP rows, uint32_t row, uint32_t c, uint32_t d, uint32_t own)
+// The placed vertices of a tile's nodes: at(j, c) is column c of node j.  In
+// LDS either whole rows or, MAPPED, the columns of `need` packed together;
+// otherwise in the level itself.
+template <bool MAPPED>
+struct LdsRows {
+    const uint32_t *p;
+    uint32_t stride, need;
+    DEV uint32_t at(uint32_t j, uint32_t c) const
+    {
+        return p[j * stride + (MAPPED ? (uint32_t)__builtin_popcount(need & ((1u << c) - 1u)) : c)];
+    }
+};
+struct LevelRows {
+    gptr_t<const uint32_t> p;
+    uint32_t d;
+    DEV uint32_t at(uint32_t j, uint32_t c) const { return p[j * d + c]; }
+};
+
+// Column c of node j's row (c < d), or `own` (the candidate itself) when
+// c == d.  The row word is read for every lane, at column c0 (one the rows
+// hold) where it is not wanted, and the value is selected afterwards: a select
+// between the two sources' addresses would put the candidates' register array
+// in scratch memory and make every such read a flat load.
+template <class RA>
+DEV uint32_t pick_row_or(const RA &rows, uint32_t j, uint32_t c, uint32_t d, uint32_t own, uint32_t c0 = 0u)
 {
-    const uint32_t v = rows[row + (c < d ? c : 0u)];
+    const uint32_t v = rows.at(j, c < d ? c : c0);
     return c < d ? v : own;
+}
+
+// ov[k] += how many entries of the segment nbr[gb[k], gb[k] + cnt[k]) are one
+// of the columns `cols` of node jj[k]'s row (column d: w[k] itself); cnt 0
+// counts nothing.  Segments of up to kTailShort entries are read whole, four
+// words a load, and every column is compared with all of them; in longer ones
+// each column is searched, the I searches in lockstep, and every copy of a
+// repeated entry counts.
+constexpr uint32_t kTailShort = 8;
+template <uint32_t I, class RA>
+DEV void tail_overlap(const uint32_t *__restrict__ nbr, const RA &rows, uint32_t d, uint32_t cols,
+                      const uint32_t (&jj)[I], const uint32_t (&w)[I], const uint32_t (&gb)[I],
+                      const uint32_t (&cnt)[I], uint32_t (&ov)[I])
+{
+    constexpr uint32_t B = I < 4 ? I : 4;
+#pragma unroll
+    for (uint32_t k0 = 0; k0 < I; k0 += B) {
+        u32x4 lo[B], hi[B];
+#pragma unroll
+        for (uint32_t b = 0; b < B; b++) {
+            const uint32_t k = k0 + b, n = cnt[k] <= kTailShort ? cnt[k] : 0u;
+            const auto at = (gptr_t<const u32x4_w>)gp(nbr + gb[k]);
+            lo[b] = n ? (u32x4)at[0] : u32x4{0u, 0u, 0u, 0u};
+            hi[b] = n > 4 ? (u32x4)at[1] : u32x4{0u, 0u, 0u, 0u};
+        }
+#pragma unroll
+        for (uint32_t b = 0; b < B; b++) {
+            const uint32_t k = k0 + b, n = cnt[k] <= kTailShort ? cnt[k] : 0u;
+#pragma unroll
+            for (uint32_t e = 0; e < 4; e++) {
+                lo[b][e] = e < n ? lo[b][e] : kSegEmpty;  // no vertex
+                hi[b][e] = e + 4 < n ? hi[b][e] : kSegEmpty;
+            }
+        }
+        for (uint32_t m = cols; m; m &= m - 1) {
+            const uint32_t c = (uint32_t)__builtin_ctz(m);
+            uint32_t x[B];
+            if (c == d) {
+#pragma unroll
+                for (uint32_t b = 0; b < B; b++) x[b] = w[k0 + b];
+            } else {
+#pragma unroll
+                for (uint32_t b = 0; b < B; b++) x[b] = rows.at(jj[k0 + b], c);
+            }
+#pragma unroll
+            for (uint32_t b = 0; b < B; b++)
+#pragma unroll
+                for (uint32_t e = 0; e < 4; e++) ov[k0 + b] += (lo[b][e] == x[b] ? 1u : 0u) + (hi[b][e] == x[b] ? 1u : 0u);
+        }
+    }
+    bool any = false;
+#pragma unroll
+    for (uint32_t k = 0; k < I; k++) any |= cnt[k] > kTailShort;
+    if (!__any(any)) return;
+    for (uint32_t m = cols; m; m &= m - 1) {
+        const uint32_t c = (uint32_t)__builtin_ctz(m);
+        uint32_t x[I], lo[I], n[I];
+#pragma unroll
+        for (uint32_t k = 0; k < I; k++) {
+            x[k] = c == d ? w[k] : rows.at(jj[k], c == d ? 0u : c);
+            lo[k] = gb[k];
+            n[k] = cnt[k] > kTailShort ? cnt[k] : 0u;
+        }
+        for (;;) {
+            bool more = false;
+#pragma unroll
+            for (uint32_t k = 0; k < I; k++) more |= n[k] > 1;
+            if (!more) break;
+            uint32_t v[I];
+#pragma unroll
+            for (uint32_t k = 0; k < I; k++) v[k] = (n[k] > 1) ? nbr[lo[k] + (n[k] >> 1)] : 0u;
+#pragma unroll
+            for (uint32_t k = 0; k < I; k++) {
+                if (n[k] > 1) {
+                    const uint32_t h = n[k] >> 1;
+                    if (v[k] <= x[k]) lo[k] += h;
+                    n[k] -= h;
+                }
+            }
+        }
+        // lo: the last entry <= x, if any; equal ones end there
+#pragma unroll
+        for (uint32_t k = 0; k < I; k++) {
+            if (!n[k]) continue;
+            for (uint32_t p = lo[k]; nbr[p] == x[k]; p--) {
+                ov[k]++;
+                if (p == gb[k]) break;
+            }
+        }
+    }
 }
 
 // Expand tile `lt` of a step (global tile gt; the step's scan starts at gt0).
@@ -605,16 +762,19 @@ DEV uint32_t pick_row_or(RP rows, uint32_t row, uint32_t c, uint32_t d, uint32_t
 // base and a pool of pool_words words that stages, per frontier node of the
 // tile, the checked ancestor segments, the next generator segment and the
 // placed vertices, as far as they fit.  `inj` is the depth's injectivity mask
-// (a scalar).  LAST_COUNT adds its embeddings and digest to the thread's accumulators; the other kinds write their output.
+// and `linj` the next depth's (scalars; linj for EXPAND_TAIL).  LAST_COUNT adds its embeddings and digest to the thread's accumulators; the other kinds write their output.
 template <uint32_t KIND, uint32_t I, class DP, class CP>
 DEV void expand_tile(const DevGraphView &g, const DP &dp, CP col, CP dcol,
                      const StepIO &io, uint64_t lt, uint64_t gt, uint64_t gt0, const ScanWS &ws, uint32_t ep,
-                     uint32_t inj, uint32_t pool_words, TileShared<I> &sh, unsigned char *dyn, uint64_t &acc_cnt,
+                     uint32_t inj, uint32_t linj, uint32_t pool_words, TileShared<I> &sh, unsigned char *dyn, uint64_t &acc_cnt,
                      uint64_t &acc_h0, uint64_t &acc_h1, bool tickets = true)
 {
     constexpr uint32_t T = kTile, TC = kTile * I, NW = TC / 64;
     constexpr bool BARE = KIND == EXPAND_LAST_BARE;  // counting, no checks, no digest
-    constexpr bool COUNTING = KIND == EXPAND_LAST_COUNT || BARE;
+    constexpr bool TAIL = KIND == EXPAND_TAIL;       // counts the last depth's embeddings from the one before
+    constexpr bool INNER = KIND == EXPAND_MID || TAIL;
+    constexpr bool COUNTING = KIND == EXPAND_LAST_COUNT || BARE || TAIL;
+    constexpr bool PACKED = BARE || TAIL;  // stages only the row columns it reads
     const uint32_t d = io.d;
     // The thread index passes through an empty asm, so the compiler sees a
     // new value per tile: the LDS offsets and addresses derived from it are
@@ -641,7 +801,7 @@ DEV void expand_tile(const DevGraphView &g, const DP &dp, CP col, CP dcol,
     const auto tot = gp(io.tot);
 
     const uint32_t nchk = BARE ? 0u : dp.nchk;
-    const uint32_t need_nxt = (KIND == EXPAND_MID) ? io.need_nxt : 0u;
+    const uint32_t need_nxt = INNER ? io.need_nxt : 0u;
     // The depth's lookups, one LDS entry each, so the staging loop below
     // selects its lookup per lane from LDS rather than indexing the plan
     // (kernel arguments or global memory) with a per-lane index.
@@ -676,13 +836,27 @@ DEV void expand_tile(const DevGraphView &g, const DP &dp, CP col, CP dcol,
     // The rows come first: every candidate reads its node's row (d words,
     // twice on inner depths), but a node's segments save lookups only for
     // its candidates after the first.
-    const uint32_t meta_words = 2 * nf * nchk + (need_nxt ? 2 * nf : 0);
-    const uint32_t row_words = (nf * d + 1) & ~1u;  // keeps the segments 8-byte aligned
+    const uint32_t meta_words = 2 * nf * nchk + (need_nxt ? (TAIL ? 3 : 2) * nf : 0);
+    // Row columns staged: all, or the compared ones, with those that lookups
+    // read where the lookups are not staged.
+    uint32_t need = (1u << d) - 1u, rw = d;
+    if (PACKED) {
+        need = (inj | (TAIL ? linj : 0u)) & ((1u << d) - 1u);
+        rw = (uint32_t)__builtin_popcount(need);
+        if (((nf * rw + 1) & ~1u) + meta_words > pool_words) {
+            for (uint32_t r = 0; r < nchk; r++)
+                if (dp.chk_dist[r]) need |= 1u << (d - dp.chk_dist[r]);
+            if (need_nxt) need |= 1u << (d + 1 - dp.nxt_dist);
+            rw = (uint32_t)__builtin_popcount(need);
+        }
+    }
+    const uint32_t row_words = (nf * rw + 1) & ~1u;  // keeps the segments 8-byte aligned
     const bool staged = row_words <= pool_words;
     const bool stage_meta = meta_words + (staged ? row_words : 0) <= pool_words;
     uint32_t *s_rows = s_pool;                                                   // [nf][d]
     uint2 *s_chk = reinterpret_cast<uint2 *>(s_pool + (staged ? row_words : 0));  // [nchk][nf]
     uint2 *s_nxt = s_chk + nchk * nf;                                            // [nf]
+    uint32_t *s_ovl = reinterpret_cast<uint32_t *>(s_nxt + nf);                  // [nf] TAIL: row columns in s_nxt
     // Digest of a counting last depth: each node's placed columns contribute
     // the same terms to all its candidates' row hashes, so their sums are
     // formed once per node (two u64 per node, after the staged data).
@@ -693,14 +867,22 @@ DEV void expand_tile(const DevGraphView &g, const DP &dp, CP col, CP dcol,
 
     // The rows' words, kStageLd loads in flight per thread before their LDS
     // stores (one load, wait, store per word would chain round trips).
-    if (staged) {
-        const uint32_t nw = nf * d;
+    if (staged && rw) {
+        const uint32_t nw = nf * rw;
+        const bool whole = !PACKED || rw == d;
         for (uint32_t u0 = tid; u0 < nw; u0 += T * kStageLd) {
             uint32_t v[kStageLd];
 #pragma unroll
             for (uint32_t b = 0; b < kStageLd; b++) {
                 const uint32_t u = u0 + b * T;
-                v[b] = u < nw ? in_rows[u] : 0u;
+                uint32_t at = u;
+                if (!whole) {  // word c of node j's packed columns: the c-th set bit of `need`
+                    const uint32_t j = u / rw;
+                    uint32_t m = need;
+                    for (uint32_t c = u - j * rw; c; c--) m &= m - 1;
+                    at = j * d + (uint32_t)__builtin_ctz(m | 0x80000000u);
+                }
+                v[b] = u < nw ? in_rows[at] : 0u;
             }
 #pragma unroll
             for (uint32_t b = 0; b < kStageLd; b++) {
@@ -775,6 +957,25 @@ DEV void expand_tile(const DevGraphView &g, const DP &dp, CP col, CP dcol,
 #pragma unroll
             for (uint32_t k = 0; k < L; k++)
                 if (act[k]) s_chk[dst[k]] = tab[k] ? make_uint2((uint32_t)dv[k], (uint32_t)(dv[k] >> 32)) : sg[k];
+            if constexpr (TAIL) {
+                // The node's placed vertices among its children's candidates.
+                if (need_nxt) {
+                    uint32_t nj[L], gbeg[L], n[L], ov[L];
+#pragma unroll
+                    for (uint32_t k = 0; k < L; k++) {
+                        const uint2 e = tab[k] ? make_uint2((uint32_t)dv[k], (uint32_t)(dv[k] >> 32)) : sg[k];
+                        const bool nx = act[k] && dst[k] >= nchk * nf;
+                        nj[k] = nx ? dst[k] - nchk * nf : 0u;
+                        gbeg[k] = e.x;
+                        n[k] = nx ? e.y - e.x : 0u;
+                        ov[k] = 0;
+                    }
+                    tail_overlap<L>(g.nbr, LevelRows{in_rows, d}, d, linj & ((1u << d) - 1u), nj, x, gbeg, n, ov);
+#pragma unroll
+                    for (uint32_t k = 0; k < L; k++)
+                        if (act[k] && dst[k] >= nchk * nf) s_ovl[nj[k]] = ov[k];
+                }
+            }
         }
     }
     __syncthreads();
@@ -846,7 +1047,7 @@ DEV void expand_tile(const DevGraphView &g, const DP &dp, CP col, CP dcol,
             const uint32_t kk = (uint32_t)__builtin_ctz(im);
             uint32_t pv[I];
 #pragma unroll
-            for (uint32_t k = 0; k < I; k++) pv[k] = rows[jj[k] * d + kk];
+            for (uint32_t k = 0; k < I; k++) pv[k] = rows.at(jj[k], kk);
 #pragma unroll
             for (uint32_t k = 0; k < I; k++) keep[k] &= pv[k] != w[k];
         }
@@ -860,7 +1061,7 @@ DEV void expand_tile(const DevGraphView &g, const DP &dp, CP col, CP dcol,
             } else {
                 uint32_t x[I];
 #pragma unroll
-                for (uint32_t k = 0; k < I; k++) x[k] = pick_row_or(rows, jj[k] * d, dist ? d - dist : d, d, w[k]);
+                for (uint32_t k = 0; k < I; k++) x[k] = pick_row_or(rows, jj[k], dist ? d - dist : d, d, w[k]);
                 const void *ct = r < kDenseChk ? dp.chk_seg[r] : nullptr;
                 if (ct) {
                     const auto tab = gp(reinterpret_cast<const uint64_t *>(ct));
@@ -876,7 +1077,7 @@ DEV void expand_tile(const DevGraphView &g, const DP &dp, CP col, CP dcol,
             seg_contains_n<I>(g.nbr, sg, w, keep);
         }
 
-        if (KIND == EXPAND_MID) {
+        if (INNER) {
             // Phase 4: the survivor's next generator segment; no children, no node.
             uint2 ns[I];
             if (need_nxt && stage_meta) {
@@ -887,7 +1088,7 @@ DEV void expand_tile(const DevGraphView &g, const DP &dp, CP col, CP dcol,
                 const auto tab = gp(reinterpret_cast<const uint64_t *>(dp.nxt_seg));
 #pragma unroll
                 for (uint32_t k = 0; k < I; k++) {
-                    const uint32_t x = pick_row_or(rows, jj[k] * d, need_nxt ? d + 1 - dp.nxt_dist : d, d, w[k]);
+                    const uint32_t x = pick_row_or(rows, jj[k], need_nxt ? d + 1 - dp.nxt_dist : d, d, w[k]);
                     const uint64_t v = keep[k] ? tab[x] : 0ull;
                     ns[k] = make_uint2((uint32_t)v, (uint32_t)(v >> 32));
                 }
@@ -895,7 +1096,7 @@ DEV void expand_tile(const DevGraphView &g, const DP &dp, CP col, CP dcol,
                 uint32_t x[I];
 #pragma unroll
                 for (uint32_t k = 0; k < I; k++)
-                    x[k] = pick_row_or(rows, jj[k] * d, need_nxt ? d + 1 - dp.nxt_dist : d, d, w[k]);
+                    x[k] = pick_row_or(rows, jj[k], need_nxt ? d + 1 - dp.nxt_dist : d, d, w[k]);
                 seg_lookup_n<I>(g, x, dp.nxt_rel, keep, ns);
             }
 #pragma unroll
@@ -958,7 +1159,7 @@ DEV void expand_tile(const DevGraphView &g, const DP &dp, CP col, CP dcol,
                 if (KIND == EXPAND_MID && coalesce) {
                     if (put[k]) {
                         uint32_t *sr = wst + kpre[k] * row_w;
-                        for (uint32_t kk = 0; kk < d; kk++) sr[kk] = rows[jj[k] * d + kk];
+                        for (uint32_t kk = 0; kk < d; kk++) sr[kk] = rows.at(jj[k], kk);
                         sr[d] = w[k];
                     }
                     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -1007,7 +1208,7 @@ DEV void expand_tile(const DevGraphView &g, const DP &dp, CP col, CP dcol,
                     const auto out = (KIND == EXPAND_MID) ? out_vec : out_rows;
 #pragma unroll
                     for (uint32_t k = 0; k < I; k++)
-                        if (put[k]) out[idx[k] * wd + ck] = rows[jj[k] * d + kk];
+                        if (put[k]) out[idx[k] * wd + ck] = rows.at(jj[k], kk);
                 }
             }
             if (lt == io.ntiles - 1 && tid == 0) {
@@ -1016,11 +1217,26 @@ DEV void expand_tile(const DevGraphView &g, const DP &dp, CP col, CP dcol,
                 if (io.host_kc) publish_kc(io.host_kc, sm.tot[0], sm.tot[1]);
                 if (KIND == EXPAND_MID && sm.tot[0] <= io.cap) out_off[sm.tot[0]] = sm.tot[1];
             }
+        } else if constexpr (TAIL) {
+            // Every entry of the survivor's next segment is an embedding, but
+            // for the placed vertices among them.
+            uint32_t ov[I];
+            const bool by_node = need_nxt && stage_meta;
+#pragma unroll
+            for (uint32_t k = 0; k < I; k++) ov[k] = by_node ? s_ovl[jj[k]] : 0u;
+            const uint32_t cols = by_node ? linj & (1u << d) : linj;
+            if (cols) tail_overlap<I>(g.nbr, rows, d, cols, jj, w, gb, cnt, ov);
+#pragma unroll
+            for (uint32_t k = 0; k < I; k++) {
+                acc_h0 += keep[k] ? 1u : 0u;
+                acc_h1 += cnt[k];
+                acc_cnt += keep[k] ? cnt[k] - ov[k] : 0u;
+            }
         } else {
 #pragma unroll
             for (uint32_t k = 0; k < I; k++) acc_cnt += keep[k] ? 1u : 0u;
         }
-        if (KIND != EXPAND_MID && !BARE && io.digest && part_ok) {
+        if (!INNER && !BARE && io.digest && part_ok) {
             const uint64_t cw = (uint64_t)col[d] << 32;
 #pragma unroll
             for (uint32_t k = 0; k < I; k++) {
@@ -1029,14 +1245,14 @@ DEV void expand_tile(const DevGraphView &g, const DP &dp, CP col, CP dcol,
                 acc_h0 += mix64(s_part[2 * jj[k]] + mix64(0x9E3779B97F4A7C15ull ^ xv));
                 acc_h1 += mix64(s_part[2 * jj[k] + 1] + mix64(0xD1B54A32D192ED03ull ^ xv));
             }
-        } else if (KIND != EXPAND_MID && !BARE && io.digest) {
+        } else if (!INNER && !BARE && io.digest) {
 #pragma unroll
             for (uint32_t k = 0; k < I; k++) {
                 if (!keep[k]) continue;
                 uint64_t x0 = 0, x1 = 0;
                 for (uint32_t c = 0; c < io.q; c++) {
                     const uint32_t dc = dcol[c];
-                    const uint32_t val = pick_row_or(rows, jj[k] * d, dc, d, w[k]);
+                    const uint32_t val = pick_row_or(rows, jj[k], dc, d, w[k]);
                     const uint64_t xv = (uint64_t)val | ((uint64_t)c << 32);
                     x0 += mix64(0x9E3779B97F4A7C15ull ^ xv);
                     x1 += mix64(0xD1B54A32D192ED03ull ^ xv);
@@ -1047,9 +1263,9 @@ DEV void expand_tile(const DevGraphView &g, const DP &dp, CP col, CP dcol,
         }
     };
     if (staged)
-        tail(s_rows);
+        tail(LdsRows<PACKED>{s_rows, rw, need});
     else
-        tail(in_rows);
+        tail(LevelRows{in_rows, d});
 }
 
 
@@ -1096,7 +1312,7 @@ __global__ __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(4))) void
         for (TileDeal dl; dl.tile() < a.io.ntiles; dl.next()) {
             const uint64_t t = dl.tile();
             __syncthreads();  // the previous tile's readers of the tile LDS are done
-            expand_tile<KIND, I>(a.g, a.dp, a.col, a.dcol, a.io, t, t, 0, a.ws, ep, a.dp.inj, a.pool_words, sh, smem, acc_cnt,
+            expand_tile<KIND, I>(a.g, a.dp, a.col, a.dcol, a.io, t, t, 0, a.ws, ep, a.dp.inj, a.linj, a.pool_words, sh, smem, acc_cnt,
                                  acc_h0, acc_h1, false);
         }
     } else {
@@ -1104,12 +1320,129 @@ __global__ __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(4))) void
         for (;;) {
             const uint64_t t = tickets_take(&sh.next);
             if (t >= a.io.ntiles) break;
-            expand_tile<KIND, I>(a.g, a.dp, a.col, a.dcol, a.io, t, t, 0, a.ws, ep, a.dp.inj, a.pool_words, sh, smem, acc_cnt,
+            expand_tile<KIND, I>(a.g, a.dp, a.col, a.dcol, a.io, t, t, 0, a.ws, ep, a.dp.inj, a.linj, a.pool_words, sh, smem, acc_cnt,
                                  acc_h0, acc_h1);
         }
     }
     if (KIND != EXPAND_MID) flush_sums(acc_cnt, acc_h0, acc_h1, a.io.tot, sh.red);
     finish_launch(a.ws);
+}
+
+// The tail kernel: depth q-2, whose survivors' children are counted without a
+// level in between, from each survivor's segment of the last generator.  Under
+// a cap (host_kc set) the tiles' sums stay apart for k_tail_cut; otherwise they
+// are added to the totals.
+// The last two depths held most of a count's candidates and nearly all of its
+// level traffic (7-vertex path on the 1400 x 1400 grid: 420 M nodes of 36 bytes
+// written and read back).  The step is bound by the loads of a candidate, of its
+// next segment's bounds and of that segment's entries, so it keeps 8 candidates
+// per thread and four waves per SIMD as k_expand, and deals its tiles without
+// tickets.  Measured, two steps against this one: that path 23.9 -> 12.2 ms; a
+// 7-vertex count on a 200,000-vertex labelled graph 8.0 -> 2.9 ms, a 6-vertex one
+// inside 60 MiB of levels 1.26 -> 0.45 ms; nine capped queries on R-MAT 18, where
+// the tile with the cap's candidate still takes the two steps, 6.7 -> 5.5 ms.
+template <uint32_t I>
+__global__ __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(4))) void k_expand_tail(ExpandArgs a)
+{
+    extern __shared__ __align__(16) unsigned char smem[];
+    __shared__ TileShared<I> sh;
+    const uint32_t ep = read_epoch(a.ws);
+    const bool capped = a.io.host_kc != nullptr;
+    uint64_t cnt = 0, kept = 0, cand = 0;
+    for (TileDeal dl; dl.tile() < a.io.ntiles; dl.next()) {
+        const uint64_t t = dl.tile();
+        __syncthreads();
+        expand_tile<EXPAND_TAIL, I>(a.g, a.dp, a.col, a.dcol, a.io, t, t, 0, a.ws, ep, a.dp.inj, a.linj, a.pool_words,
+                                    sh, smem, cnt, kept, cand, false);
+        if (capped) {
+            tail_tile_sums(a.tail_sums, t, cnt, kept, cand, sh.red);
+            cnt = kept = cand = 0;
+        }
+    }
+    if (!capped) flush_tail(cnt, kept, cand, a.io.tot, sh.red);
+    finish_launch(a.ws);
+}
+
+// After a capped tail step (one workgroup): sums the tiles in order up to the
+// first one whose last-depth candidates no longer fit `room`, and tells the
+// host how far it came and the sums so far: {nodes kept, candidates,
+// embeddings, tiles}, the polled first word last.  A kernel of its own: inside
+// the tail kernel its registers would be spilled by every tile.
+__global__ __launch_bounds__(kTile) void k_tail_cut(const uint64_t *tile_sums, uint64_t ntiles, uint64_t room,
+                                                    uint64_t *kc)
+{
+    constexpr uint32_t B = 8;
+    __shared__ uint64_t s_red[3][kWaves];
+    const uint32_t lane = lane_id(), wave = threadIdx.x >> 6;
+    uint64_t kept = 0, cand = 0, cnt = 0, tiles = ntiles;
+    for (uint64_t t0 = 0; t0 < ntiles; t0 += kTile * B) {
+        // this thread's B consecutive tiles: their sums, then the prefix before them
+        uint64_t c[B], k[B], e[B], mine = 0;
+#pragma unroll
+        for (uint32_t b = 0; b < B; b++) {
+            const uint64_t t = t0 + threadIdx.x * B + b;
+            e[b] = t < ntiles ? tile_sums[2 * t] : 0ull;
+            c[b] = t < ntiles ? tile_sums[2 * t + 1] : 0ull;
+        }
+#pragma unroll
+        for (uint32_t b = 0; b < B; b++) {
+            k[b] = c[b] >> kTailKeptShift;
+            c[b] &= (1ull << kTailKeptShift) - 1;
+            mine += c[b];
+        }
+        uint64_t inc = mine;
+        for (uint32_t o = 1; o < 64; o <<= 1) {
+            const uint64_t v = __shfl_up(inc, o, 64);
+            if (lane >= o) inc += v;
+        }
+        if (lane == 63) s_red[0][wave] = inc;
+        __syncthreads();
+        uint64_t run = cand + inc - mine, all = cand;
+        for (uint32_t w = 0; w < kWaves; w++) {
+            if (w < wave) run += s_red[0][w];
+            all += s_red[0][w];
+        }
+        // this thread's tiles that fit
+        uint64_t my_k = 0, my_e = 0, my_c = 0, fit = 0;
+#pragma unroll
+        for (uint32_t b = 0; b < B; b++) {
+            run += c[b];
+            if (run <= room) {
+                my_k += k[b];
+                my_e += e[b];
+                my_c += c[b];
+                fit += t0 + threadIdx.x * B + b < ntiles ? 1 : 0;
+            }
+        }
+        my_k = wave_sum64(my_k << 32 | fit);
+        my_e = wave_sum64(my_e);
+        my_c = wave_sum64(my_c);
+        __syncthreads();
+        if (lane == 0) {
+            s_red[0][wave] = my_k;
+            s_red[1][wave] = my_e;
+            s_red[2][wave] = my_c;
+        }
+        __syncthreads();
+        uint64_t fits = 0;
+        for (uint32_t w = 0; w < kWaves; w++) {
+            kept += s_red[0][w] >> 32;
+            fits += s_red[0][w] & 0xFFFFFFFFull;
+            cnt += s_red[1][w];
+            cand += s_red[2][w];
+        }
+        __syncthreads();
+        if (all > room) {  // candidate counts only grow: the tiles that fit are the first ones
+            tiles = t0 + fits;
+            break;
+        }
+    }
+    if (threadIdx.x == 0) {
+        __hip_atomic_store(kc + 1, cand, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        __hip_atomic_store(kc + 2, cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        __hip_atomic_store(kc + 3, tiles, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        __hip_atomic_store(kc, kept, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
 }
 
 // The lean last-depth kernel: counting only, no checks, no digest, a small
@@ -1125,7 +1458,7 @@ __global__ __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(8))) void
     for (TileDeal dl; dl.tile() < a.io.ntiles; dl.next()) {  // dealt by XCD, as for LAST_COUNT
         const uint64_t t = dl.tile();
         __syncthreads();
-        expand_tile<EXPAND_LAST_BARE, I>(a.g, a.dp, a.col, a.dcol, a.io, t, t, 0, a.ws, ep, a.dp.inj, a.pool_words, sh, smem,
+        expand_tile<EXPAND_LAST_BARE, I>(a.g, a.dp, a.col, a.dcol, a.io, t, t, 0, a.ws, ep, a.dp.inj, a.linj, a.pool_words, sh, smem,
                                          acc_cnt, acc_h0, acc_h1, false);
     }
     flush_sums(acc_cnt, 0, 0, a.io.tot, sh.red);
@@ -1562,13 +1895,13 @@ __global__ __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(4))) void
             const StepIO io = uniform_copy(B.io);
             const uint32_t inj = (uint32_t)__builtin_amdgcn_readfirstlane((int)plan->depth[B.d].inj);
             expand_tile<EXPAND_MID, I>(cfg.g, plan->depth[B.d], plan->col, plan->dcol, io, t - t0, t, t0, cfg.ws,
-                                       ep, inj, cfg.pool_words, sh, smem, c, h0, h1);
+                                       ep, inj, 0u, cfg.pool_words, sh, smem, c, h0, h1);
         } else {
             uint64_t c = 0, h0 = 0, h1 = 0;
             const StepIO io = uniform_copy(B.io);
             const uint32_t inj = (uint32_t)__builtin_amdgcn_readfirstlane((int)plan->depth[B.d].inj);
             expand_tile<EXPAND_LAST_COUNT, I>(cfg.g, plan->depth[B.d], plan->col, plan->dcol, io, t - t0, t, t0,
-                                              cfg.ws, ep, inj, cfg.pool_words, sh, smem, c, h0, h1);
+                                              cfg.ws, ep, inj, 0u, cfg.pool_words, sh, smem, c, h0, h1);
             flush_sums(c, h0, h1, io.tot, sh.red);
         }
     }
@@ -1734,6 +2067,32 @@ static hipError_t launch_expand_bare_t(const ExpandArgs &a, uint32_t grid, hipSt
     return hipGetLastError();
 }
 
+template <uint32_t I>
+static hipError_t launch_expand_tail_t(const ExpandArgs &a, uint32_t grid, hipStream_t s)
+{
+    static bool attr = false;
+    const size_t lds = expand_lds_bytes(I, a.pool_words);
+    if (lds > kMaxDynLds) return hipErrorInvalidValue;
+    hipError_t e = allow_lds(&k_expand_tail<I>, attr);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL((k_expand_tail<I>), dim3(grid), dim3(kTile), lds, s, a);
+    e = hipGetLastError();
+    if (e != hipSuccess || !a.io.host_kc) return e;
+    hipLaunchKernelGGL(k_tail_cut, dim3(1), dim3(kTile), 0, s, a.tail_sums, a.io.ntiles, a.room, a.io.host_kc);
+    return hipGetLastError();
+}
+
+static hipError_t launch_expand_tail(const ExpandArgs &a, uint32_t grid, hipStream_t s)
+{
+    switch (a.items) {
+    case 1: return launch_expand_tail_t<1>(a, grid, s);
+    case 2: return launch_expand_tail_t<2>(a, grid, s);
+    case 4: return launch_expand_tail_t<4>(a, grid, s);
+    case 8: return launch_expand_tail_t<8>(a, grid, s);
+    default: return hipErrorInvalidValue;
+    }
+}
+
 static hipError_t launch_expand_bare(const ExpandArgs &a, uint32_t grid, hipStream_t s)
 {
     switch (a.items) {
@@ -1763,6 +2122,7 @@ hipError_t launch_expand(const ExpandArgs &a, uint32_t grid, hipStream_t s)
     case EXPAND_MID: return launch_expand_k<EXPAND_MID>(a, grid, s);
     case EXPAND_LAST_COUNT: return launch_expand_k<EXPAND_LAST_COUNT>(a, grid, s);
     case EXPAND_LAST_ROWS: return launch_expand_k<EXPAND_LAST_ROWS>(a, grid, s);
+    case EXPAND_TAIL: return launch_expand_tail(a, grid, s);
     case EXPAND_LAST_BARE: return launch_expand_bare(a, grid, s);
     default: return hipErrorInvalidValue;
     }
