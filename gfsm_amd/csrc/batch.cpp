@@ -262,6 +262,7 @@ Status BatchEngine::init(const BatchShape &shape, uint64_t arena_bytes, char *ar
     cfg_.g = dg_->view;
     cfg_.ws = lane_.ws;
     grid_ = std::max<uint32_t>(ctx_.num_cus, 1) * std::max<uint32_t>(shape_.wgs_per_cu, 1);
+    cfg_.fill_tiles = grid_;
     // The schedule is fresh between replays: replays run [tile index, step,
     // schedule] x K.  One empty step outside capture also sets the step
     // kernel's LDS limit.

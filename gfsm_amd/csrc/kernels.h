@@ -285,7 +285,7 @@ struct BatchCfg {
     uint32_t nslots;
     uint32_t items;               // candidates per thread (tile = 256 * items)
     uint32_t pool_words;
-    uint32_t pad;
+    uint32_t fill_tiles;          // tiles that fill the GPU (the step kernel's workgroups)
     uint64_t max_step_cand;       // upper bound of BatchCtl::step_cand (workspace size)
     uint64_t max_degree;          // of the data graph (scan value bound)
     DevGraphView g;
