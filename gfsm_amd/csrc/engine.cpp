@@ -671,6 +671,7 @@ struct Runner {
             a.nchk = plan.dev.nroot_chk;
             std::memcpy(a.chk_rel, plan.dev.root_chk_rel, sizeof(a.chk_rel));
             a.ws = lane.ws;
+            a.ws.brief = a.io.ntiles <= grid_cap;
             if (a.io.ntiles > lane.ws.max_tiles || e > data.rel_vtx.size())
                 return Status::err(GFSM_ERR_ARG, "internal: root launch shape check failed");
             HIP_TRY(lane.before_launch());
@@ -775,6 +776,7 @@ struct Runner {
                              : nullptr;
             io.ntiles = (e - c + tc - 1) / tc;
             a.ws = lane.ws;
+            a.ws.brief = a.io.ntiles <= grid_cap;
             // Launch-shape checks: the workspace holds every tile, the frontier
             // is non-empty and the LDS staging fits.
             if (io.ntiles == 0 || io.ntiles > lane.ws.max_tiles || S_prev == 0 || S_prev > cap[d - 1] ||

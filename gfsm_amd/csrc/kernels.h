@@ -42,6 +42,7 @@ struct ScanWS {
     uint64_t *wc;     // [max_tiles] candidate words
     uint32_t *ctl;    // [4]
     uint64_t max_tiles;
+    bool brief = false; // every tile of the launch is in flight at once: poll often (see lookback)
 };
 
 // Results of one step, written on the device, read by the host afterwards.

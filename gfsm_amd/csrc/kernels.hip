@@ -222,7 +222,7 @@ DEV uint64_t pack(uint64_t st, uint32_t ep, uint64_t v)
 // tile t0 (the first tile of the step's query), computed by all 64 lanes of
 // one wave: each pass reads the words of the 64 preceding tiles, waits until
 // every tile up to the nearest inclusive prefix has published, and sums.
-DEV uint64_t lookback(const uint64_t *words, uint32_t ep, uint64_t t, uint64_t t0)
+DEV uint64_t lookback(const ScanWS &ws, const uint64_t *words, uint32_t ep, uint64_t t, uint64_t t0)
 {
     const uint32_t lane = lane_id();
     const uint64_t epm = (uint64_t)(ep & ((1u << kEpochBits) - 1));
@@ -249,7 +249,13 @@ DEV uint64_t lookback(const uint64_t *words, uint32_t ep, uint64_t t, uint64_t t
             // aggregate is already published (measured: polling after
             // s_sleep(1) made the power-law sample 5% slower; a short first
             // retry and then the longest gained nothing over the longest alone).
-            __builtin_amdgcn_s_sleep(127);
+            // Where every tile of the launch is in flight at once nothing else
+            // runs meanwhile, and a wait costs up to a whole back-off (2-3% of
+            // small queries, capped ones, batches and served streams).
+            if (ws.brief)
+                __builtin_amdgcn_s_sleep(8);
+            else
+                __builtin_amdgcn_s_sleep(127);
         }
         const uint64_t upto = pm ? (pm ^ (pm - 1)) : ~0ull;
         const uint64_t v = ((upto >> lane) & 1ull) ? (w & kValueMask) : 0ull;
@@ -314,8 +320,8 @@ DEV void tile_prefix(uint64_t t, uint64_t t0, const ScanWS &ws, uint32_t ep, Sca
                 st_word(ws.wk + t, pack(1, ep, ak));
                 st_word(ws.wc + t, pack(1, ep, ac));
             }
-            ek = lookback(ws.wk, ep, t, t0);
-            ec = lookback(ws.wc, ep, t, t0);
+            ek = lookback(ws, ws.wk, ep, t, t0);
+            ec = lookback(ws, ws.wc, ep, t, t0);
         }
         if (lane == 0) {
             st_word(ws.wk + t, pack(2, ep, ek + ak));
@@ -1890,8 +1896,10 @@ __global__ __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(4))) void
     // batch 16.4 -> 11.9 ms, 1,000 served queries 22.5 -> 17.0 ms by both).
     const uint32_t nwg = total < gridDim.x ? (uint32_t)total : gridDim.x;
     if (blockIdx.x >= nwg) return;
-    const uint32_t ep = read_epoch(cfg.ws);
-    tickets_init(cfg.ws, &sh.next);
+    ScanWS ws = cfg.ws;
+    ws.brief = total <= gridDim.x;
+    const uint32_t ep = read_epoch(ws);
+    tickets_init(ws, &sh.next);
     for (;;) {
         const uint64_t t = tickets_take(&sh.next);
         if (t >= total) break;
@@ -1906,25 +1914,25 @@ __global__ __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(4))) void
         const uint64_t t0 = B.tile0;
         const auto plan = gp(B.plan);  // loaded from memory: keep its reads global
         if (step == STEP_ROOT) {
-            root_tile<I>(cfg.g, B.rio, plan->nroot_chk, plan->root_chk_rel, t - t0, t, t0, cfg.ws, ep, sh.sm, &sh.next);
+            root_tile<I>(cfg.g, B.rio, plan->nroot_chk, plan->root_chk_rel, t - t0, t, t0, ws, ep, sh.sm, &sh.next);
         } else if (step == EXPAND_MID) {
             // the slot's step descriptor in scalar registers (measured: the
             // 256-query batch 36.3 against 39.3 ms)
             uint64_t c = 0, h0 = 0, h1 = 0;
             const StepIO io = uniform_copy(B.io);
             const uint32_t inj = (uint32_t)__builtin_amdgcn_readfirstlane((int)plan->depth[B.d].inj);
-            expand_tile<EXPAND_MID, I>(cfg.g, plan->depth[B.d], plan->col, plan->dcol, io, t - t0, t, t0, cfg.ws,
+            expand_tile<EXPAND_MID, I>(cfg.g, plan->depth[B.d], plan->col, plan->dcol, io, t - t0, t, t0, ws,
                                        ep, inj, 0u, cfg.pool_words, sh, smem, c, h0, h1);
         } else {
             uint64_t c = 0, h0 = 0, h1 = 0;
             const StepIO io = uniform_copy(B.io);
             const uint32_t inj = (uint32_t)__builtin_amdgcn_readfirstlane((int)plan->depth[B.d].inj);
             expand_tile<EXPAND_LAST_COUNT, I>(cfg.g, plan->depth[B.d], plan->col, plan->dcol, io, t - t0, t, t0,
-                                              cfg.ws, ep, inj, 0u, cfg.pool_words, sh, smem, c, h0, h1);
+                                              ws, ep, inj, 0u, cfg.pool_words, sh, smem, c, h0, h1);
             flush_sums(c, h0, h1, io.tot, sh.red);
         }
     }
-    finish_launch(cfg.ws, nwg);
+    finish_launch(ws, nwg);
 }
 
 // ---------------------------------------------------------------------------
