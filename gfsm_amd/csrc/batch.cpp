@@ -384,6 +384,7 @@ bool BatchEngine::try_admit(std::unique_ptr<BatchJob> &job, Status &st)
     s.max_depth_cand = job->opts.max_depth_cand;
     s.q = plan.q;
     s.digest = (job->opts.flags & GFSM_DIGEST) ? 1u : 0u;
+    s.tail = !s.digest && plan.q >= 3 && plan.dev.depth[plan.q - 1].nchk == 0;
     s.state = SLOT_NEW;
     s.step = STEP_NONE;
     n_admit_++;  // installed by the next replay's first scheduler launch

@@ -232,6 +232,8 @@ struct BatchSlot {
     uint64_t max_cand;            // work cap (0 = none)
     uint64_t max_depth_cand;      // deterministic per-depth cap (0 = none)
     uint32_t q, digest;
+    uint32_t tail, pad;           // depth q-2 counts the last depth's embeddings (EXPAND_TAIL); cleared
+                                  // by the scheduler once a cap ends inside a tail step
     uint32_t state;               // SLOT_NEW at admission
     uint32_t error;
     // Depth-first chunk walk, maintained by the scheduler.
@@ -281,7 +283,8 @@ struct BatchCfg {
     SlotReport *report;           // [nslots]
     SlotFinal *final;             // [nslots], written when a slot finishes
     uint64_t *tile_start;         // [nslots + 1]
-    uint64_t *tile_node;          // [2 * tiles of a step] frontier nodes of every expand tile (k_batch_tile_index)
+    uint64_t *tile_node;          // [2 * tiles of a step] frontier nodes of every expand tile
+                                  // (k_batch_tile_index); after the step, the sums of its tail tiles
     BatchCtl *ctl;
     uint32_t nslots;
     uint32_t items;               // candidates per thread (tile = 256 * items)

@@ -840,7 +840,7 @@ DEV void expand_tile(const DevGraphView &g, const DP &dp, CP col, CP dcol,
         if (sub == 0) sh.node[tid >> 5] = i;
     }
     __syncthreads();
-    if (KIND == EXPAND_LAST_COUNT && tickets) ticket_prefetch(ws, &sh.next);  // no look-back in this kind
+    if ((KIND == EXPAND_LAST_COUNT || TAIL) && tickets) ticket_prefetch(ws, &sh.next);  // no look-back in this kind
     const uint64_t ilo = sh.node[0];
     const uint32_t nf = (uint32_t)(sh.node[1] - ilo + 1);
     // The rows come first: every candidate reads its node's row (d words,
@@ -1501,13 +1501,57 @@ DEV uint64_t capped_chunk(const BatchSlot &B, uint32_t d, uint64_t n, uint64_t c
     return umax64(TC, umin64(umin64(chunk, umax64(need, floor)), limit));
 }
 
+// What a slot's finished tail step counted: the sums over its first tiles whose
+// last-depth candidates fit the cap, and how many tiles those are.
+struct TailSums {
+    uint64_t kept, cand, cnt, tiles;
+};
+
+// Last-depth candidates that the caps of slot B leave for its running tail step.
+DEV uint64_t tail_room(const BatchSlot &B)
+{
+    uint64_t room = ~0ull;
+    if (B.max_depth_cand) room = B.max_depth_cand - umin64(B.max_depth_cand, B.cand[B.q - 1]);
+    if (B.max_cand) room = umin64(room, B.max_cand - umin64(B.max_cand, B.cand_done));
+    return room;
+}
+
+// The sums of a slot's `n` tail tiles, by all 64 lanes of one wave.
+DEV TailSums wave_tail_sums(gptr_t<const uint64_t> sums, uint64_t n, uint64_t room)
+{
+    const uint32_t lane = lane_id();
+    TailSums r{0, 0, 0, n};
+    for (uint64_t t0 = 0; t0 < n; t0 += 64) {
+        const uint64_t t = t0 + lane;
+        const uint64_t e = t < n ? sums[2 * t] : 0ull, p = t < n ? sums[2 * t + 1] : 0ull;
+        const uint64_t c = p & ((1ull << kTailKeptShift) - 1);
+        uint64_t inc = c;
+        for (uint32_t o = 1; o < 64; o <<= 1) {
+            const uint64_t v = __shfl_up(inc, o, 64);
+            if (lane >= o) inc += v;
+        }
+        const bool fit = r.cand + inc <= room;
+        r.kept += wave_sum64(fit ? p >> kTailKeptShift : 0ull);
+        r.cnt += wave_sum64(fit ? e : 0ull);
+        const uint64_t cand = wave_sum64(fit ? c : 0ull);
+        const uint64_t m = __ballot(fit);
+        r.cand += cand;
+        if (m != ~0ull) {
+            r.tiles = t0 + (uint64_t)__builtin_ctzll(~m);
+            break;
+        }
+    }
+    return r;
+}
+
 // Consume the finished step of slot B (depth-first chunk walk), then
 // schedule its next step.  B may be a copy of the slot; `tot` is the slot's
-// own totals word block, which the step writes.  Returns the new step's tile count (0 when the slot
+// own totals word block, which the step writes; `ts` the sums of a finished tail
+// step.  Returns the new step's tile count (0 when the slot
 // has no step).  Mirrors the single-query driver's recursion: a level that
 // overflows its buffer is retried on half the range; otherwise the chunk is
 // re-estimated from the observed selectivity.
-DEV uint32_t schedule_slot(const BatchCfg &cfg, BatchSlot &B, Totals *tot)
+DEV uint32_t schedule_slot(const BatchCfg &cfg, BatchSlot &B, Totals *tot, const TailSums &ts)
 {
     const uint64_t TC = (uint64_t)kTile * cfg.items;
     const uint64_t by_val = kValueMask / umax64(cfg.max_degree, 1);
@@ -1524,6 +1568,7 @@ DEV uint32_t schedule_slot(const BatchCfg &cfg, BatchSlot &B, Totals *tot)
             B.chunk[k] = (k + 1 < q) ? umin64(B.cap[k], limit) : limit;
         }
         B.chunk[0] = umax64(TC, umin64(B.cap[0], limit));
+        if (B.tail && q >= 3) B.chunk[q - 2] = limit;  // writes no level
         if (B.max_depth_cand) {  // capped: start small, grow from the observed fan-out
             B.chunk[0] = umax64(TC, umin64(B.chunk[0], umax64(B.max_depth_cand / 64, floor)));
             for (uint32_t k = 1; k < GFSM_MAXQ; k++) B.chunk[k] = 0;  // set at the depth's first step
@@ -1569,6 +1614,26 @@ DEV uint32_t schedule_slot(const BatchCfg &cfg, BatchSlot &B, Totals *tot)
                     B.chunk[d] = umin64(B.chunk[d] * 4, limit);
                 }
             }
+        } else if (B.step == EXPAND_TAIL) {
+            B.steps++;
+            uint64_t to = e;
+            if (ts.tiles < B.io.ntiles) {
+                // The cap's last candidate falls in the next tile, which is
+                // expanded level by level and ends the match.
+                to = b + ts.tiles * TC;
+                B.cand_done -= e - to;
+                B.tail = 0;
+            }
+            if (B.max_depth_cand && to > b)
+                B.chunk[d] = capped_chunk(B, d, to - b, ts.cand, limit, TC, limit, floor);
+            if (!B.tail) B.chunk[d] = TC;
+            B.lo[d] = to;
+            B.cand[d] += to - b;
+            B.level[d] += ts.kept;
+            B.cand[d + 1] += ts.cand;
+            B.level[d + 1] += ts.cnt;
+            B.cand_done += ts.cand;
+            B.count += ts.cnt;
         } else if (B.step == EXPAND_LAST_COUNT) {
             B.steps++;
             B.lo[d] = e;
@@ -1609,7 +1674,9 @@ DEV uint32_t schedule_slot(const BatchCfg &cfg, BatchSlot &B, Totals *tot)
         return 0;
     }
     if (d >= 1) {
-        const uint32_t kind = (d == (int32_t)q - 1) ? (uint32_t)EXPAND_LAST_COUNT : (uint32_t)EXPAND_MID;
+        const uint32_t kind = (d == (int32_t)q - 1)                ? (uint32_t)EXPAND_LAST_COUNT
+                              : (B.tail && d == (int32_t)q - 2) ? (uint32_t)EXPAND_TAIL
+                                                                : (uint32_t)EXPAND_MID;
         const uint64_t b = B.lo[d];
         if (!B.chunk[d])
             B.chunk[d] = umax64(TC, umin64(umin64(kind == EXPAND_MID ? B.cap[d] : limit, limit),
@@ -1641,8 +1708,8 @@ DEV uint32_t schedule_slot(const BatchCfg &cfg, BatchSlot &B, Totals *tot)
             io.out_off = B.off[d];
             io.out_gbeg = B.gbeg[d];
             io.cap = B.cap[d];
-            io.need_nxt = dp.nxt_dist > 1 ? 1u : 0u;
         }
+        io.need_nxt = kind != EXPAND_LAST_COUNT && dp.nxt_dist > 1 ? 1u : 0u;
         io.tot = tot;
         io.ntiles = (e - b + TC - 1) / TC;
         io.d = (uint32_t)d;
@@ -1759,9 +1826,12 @@ __global__ __launch_bounds__(kTile) void k_batch_schedule(BatchCfg cfg)
         wave_sync_lds();
         BatchSlot &B = *reinterpret_cast<BatchSlot *>(lw);
         uint32_t fin = 0;
+        TailSums ts{0, 0, 0, 0};
+        if (B.state == SLOT_RUN && B.step == EXPAND_TAIL)
+            ts = wave_tail_sums(gp((const uint64_t *)cfg.tile_node) + 2 * B.tile0, B.io.ntiles, tail_room(B));
         if (lane == 0) {
             const uint32_t before = B.state;
-            const uint32_t nt = schedule_slot(cfg, B, &cfg.slots[s].tot);
+            const uint32_t nt = schedule_slot(cfg, B, &cfg.slots[s].tot, ts);
             fin = (B.state >= SLOT_DONE && before < SLOT_DONE) ? 1u : 0u;  // just finished: its statistics
             SlotReport &rp = cfg.report[s];
             rp.state = B.state;
@@ -1769,7 +1839,7 @@ __global__ __launch_bounds__(kTile) void k_batch_schedule(BatchCfg cfg)
             rp.count = B.count;
             rp.dg0 = B.dg0;
             rp.dg1 = B.dg1;
-            const bool indexed = nt && (B.step == EXPAND_MID || B.step == EXPAND_LAST_COUNT);
+            const bool indexed = nt && B.step != STEP_ROOT;
             tile_start[s] = (uint64_t)nt | (B.state == SLOT_RUN ? kSchedRun : 0ull) | (indexed ? kSchedIndexed : 0ull);
         }
         fin = __builtin_amdgcn_readfirstlane(fin);
@@ -1870,7 +1940,7 @@ __global__ __launch_bounds__(kTile) void k_batch_tile_index(BatchCfg cfg)
     for (uint64_t t = ((uint64_t)blockIdx.x * kTile + threadIdx.x) >> 6; t < total; t += nwaves) {
         const uint32_t s = slot_search(cfg.tile_start, cfg.nslots, t);
         const BatchSlot &B = cfg.slots[s];
-        if (B.step != EXPAND_MID && B.step != EXPAND_LAST_COUNT) continue;
+        if (B.step != EXPAND_MID && B.step != EXPAND_LAST_COUNT && B.step != EXPAND_TAIL) continue;
         const uint64_t lt = t - B.tile0;
         const uint64_t c0 = B.io.g_begin + lt * TC;
         const uint64_t c1 = (c0 + TC < B.io.g_end) ? c0 + TC : B.io.g_end;
@@ -1923,6 +1993,14 @@ __global__ __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(4))) void
             const uint32_t inj = (uint32_t)__builtin_amdgcn_readfirstlane((int)plan->depth[B.d].inj);
             expand_tile<EXPAND_MID, I>(cfg.g, plan->depth[B.d], plan->col, plan->dcol, io, t - t0, t, t0, ws,
                                        ep, inj, 0u, cfg.pool_words, sh, smem, c, h0, h1);
+        } else if (step == EXPAND_TAIL) {
+            uint64_t c = 0, kept = 0, cand = 0;
+            const StepIO io = uniform_copy(B.io);
+            const uint32_t inj = (uint32_t)__builtin_amdgcn_readfirstlane((int)plan->depth[B.d].inj);
+            const uint32_t linj = (uint32_t)__builtin_amdgcn_readfirstlane((int)plan->depth[B.d + 1].inj);
+            expand_tile<EXPAND_TAIL, I>(cfg.g, plan->depth[B.d], plan->col, plan->dcol, io, t - t0, t, t0, ws, ep, inj,
+                                        linj, cfg.pool_words, sh, smem, c, kept, cand);
+            tail_tile_sums(cfg.tile_node, t, c, kept, cand, sh.red);
         } else {
             uint64_t c = 0, h0 = 0, h1 = 0;
             const StepIO io = uniform_copy(B.io);
