@@ -39,6 +39,7 @@ static double now_ms()
 
 static uint64_t round_up(uint64_t b, uint64_t a) { return (b + a - 1) / a * a; }
 static constexpr uint64_t kRegionAlign = 2ull << 20;
+static constexpr uint64_t kMinStepCand = 1ull << 20;  // candidates of a slot's step, however many run
 static constexpr uint64_t kMinLevelNodes = 8 * kTile;  // >= the largest tile's survivors
 
 // ---------------------------------------------------------------------------
@@ -204,7 +205,10 @@ Status BatchEngine::init(const BatchShape &shape, uint64_t arena_bytes, char *ar
     // The per-slot step size is step_budget / running (set before each
     // replay), so one step needs at most step_budget / tc + n tiles.
     shape_.step_budget = std::max<uint64_t>(tc, std::min<uint64_t>(shape_.step_budget, (max_tiles - n) * tc));
-    st = lane_.init(max_tiles, true);
+    // (a slot's step is at least kMinStepCand however many run: see replay)
+    step_limit_ = (max_tiles - n) / n * tc;
+    const uint64_t most = std::max<uint64_t>(shape_.step_budget, n * std::min(kMinStepCand, step_limit_)) / tc + n;
+    st = lane_.init(max_tiles, true, std::min(most, max_tiles));
     if (!st.good()) return st;
     HIP_TRY(hipMalloc(&slots_d_, sizeof(BatchSlot) * n));
     HIP_TRY(hipMalloc(&report_d_, sizeof(SlotReport) * n));
@@ -253,6 +257,7 @@ Status BatchEngine::init(const BatchShape &shape, uint64_t arena_bytes, char *ar
     cfg_.final = final_d_;
     cfg_.tile_start = tile_start_d_;
     cfg_.tile_node = lane_.tile_node;
+    cfg_.tail_sums = lane_.tail_sums;
     cfg_.ctl = ctl_d_;
     cfg_.nslots = n;
     cfg_.items = shape_.items;
@@ -384,7 +389,8 @@ bool BatchEngine::try_admit(std::unique_ptr<BatchJob> &job, Status &st)
     s.max_depth_cand = job->opts.max_depth_cand;
     s.q = plan.q;
     s.digest = (job->opts.flags & GFSM_DIGEST) ? 1u : 0u;
-    s.tail = !s.digest && plan.q >= 3 && plan.dev.depth[plan.q - 1].nchk == 0;
+    s.tail = 0;
+    for (uint32_t m = 1; !s.digest && m <= GFSM_MAXTAIL && plan.dev.tail[m - 1].m; m++) s.tail = m;
     s.state = SLOT_NEW;
     s.step = STEP_NONE;
     n_admit_++;  // installed by the next replay's first scheduler launch
@@ -399,8 +405,9 @@ Status BatchEngine::replay()
     // Per-slot step size: the step budget shared by the running slots, so a
     // lone query takes large steps and a full batch keeps steps short.
     const uint64_t tc = (uint64_t)kTile * shape_.items;
-    const uint64_t want = std::max<uint64_t>(
-        tc, std::min<uint64_t>(shape_.step_budget, std::max<uint64_t>(1ull << 20, shape_.step_budget / std::max<uint32_t>(running_, 1))));
+    uint64_t want = std::max<uint64_t>(kMinStepCand, shape_.step_budget / std::max<uint32_t>(running_, 1));
+    want = std::max<uint64_t>(tc, std::min<uint64_t>(shape_.step_budget, want));
+    if (want * running_ > shape_.step_budget) want = std::max<uint64_t>(tc, std::min(want, step_limit_));
     if (want != step_cand_) {
         *step_cand_h_ = want;
         HIP_TRY(hipMemcpyAsync(&ctl_d_->step_cand, step_cand_h_, sizeof(uint64_t), hipMemcpyHostToDevice,
@@ -554,7 +561,7 @@ Status match_batch_shaped(Ctx &ctx, const HostGraph &data, const std::vector<con
         job->id = i;
         job->query = queries[i];
         job->opts = o;
-        Status st = plan_for(data, *queries[i], o, job->plan);
+        Status st = plan_for(data, *queries[i], o, job->plan, false);
         if (!st.good()) {
             out[i].status = st.code;
             continue;

@@ -35,9 +35,11 @@ static double now_ms()
         if (e_ != hipSuccess) return hip_status(e_, #expr);              \
     } while (0)
 
-Status Lane::init(uint64_t max_tiles, bool tile_index)
+Status Lane::init(uint64_t max_tiles, bool tile_index, uint64_t tail)
 {
     if (tile_index) HIP_TRY(hipMalloc(&tile_node, 2 * max_tiles * sizeof(uint64_t)));
+    tail_tiles = tail;
+    HIP_TRY(hipMalloc(&tail_sums, kTailWords * tail_tiles * sizeof(uint64_t)));
     HIP_TRY(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
     ws.max_tiles = max_tiles;
     HIP_TRY(hipMalloc(&ws.wk, max_tiles * sizeof(uint64_t)));
@@ -50,8 +52,8 @@ Status Lane::init(uint64_t max_tiles, bool tile_index)
     HIP_TRY(hipMemset(tot_d, 0, sizeof(Totals)));
     HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&tot_h), sizeof(Totals), hipHostMallocDefault));
     std::memset(tot_h, 0, sizeof(Totals));
-    HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&kc_h), 4 * sizeof(uint64_t), hipHostMallocCoherent));
-    std::memset(kc_h, 0, 4 * sizeof(uint64_t));
+    HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&kc_h), kHostWords * sizeof(uint64_t), hipHostMallocCoherent));
+    std::memset(kc_h, 0, kHostWords * sizeof(uint64_t));
     for (int i = 0; i < 2; i++) HIP_TRY(hipEventCreate(&ev[i]));
     return Status::ok();
 }
@@ -74,6 +76,7 @@ void Lane::destroy()
     (void)hipFree(ws.ctl);
     (void)hipFree(tile_node);
     tile_node = nullptr;
+    (void)hipFree(tail_sums);
     (void)hipFree(tot_d);
     if (tot_h) (void)hipHostFree(tot_h);
     if (kc_h) (void)hipHostFree(kc_h);
@@ -296,13 +299,17 @@ Status upload_graph(Ctx &ctx, const HostGraph &g, DevGraph *&out)
     return Status::ok();
 }
 
-Status plan_for(const HostGraph &data, const HostGraph &query, const gfsm_match_opts &o, Plan &plan)
+Status plan_for(const HostGraph &data, const HostGraph &query, const gfsm_match_opts &o, Plan &plan,
+                bool wide_tails)
 {
     const bool by_cost = o.flags & GFSM_ORDER_COST;
     if (by_cost && (o.root_lo || o.root_hi))
         return Status::err(GFSM_ERR_ARG, "root windows refer to the reference order's root; not with GFSM_ORDER_COST");
     Status st = plan_query(query, plan, by_cost ? &data : nullptr);
-    if (st.good()) set_injectivity(data, plan);
+    if (st.good()) {
+        set_injectivity(data, plan);
+        set_tails(data, plan, wide_tails);
+    }
     return st;
 }
 
@@ -415,7 +422,7 @@ struct Runner {
     Result &res;
     uint32_t q = 0;
     bool rows_mode = false, digest = false, prof = false;
-    bool tail = false;          // depth q-2 counts the last depth's embeddings (EXPAND_TAIL)
+    uint32_t leaves = 0;        // depths at the end counted without placing them (EXPAND_TAIL)
     uint64_t tail_count = 0;    // embeddings counted by capped tail steps
     uint32_t *vec[GFSM_MAXQ] = {}, *gbeg[GFSM_MAXQ] = {};
     uint64_t *off[GFSM_MAXQ] = {};
@@ -457,7 +464,7 @@ struct Runner {
     // (Only when the next generator is an older ancestor, not the new vertex.)
     uint32_t need_nxt(uint32_t kind, uint32_t d) const
     {
-        return ((kind == EXPAND_MID || kind == EXPAND_TAIL) && plan.dev.depth[d].nxt_dist > 1) ? 1u : 0u;
+        return (kind == EXPAND_MID && plan.dev.depth[d].nxt_dist > 1) ? 1u : 0u;
     }
 
     // Candidates per thread for one expand launch: forced, else tuned.
@@ -489,7 +496,9 @@ struct Runner {
         rows_mode = flags & (GFSM_ROWS | GFSM_SORTED);
         digest = (flags & GFSM_DIGEST) && !rows_mode;  // rows mode: digest from the host rows
         prof = flags & GFSM_PROFILE;
-        tail = (lane.kc_h && lane.tile_node) && !rows_mode && !digest && q >= 3 && plan.dev.depth[q - 1].nchk == 0;
+        leaves = 0;
+        if (!rows_mode && !digest && lane.kc_h && lane.tail_sums)
+            for (uint32_t m = 1; m <= GFSM_MAXTAIL && plan.dev.tail[m - 1].m; m++) leaves = m;
         grid_cap = std::max<uint32_t>(ctx.num_cus, 1) * ctx.tune.wgs_per_cu;
         const uint64_t min_nodes = 8 * kTile;  // a level must hold one launch tile's survivors
         uint64_t row_bytes = 0;
@@ -511,7 +520,7 @@ struct Runner {
             chunk[k + 1] = std::min<uint64_t>(c, launch_limit());
         }
         chunk[q - 1] = launch_limit();
-        if (tail) chunk[q - 2] = launch_limit();  // writes no level
+        if (leaves) chunk[q - 1 - leaves] = launch_limit();  // writes no level
         char *p = nullptr;
         if (fixed) {
             if (total > fixed->bytes)
@@ -708,16 +717,21 @@ struct Runner {
         // registers under 64 for eight waves per SIMD).
         const bool bare = last && !rows_mode && !digest && plan.dev.depth[d].nchk == 0 &&
                           !(forced_items > kBareItems);
-        const bool at_tail = tail && d + 2 == q;
+        // The tail: every later depth is a leaf.  Deeper than its first depth
+        // only where a cap ended inside a tail step.
+        const bool at_tail = !last && d + 1 + leaves >= q;
+        const TailPlanDev *tp = at_tail ? &plan.dev.tail[q - 2 - d] : nullptr;
+        const uint32_t m = at_tail ? tp->m : 0u;
         const uint32_t inner_kind =
             last ? (rows_mode ? EXPAND_LAST_ROWS : (bare ? EXPAND_LAST_BARE : EXPAND_LAST_COUNT)) : EXPAND_MID;
         const uint64_t tile_limit = launch_limit();
         const uint32_t items = bare ? std::min(pick_items(EXPAND_LAST_COUNT, d), bare_items(g1 - g0, S_prev, d))
-                                    : pick_items(inner_kind, d);
+                                    : at_tail && tp->wide ? std::min(pick_items(inner_kind, d), kWideItems)
+                                                          : pick_items(inner_kind, d);
         const uint32_t pool_words = bare ? std::min(ctx.tune.pool_words, kBarePoolWords) : ctx.tune.pool_words;
         const uint32_t grid_mul = bare ? 2 : 1;  // twice the resident workgroups
         const uint64_t tc = (uint64_t)kTile * items;
-        const bool capped = max_depth_cand || max_cand;  // then lane.kc_h and lane.tile_node are there
+        const bool capped = max_depth_cand || max_cand;
         uint64_t untailed = g0;  // candidates before it take the two steps (a cap ends inside them)
         bool first = true;
         for (uint64_t c = g0; c < g1;) {
@@ -730,6 +744,7 @@ struct Runner {
                 if (depth_done[d] >= max_depth_cand) return Status::err(GFSM_ERR_CAP, "per-depth candidate cap reached");
                 e = std::min(e, c + (max_depth_cand - depth_done[d]));
             }
+            if (kind == EXPAND_TAIL && capped) e = std::min(e, c + lane.tail_tiles * tc);
             if (at_tail && kind == EXPAND_MID)  // writes the level, up to the range's end
                 e = std::min(e, std::min(untailed, c + std::max<uint64_t>(tc, cap[d])));
             ExpandArgs a{};
@@ -742,12 +757,18 @@ struct Runner {
             StepIO &io = a.io;
             io.need_nxt = need_nxt(kind, d);
             if (kind == EXPAND_TAIL) {
-                a.linj = plan.dev.depth[d + 1].inj;
-                a.tail_sums = lane.tile_node;
-                a.room = max_depth_cand ? max_depth_cand - std::min(max_depth_cand, depth_done[d + 1]) : ~0ull;
-                if (max_cand) a.room = std::min(a.room, max_cand - std::min(max_cand, cand_total + (e - c)));
+                a.tail = *tp;
+                for (uint32_t i = 0; i < m; i++) {
+                    TailLeafDev &l = a.tail.leaf[i];
+                    l.tab = dense(l.rel, e - c);
+                    for (uint32_t r = 0; r < l.nchk; r++) l.chk_tab[r] = dense(l.chk_rel[r], e - c);
+                    a.room[i] = max_depth_cand ? max_depth_cand - std::min(max_depth_cand, depth_done[d + 1 + i]) : ~0ull;
+                }
+                // All candidates count for max_cand, so it bounds the leaves together.
+                a.room_all = max_cand ? max_cand - std::min(max_cand, cand_total + (e - c)) : ~0ull;
+                a.tail_sums = lane.tail_sums;
             }
-            if (kind == EXPAND_MID || kind == EXPAND_TAIL)
+            if (kind == EXPAND_MID)
                 a.dp.nxt_seg = dense(plan.dev.depth[d].nxt_rel, e - c);
             for (uint32_t r = 0; r < std::min<uint32_t>(plan.dev.depth[d].nchk, kDenseChk); r++)
                 a.dp.chk_seg[r] = dense(plan.dev.depth[d].chk_rel[r], e - c);
@@ -818,7 +839,7 @@ struct Runner {
                     st = sync_step_totals(io.host_kc, true);
                     if (!st.good()) return st;
                     const volatile uint64_t *w = reinterpret_cast<const volatile uint64_t *>(io.host_kc);
-                    const uint64_t kept = w[0], cnt = w[1], emb = w[2], tiles = w[3];
+                    const uint64_t tiles = w[0];
                     if (tiles < io.ntiles) {
                         // The cap's last candidate falls in tile `tiles`: that tile
                         // is expanded level by level, which stops there.
@@ -827,12 +848,20 @@ struct Runner {
                         cand_total -= e - to;
                         e = to;
                     }
-                    if (max_depth_cand && e > c) chunk[d] = capped_chunk(d, e - c, cnt, tile_limit, tc);
-                    cand_total += cnt;
-                    tail_count += emb;
-                    res.stats.level[d] += kept;
-                    res.stats.cand[d + 1] += cnt;
-                    depth_done[d + 1] += cnt;
+                    if (max_depth_cand && e > c) {
+                        uint64_t ch = tile_limit;
+                        for (uint32_t i = 0; i < m; i++) ch = capped_chunk(d + i, e - c, w[2 + 2 * i], ch, tc);
+                        chunk[d] = ch;
+                    }
+                    res.stats.level[d] += w[1];
+                    for (uint32_t i = 0; i < m; i++) {
+                        const uint64_t cnt = w[2 + 2 * i];
+                        cand_total += cnt;
+                        res.stats.cand[d + 1 + i] += cnt;
+                        depth_done[d + 1 + i] += cnt;
+                        if (i + 1 < m) res.stats.level[d + 1 + i] += w[3 + 2 * i];
+                    }
+                    tail_count += w[1 + 2 * m];
                 }
                 res.stats.cand[d] += e - c;
                 depth_done[d] += e - c;
@@ -1090,9 +1119,14 @@ Status run_match(Ctx &ctx, const HostGraph &data, const DevGraph &dg, const Plan
         if (o.flags & GFSM_SORTED) sort_rows(res.rows, q);
     } else {
         res.count = L.tot_h->count + run.tail_count;
-        if (run.tail && !o.max_depth_cand && !o.max_cand) {
-            res.stats.level[q - 2] = L.tot_h->tail_keep;
-            res.stats.cand[q - 1] = L.tot_h->tail_cand;
+        if (run.leaves && !o.max_depth_cand && !o.max_cand) {
+            const uint32_t m = run.leaves, d = q - 1 - m;
+            res.stats.level[d] = L.tot_h->tail[0];
+            for (uint32_t i = 0; i < m; i++) {
+                res.stats.cand[d + 1 + i] = L.tot_h->tail[1 + 2 * i];
+                res.stats.level[d + 1 + i] = L.tot_h->tail[2 + 2 * i];
+            }
+            res.count = L.tot_h->tail[2 * m];
         }
         res.stats.level[q - 1] = res.count;
         res.digest[0] = L.tot_h->dg0;
@@ -1196,6 +1230,8 @@ Status match_noalloc(Ctx &ctx, const HostGraph &data, const HostGraph &query, co
     L.ws.wc = L.ws.wk + kNoAllocTiles;
     L.tile_node = L.ws.wc + kNoAllocTiles;
     L.ws.max_tiles = kNoAllocTiles;
+    L.tail_sums = L.tile_node + 2 * kNoAllocTiles;
+    L.tail_tiles = kNoAllocTailTiles;
     Arena levels;
     levels.base = p + kNoAllocWorkBytes;
     levels.bytes = kNoAllocLevelBytes;

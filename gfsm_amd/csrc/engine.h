@@ -55,7 +55,9 @@ struct Lane {
     std::vector<hipEvent_t> kev;  // begin/end pairs of timed launches (grown on demand)
     uint64_t launches = 0;  // chained-scan launches issued on this lane
     uint64_t *tile_node = nullptr;  // [2*max_tiles] per-tile frontier nodes (single-query lane only)
-    Status init(uint64_t max_tiles, bool tile_index = false);
+    uint64_t *tail_sums = nullptr;  // [kTailWords*tail_tiles] sums of a capped tail step's tiles
+    uint64_t tail_tiles = 0;
+    Status init(uint64_t max_tiles, bool tile_index = false, uint64_t tail_tiles = kTailTiles);
     // Call before every chained-scan launch: clears the tile words when the
     // 16-bit launch epoch is about to repeat.
     hipError_t before_launch();
@@ -145,7 +147,9 @@ std::mutex &noalloc_mutex(int device);
 
 // The query's plan for these options: the reference order, or with
 // GFSM_ORDER_COST the data-statistics order (root windows then rejected).
-Status plan_for(const HostGraph &data, const HostGraph &query, const gfsm_match_opts &o, Plan &plan);
+// wide_tails: see set_tails (the batch step kernel has no wide ones).
+Status plan_for(const HostGraph &data, const HostGraph &query, const gfsm_match_opts &o, Plan &plan,
+                bool wide_tails = true);
 
 // Matcher helpers shared with the batched and serving paths.
 void root_range(const HostGraph &data, const Plan &plan, uint32_t root_lo, uint32_t root_hi, uint64_t &lo,

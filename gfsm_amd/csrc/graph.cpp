@@ -199,19 +199,21 @@ Status build_graph(uint32_t nv, const uint32_t *vlabel, uint64_t ne, const uint3
     uint64_t nd = g->dir_ptr[nv];
     g->dir.resize(nd + 1);
     g->nbr.resize(ne);
-    std::atomic<bool> loops{false};
+    std::atomic<bool> loops{false}, dups{false};
     parallel_for(nv, [&](uint64_t b, uint64_t e) {
         for (uint64_t v = b; v < e; v++) {
             uint32_t j = g->dir_ptr[v];
             for (uint64_t p = rowp[v]; p < rowp[v + 1]; p++) {
                 g->nbr[p] = (uint32_t)sorted[p];
                 if (g->nbr[p] == v) loops = true;
+                if (p > rowp[v] && sorted[p] == sorted[p - 1]) dups = true;
                 if (p == rowp[v] || (sorted[p] >> 32) != (sorted[p - 1] >> 32))
                     g->dir[j++] = DirEnt{(uint32_t)(sorted[p] >> 32), (uint32_t)p};
             }
         }
     });
     g->has_loops = loops;
+    g->has_dups = dups;
     g->dir[nd] = DirEnt{0xFFFFFFFFu, (uint32_t)ne};
     std::vector<uint64_t>().swap(sorted);
 

@@ -160,15 +160,20 @@ bool layout_ok(const HostGraph &g)
     return !bad;
 }
 
-bool any_loop(const HostGraph &g)
+// has_loops and has_dups, as build_graph finds them.
+void find_loops_dups(HostGraph &g)
 {
-    std::atomic<bool> loops{false};
+    std::atomic<bool> loops{false}, dups{false};
     parallel_for(g.V, [&](uint64_t b, uint64_t e) {
         for (uint64_t x = b; x < e; x++)
-            for (uint32_t p = g.dir[g.dir_ptr[x]].beg; p < g.dir[g.dir_ptr[x + 1]].beg; p++)
-                if (g.nbr[p] == x) loops = true;
+            for (uint32_t j = g.dir_ptr[x]; j < g.dir_ptr[x + 1]; j++)
+                for (uint32_t p = g.dir[j].beg; p < g.dir[j + 1].beg; p++) {
+                    if (g.nbr[p] == x) loops = true;
+                    if (p > g.dir[j].beg && g.nbr[p] == g.nbr[p - 1]) dups = true;
+                }
     });
-    return loops;
+    g.has_loops = loops;
+    g.has_dups = dups;
 }
 
 }  // namespace
@@ -234,7 +239,7 @@ Status load_bin(const char *path, HostGraph *&out)
     if (!ok) return Status::err(GFSM_ERR_INVALID_DATA, "truncated graph image");
     if (payload_checksum(*g) != h.checksum) return Status::err(GFSM_ERR_INVALID_DATA, "graph image checksum mismatch");
     if (!layout_ok(*g)) return Status::err(GFSM_ERR_INVALID_DATA, "graph image layout is inconsistent");
-    g->has_loops = any_loop(*g);
+    find_loops_dups(*g);
     out = g.release();
     return Status::ok();
 }

@@ -56,6 +56,7 @@ struct HostGraph {
     std::vector<uint32_t> rel_vtx, rel_beg, rel_cnt;
     uint32_t max_degree = 0;
     bool has_loops = true;  // some entry x -> x (whatever its relation)
+    bool has_dups = true;   // some segment holds a target twice
     uint64_t nent() const { return nbr.size(); }
     uint64_t ndir() const { return dir.empty() ? 0 : dir.size() - 1; }
 
@@ -109,6 +110,9 @@ struct Plan {
 };
 // Fill the plan's injectivity masks (DepthPlanDev::inj) for a data graph.
 void set_injectivity(const HostGraph &data, Plan &plan);
+// Fill the plan's tails (QueryPlanDev::tail) for a data graph; `wide`: leaves
+// with checks and pairs too, where the graph allows them.  After set_injectivity.
+void set_tails(const HostGraph &data, Plan &plan, bool wide);
 // The reference's matching order, or with `by_cost` (a data graph) the
 // order chosen from its relation statistics.
 Status plan_query(const HostGraph &query, Plan &out, const HostGraph *by_cost = nullptr);

@@ -51,8 +51,7 @@ struct Totals {
     uint64_t cnt;     // candidates of the next depth
     uint64_t count;   // last level, count-only: embeddings
     uint64_t dg0, dg1;// digest sums
-    uint64_t tail_keep, tail_cand; // tail steps: nodes kept, candidates of the last depth (sums)
-    uint64_t pad;
+    uint64_t tail[2 * GFSM_MAXTAIL + 1]; // tail steps: sums of nodes kept, then {candidates, nodes kept} per leaf
 };
 
 enum ExpandKind : uint32_t {
@@ -61,8 +60,9 @@ enum ExpandKind : uint32_t {
     EXPAND_LAST_ROWS = 2,  // last depth: write rows in original ids (and digest)
     EXPAND_LAST_BARE = 3,  // last depth, count only, no checks and no digest: a lean kernel
                            // that fits twice the resident workgroups of the others
-    EXPAND_TAIL = 4,       // depth q-2 of a count whose last depth has no checks: the survivors'
-                           // children are counted from their segments, no level is written
+    EXPAND_TAIL = 4,       // the last depth before a count's leaves (TailPlanDev): the survivors'
+                           // completions are counted from the leaves' segments, no level is written
+    EXPAND_TAIL_WIDE = 5,  // ... whose leaves have checks or pairs (TailPlanDev::wide; kernel selection only)
 };
 constexpr uint32_t kBarePoolWords = 2048;  // LDS pool of the lean last-depth kernel
 
@@ -97,6 +97,9 @@ struct StepIO {
                                // so the host reads a step's totals without a copy (a capped
                                // EXPAND_TAIL: see ExpandArgs::room)
 };
+constexpr uint32_t kTailWords = 8;  // words of a tail tile's sums (2 * GFSM_MAXTAIL + 1 used)
+constexpr uint32_t kTailTiles = 1u << 18;  // tiles of a capped tail step (sums buffer)
+constexpr uint32_t kHostWords = 16;        // host words of a step's totals (Lane::kc_h)
 constexpr uint32_t kNbrPad = 4;     // words allocated past nbr's end (four-word loads of a segment's end)
 constexpr uint32_t kDenseChk = 4;  // checked relations per depth with a dense-table slot (DepthPlanDev)
 
@@ -124,14 +127,13 @@ struct ExpandArgs {
     ScanWS ws;
     uint32_t items;            // candidates per thread: 1, 2, 4 or 8 (tile = 256 * items)
     uint32_t pool_words;       // LDS words for per-node staging (checked segments, rows)
-    uint32_t linj;             // EXPAND_TAIL: injectivity mask of the last depth
-    uint32_t pad;
-    // EXPAND_TAIL under a cap (io.host_kc set): last-depth candidates left.  The
-    // step counts its first tiles whose candidates fit and tells the host {nodes
-    // kept, candidates, embeddings, tiles} of those; nothing goes to io.tot.
-    uint64_t room;
-    uint64_t *tail_sums;       // [2*ntiles] the tiles' {embeddings, kept and candidates}; may be
-                               // io.tile_node's array (a tile reads its entries before it writes them)
+    TailPlanDev tail;          // EXPAND_TAIL: the leaves
+    // EXPAND_TAIL under a cap (io.host_kc set): candidates left to every leaf's
+    // depth.  The step counts its first tiles whose candidates fit and tells the
+    // host {tiles, sums of those as Totals::tail}; nothing goes to io.tot.
+    uint64_t room[GFSM_MAXTAIL];
+    uint64_t room_all;         // ... and to all of them together
+    uint64_t *tail_sums;       // [kTailWords * ntiles]
 };
 
 struct RootArgs {
@@ -161,6 +163,7 @@ hipError_t launch_single(const SingleArgs &a, uint32_t grid, hipStream_t s);
 
 constexpr uint32_t kTile = 256;     // threads per workgroup
 constexpr uint32_t kItems = 8;      // default candidates per thread per tile
+constexpr uint32_t kWideItems = 4;  // most candidates per thread of a tail step with checks or pairs
 constexpr uint32_t kRootItems = 4;  // root level (single-query path)
 constexpr uint32_t kRootTile = kTile * kRootItems;
 constexpr uint32_t kPoolWords = 7680;  // default staging pool (30 KB: four workgroups fit a CU's LDS)
@@ -232,8 +235,8 @@ struct BatchSlot {
     uint64_t max_cand;            // work cap (0 = none)
     uint64_t max_depth_cand;      // deterministic per-depth cap (0 = none)
     uint32_t q, digest;
-    uint32_t tail, pad;           // depth q-2 counts the last depth's embeddings (EXPAND_TAIL); cleared
-                                  // by the scheduler once a cap ends inside a tail step
+    uint32_t tail, pad;           // leaves counted without being placed (EXPAND_TAIL); the scheduler takes
+                                  // one off once a cap ends inside a tail step
     uint32_t state;               // SLOT_NEW at admission
     uint32_t error;
     // Depth-first chunk walk, maintained by the scheduler.
@@ -283,8 +286,8 @@ struct BatchCfg {
     SlotReport *report;           // [nslots]
     SlotFinal *final;             // [nslots], written when a slot finishes
     uint64_t *tile_start;         // [nslots + 1]
-    uint64_t *tile_node;          // [2 * tiles of a step] frontier nodes of every expand tile
-                                  // (k_batch_tile_index); after the step, the sums of its tail tiles
+    uint64_t *tile_node;          // [2 * tiles of a step] frontier nodes of every expand tile (k_batch_tile_index)
+    uint64_t *tail_sums;          // [kTailWords * tiles of a step] sums of every tail tile
     BatchCtl *ctl;
     uint32_t nslots;
     uint32_t items;               // candidates per thread (tile = 256 * items)
@@ -321,13 +324,16 @@ hipError_t launch_seg_hash_build(const uint32_t *dir_ptr, const uint32_t *dir, u
 // Device scratch of the allocation-free match: a file-scope array of
 // kNoAllocScratchBytes in kernels.hip, one per GPU, held until the process
 // ends.  Layout: control block (256 B), totals (256 B), the scan words of
-// kNoAllocTiles tiles (two arrays), the tile index (2 words per tile), then
-// from kNoAllocWorkBytes on the level arena of kNoAllocLevelBytes.
+// kNoAllocTiles tiles (two arrays), the tile index (2 words per tile), the sums
+// of kNoAllocTailTiles tail tiles, then from kNoAllocWorkBytes on the level arena of kNoAllocLevelBytes.
 constexpr uint64_t kNoAllocScratchBytes = 64ull << 20;
 constexpr uint64_t kNoAllocTiles = 1ull << 16;
 constexpr uint64_t kNoAllocWorkBytes = 4ull << 20;
 constexpr uint64_t kNoAllocLevelBytes = kNoAllocScratchBytes - kNoAllocWorkBytes;
-static_assert(512 + 32 * kNoAllocTiles <= kNoAllocWorkBytes, "scratch workspace layout");
+constexpr uint64_t kNoAllocTailTiles = (kNoAllocWorkBytes - 512 - 32 * kNoAllocTiles) / (8 * kTailWords);
+static_assert(512 + 32 * kNoAllocTiles + 8 * kTailWords * kNoAllocTailTiles <= kNoAllocWorkBytes &&
+                  kNoAllocTailTiles >= 1024,
+              "scratch workspace layout");
 // Device address of `device`'s scratch array: looked up with
 // hipGetSymbolAddress on the first call for a device (that device made
 // current; its workspace part cleared on `s`), then cached.

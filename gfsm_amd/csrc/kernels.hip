@@ -27,6 +27,7 @@
 #include <hip/hip_runtime.h>
 
 #include <mutex>
+#include <type_traits>
 
 #include "kernels.h"
 
@@ -432,33 +433,6 @@ DEV void flush_sums(uint64_t cnt, uint64_t h0, uint64_t h1, Totals *tot_ptr, uin
     }
 }
 
-// The same for a tail step: embeddings, nodes kept and candidates of the last depth.
-DEV void flush_tail(uint64_t cnt, uint64_t kept, uint64_t cand, Totals *tot_ptr, uint64_t (*s_red)[kWaves])
-{
-    const uint32_t lane = lane_id(), wave = threadIdx.x >> 6;
-    cnt = wave_sum64(cnt);
-    kept = wave_sum64(kept);
-    cand = wave_sum64(cand);
-    if (lane == 0) {
-        s_red[0][wave] = cnt;
-        s_red[1][wave] = kept;
-        s_red[2][wave] = cand;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        uint64_t c = 0, a = 0, b = 0;
-        for (uint32_t w = 0; w < kWaves; w++) {
-            c += s_red[0][w];
-            a += s_red[1][w];
-            b += s_red[2][w];
-        }
-        const auto tot = gp(tot_ptr);
-        if (c) __hip_atomic_fetch_add(&tot->count, c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (a) __hip_atomic_fetch_add(&tot->tail_keep, a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (b) __hip_atomic_fetch_add(&tot->tail_cand, b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-}
-
 // One per-node lookup of a tile's staging (a checked ancestor's segment or
 // the next generator's): the row column whose vertex is looked up (~0u: none,
 // the check is the candidate's own), its relation and its dense table.
@@ -476,8 +450,17 @@ struct TileShared {
     uint64_t red[3][kWaves];
     uint32_t slot;
     uint32_t next;  // prefetched tile ticket
-    NodeLookup lk[GFSM_MAXCHK + 1];  // the depth's lookups, read per lane from LDS
+    // the depth's lookups, read per lane from LDS (with a tail's leaves')
+    NodeLookup lk[GFSM_MAXCHK + 1 + GFSM_MAXTAIL * (1 + GFSM_TAILCHK)];
+    uint64_t tsum[kTailWords];  // tail sums (Totals::tail) of the tile, or of all tiles so far
 };
+
+// tsum[i] += the sum of v over the workgroup's threads, wave by wave.
+DEV void tail_add(uint64_t *tsum, uint32_t i, uint64_t v)
+{
+    v = wave_sum64(v);
+    if (lane_id() == 0) atomicAdd((unsigned long long *)tsum + i, (unsigned long long)v);
+}
 
 // ---------------------------------------------------------------------------
 // root level (hnInit, HnGPU.cu:76-109)
@@ -489,27 +472,6 @@ DEV void publish_kc(uint64_t *kc, uint64_t keep, uint64_t cnt)
 {
     __hip_atomic_store(kc + 1, cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     __hip_atomic_store(kc, keep, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-}
-
-// One tile's sums of a capped tail step: a tile keeps at most 2,048 nodes, of
-// fewer than 2^26 candidates each.
-constexpr uint32_t kTailKeptShift = 48;
-DEV void tail_tile_sums(uint64_t *sums, uint64_t t, uint64_t cnt, uint64_t kept, uint64_t cand,
-                        uint64_t (*s_red)[kWaves])
-{
-    const uint32_t lane = lane_id(), wave = threadIdx.x >> 6;
-    cnt = wave_sum64(cnt);
-    cand = wave_sum64(kept << kTailKeptShift | cand);
-    if (lane == 0) {
-        s_red[0][wave] = cnt;
-        s_red[1][wave] = cand;
-    }
-    __syncthreads();
-    if (threadIdx.x < 2) {
-        uint64_t v = 0;
-        for (uint32_t w = 0; w < kWaves; w++) v += s_red[threadIdx.x][w];
-        gp(sums)[2 * t + threadIdx.x] = v;
-    }
 }
 
 // Root tile `lt` of a root step (global tile gt, the step's scan starting at
@@ -684,6 +646,7 @@ DEV uint32_t pick_row_or(const RA &rows, uint32_t j, uint32_t c, uint32_t d, uin
 // each column is searched, the I searches in lockstep, and every copy of a
 // repeated entry counts.
 constexpr uint32_t kTailShort = 8;
+constexpr uint32_t kNoEntry = 0xFFFFFFFEu;  // no vertex either (wide tails: V < kNoEntry), nor kSegEmpty
 template <uint32_t I, class RA>
 DEV void tail_overlap(const uint32_t *__restrict__ nbr, const RA &rows, uint32_t d, uint32_t cols,
                       const uint32_t (&jj)[I], const uint32_t (&w)[I], const uint32_t (&gb)[I],
@@ -767,21 +730,72 @@ DEV void tail_overlap(const uint32_t *__restrict__ nbr, const RA &rows, uint32_t
     }
 }
 
+// Up to eight entries from nbr[at] on, `none` past the first n.
+DEV void load8(const uint32_t *__restrict__ nbr, uint32_t at, uint32_t n, uint32_t none, uint32_t (&e)[8])
+{
+    const auto p = (gptr_t<const u32x4_w>)gp(nbr + at);
+    const u32x4 lo = n ? (u32x4)p[0] : u32x4{0u, 0u, 0u, 0u};
+    const u32x4 hi = n > 4 ? (u32x4)p[1] : u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+    for (uint32_t b = 0; b < 4; b++) {
+        e[b] = b < n ? lo[b] : none;
+        e[b + 4] = b + 4 < n ? hi[b] : none;
+    }
+}
+
+// Entries of `e` that are not in the segment become kSegEmpty.
+DEV void keep_in(const uint32_t *__restrict__ nbr, uint2 seg, uint32_t (&e)[8])
+{
+    const uint32_t len = seg.y - seg.x;
+    bool hit[8];
+#pragma unroll
+    for (uint32_t b = 0; b < 8; b++) hit[b] = false;
+    for (uint32_t f0 = 0; __any(f0 < len); f0 += 8) {
+        uint32_t f[8];
+        load8(nbr, seg.x + f0, f0 < len ? len - f0 : 0u, kNoEntry, f);
+#pragma unroll
+        for (uint32_t a = 0; a < 8; a++)
+#pragma unroll
+            for (uint32_t b = 0; b < 8; b++) hit[b] |= e[b] == f[a];
+    }
+#pragma unroll
+    for (uint32_t b = 0; b < 8; b++) e[b] = hit[b] ? e[b] : kSegEmpty;
+}
+
+// Pairs of equal entries of `e` and of the segment.
+DEV uint32_t equal_in(const uint32_t *__restrict__ nbr, uint2 seg, const uint32_t (&e)[8])
+{
+    const uint32_t len = seg.y - seg.x;
+    uint32_t n = 0;
+    for (uint32_t f0 = 0; __any(f0 < len); f0 += 8) {
+        uint32_t f[8];
+        load8(nbr, seg.x + f0, f0 < len ? len - f0 : 0u, kNoEntry, f);
+#pragma unroll
+        for (uint32_t a = 0; a < 8; a++)
+#pragma unroll
+            for (uint32_t b = 0; b < 8; b++) n += e[b] == f[a] ? 1u : 0u;
+    }
+    return n;
+}
+
 // Expand tile `lt` of a step (global tile gt; the step's scan starts at gt0).
 // `dyn` is the dynamic LDS: the node-start bitmap, the per-position generator
 // base and a pool of pool_words words that stages, per frontier node of the
 // tile, the checked ancestor segments, the next generator segment and the
 // placed vertices, as far as they fit.  `inj` is the depth's injectivity mask
-// and `linj` the next depth's (scalars; linj for EXPAND_TAIL).  LAST_COUNT adds its embeddings and digest to the thread's accumulators; the other kinds write their output.
-template <uint32_t KIND, uint32_t I, class DP, class CP>
-DEV void expand_tile(const DevGraphView &g, const DP &dp, CP col, CP dcol,
+// (a scalar), `tl` the leaves of a tail step.  LAST_COUNT adds its embeddings
+// and digest to the thread's accumulators, a tail step its sums to sh.tsum; the
+// other kinds write their output.
+template <uint32_t KIND, uint32_t I, class DP, class TP, class CP>
+DEV void expand_tile(const DevGraphView &g, const DP &dp, const TP &tl, CP col, CP dcol,
                      const StepIO &io, uint64_t lt, uint64_t gt, uint64_t gt0, const ScanWS &ws, uint32_t ep,
-                     uint32_t inj, uint32_t linj, uint32_t pool_words, TileShared<I> &sh, unsigned char *dyn, uint64_t &acc_cnt,
+                     uint32_t inj, uint32_t pool_words, TileShared<I> &sh, unsigned char *dyn, uint64_t &acc_cnt,
                      uint64_t &acc_h0, uint64_t &acc_h1, bool tickets = true)
 {
     constexpr uint32_t T = kTile, TC = kTile * I, NW = TC / 64;
     constexpr bool BARE = KIND == EXPAND_LAST_BARE;  // counting, no checks, no digest
-    constexpr bool TAIL = KIND == EXPAND_TAIL;       // counts the last depth's embeddings from the one before
+    constexpr bool WIDE = KIND == EXPAND_TAIL_WIDE;
+    constexpr bool TAIL = KIND == EXPAND_TAIL || WIDE;  // counts the completions of its survivors
     constexpr bool INNER = KIND == EXPAND_MID || TAIL;
     constexpr bool COUNTING = KIND == EXPAND_LAST_COUNT || BARE || TAIL;
     constexpr bool PACKED = BARE || TAIL;  // stages only the row columns it reads
@@ -811,7 +825,32 @@ DEV void expand_tile(const DevGraphView &g, const DP &dp, CP col, CP dcol,
     const auto tot = gp(io.tot);
 
     const uint32_t nchk = BARE ? 0u : dp.nchk;
-    const uint32_t need_nxt = INNER ? io.need_nxt : 0u;
+    const uint32_t need_nxt = KIND == EXPAND_MID ? io.need_nxt : 0u;
+    // A tail's leaves: the segments staged per node follow the checks', in leaf
+    // order (generator, then its checks); then, for every leaf whose overlap
+    // with the placed row is formed per node, a word per node.
+    const uint32_t row_mask = (1u << d) - 1u;
+    uint32_t nstage = nchk + need_nxt, novl = 0, tinj = 0, tcols = 0;
+    if constexpr (TAIL) {
+        for (uint32_t i = 0; i < tl.m; i++) {
+            const uint32_t r0 = nstage;
+            const uint32_t lc = tl.leaf[i].col, ln = WIDE ? tl.leaf[i].nchk : 0u;
+            tinj |= tl.leaf[i].inj;
+            tcols |= 1u << lc;
+            if (lc < d) {
+                if (tid == 0) sh.lk[nstage] = NodeLookup{lc, tl.leaf[i].rel, tl.leaf[i].tab};
+                nstage++;
+            }
+            for (uint32_t r = 0; r < ln; r++) {
+                const uint32_t cc = tl.leaf[i].chk_col[r];
+                tcols |= 1u << cc;
+                if (cc >= d) continue;
+                if (tid == 0) sh.lk[nstage] = NodeLookup{cc, tl.leaf[i].chk_rel[r], tl.leaf[i].chk_tab[r]};
+                nstage++;
+            }
+            if (nstage > r0 && lc < d && !ln && !(WIDE && tl.leaf[i].pair) && (tl.leaf[i].inj & row_mask)) novl++;
+        }
+    }
     // The depth's lookups, one LDS entry each, so the staging loop below
     // selects its lookup per lane from LDS rather than indexing the plan
     // (kernel arguments or global memory) with a per-lane index.
@@ -846,17 +885,17 @@ DEV void expand_tile(const DevGraphView &g, const DP &dp, CP col, CP dcol,
     // The rows come first: every candidate reads its node's row (d words,
     // twice on inner depths), but a node's segments save lookups only for
     // its candidates after the first.
-    const uint32_t meta_words = 2 * nf * nchk + (need_nxt ? (TAIL ? 3 : 2) * nf : 0);
+    const uint32_t meta_words = 2 * nf * nstage + novl * nf;
     // Row columns staged: all, or the compared ones, with those that lookups
     // read where the lookups are not staged.
-    uint32_t need = (1u << d) - 1u, rw = d;
+    uint32_t need = row_mask, rw = d;
     if (PACKED) {
-        need = (inj | (TAIL ? linj : 0u)) & ((1u << d) - 1u);
+        need = (inj | tinj) & row_mask;
         rw = (uint32_t)__builtin_popcount(need);
         if (((nf * rw + 1) & ~1u) + meta_words > pool_words) {
             for (uint32_t r = 0; r < nchk; r++)
                 if (dp.chk_dist[r]) need |= 1u << (d - dp.chk_dist[r]);
-            if (need_nxt) need |= 1u << (d + 1 - dp.nxt_dist);
+            need |= tcols & row_mask;
             rw = (uint32_t)__builtin_popcount(need);
         }
     }
@@ -866,7 +905,7 @@ DEV void expand_tile(const DevGraphView &g, const DP &dp, CP col, CP dcol,
     uint32_t *s_rows = s_pool;                                                   // [nf][d]
     uint2 *s_chk = reinterpret_cast<uint2 *>(s_pool + (staged ? row_words : 0));  // [nchk][nf]
     uint2 *s_nxt = s_chk + nchk * nf;                                            // [nf]
-    uint32_t *s_ovl = reinterpret_cast<uint32_t *>(s_nxt + nf);                  // [nf] TAIL: row columns in s_nxt
+    uint32_t *s_ovl = reinterpret_cast<uint32_t *>(s_chk + nstage * nf);         // [novl][nf]
     // Digest of a counting last depth: each node's placed columns contribute
     // the same terms to all its candidates' row hashes, so their sums are
     // formed once per node (two u64 per node, after the staged data).
@@ -929,7 +968,7 @@ DEV void expand_tile(const DevGraphView &g, const DP &dp, CP col, CP dcol,
     // run one after another.
     if (!BARE && stage_meta) {  // the lean kind has no lookups to stage
         constexpr uint32_t L = kNodeLk;
-        const uint32_t nl = nchk + need_nxt;
+        const uint32_t nl = nstage;
         const uint32_t total = nf * nl;
         for (uint32_t u0 = tid; u0 < total; u0 += T * L) {
             uint32_t x[L], rel[L], dst[L];
@@ -967,25 +1006,6 @@ DEV void expand_tile(const DevGraphView &g, const DP &dp, CP col, CP dcol,
 #pragma unroll
             for (uint32_t k = 0; k < L; k++)
                 if (act[k]) s_chk[dst[k]] = tab[k] ? make_uint2((uint32_t)dv[k], (uint32_t)(dv[k] >> 32)) : sg[k];
-            if constexpr (TAIL) {
-                // The node's placed vertices among its children's candidates.
-                if (need_nxt) {
-                    uint32_t nj[L], gbeg[L], n[L], ov[L];
-#pragma unroll
-                    for (uint32_t k = 0; k < L; k++) {
-                        const uint2 e = tab[k] ? make_uint2((uint32_t)dv[k], (uint32_t)(dv[k] >> 32)) : sg[k];
-                        const bool nx = act[k] && dst[k] >= nchk * nf;
-                        nj[k] = nx ? dst[k] - nchk * nf : 0u;
-                        gbeg[k] = e.x;
-                        n[k] = nx ? e.y - e.x : 0u;
-                        ov[k] = 0;
-                    }
-                    tail_overlap<L>(g.nbr, LevelRows{in_rows, d}, d, linj & ((1u << d) - 1u), nj, x, gbeg, n, ov);
-#pragma unroll
-                    for (uint32_t k = 0; k < L; k++)
-                        if (act[k] && dst[k] >= nchk * nf) s_ovl[nj[k]] = ov[k];
-                }
-            }
         }
     }
     __syncthreads();
@@ -1050,6 +1070,38 @@ DEV void expand_tile(const DevGraphView &g, const DP &dp, CP col, CP dcol,
     // pointer that could be either would turn the LDS reads into flat loads,
     // which take the vector-memory path.
     auto tail = [&](auto rows) {
+        if constexpr (TAIL) {
+            // Per node: how many of its placed vertices are among a leaf's candidates.
+            if (novl && stage_meta) {
+                uint32_t r = nchk, o = 0;
+                for (uint32_t i = 0; i < tl.m; i++) {
+                    const uint32_t lc = tl.leaf[i].col, ln = WIDE ? tl.leaf[i].nchk : 0u;
+                    const uint32_t r0 = r;
+                    r += lc < d ? 1u : 0u;
+                    for (uint32_t q = 0; q < ln; q++) r += tl.leaf[i].chk_col[q] < d ? 1u : 0u;
+                    const uint32_t cols = tl.leaf[i].inj & row_mask;
+                    if (!(r > r0 && lc < d && !ln && !(WIDE && tl.leaf[i].pair) && cols)) continue;
+                    for (uint32_t j0 = tid; j0 < nf; j0 += 2 * T) {
+                        uint32_t nj[2], nb[2], nn[2], nw[2], ov[2];
+#pragma unroll
+                        for (uint32_t b = 0; b < 2; b++) {
+                            const bool in = j0 + b * T < nf;
+                            nj[b] = in ? j0 + b * T : 0u;
+                            const uint2 e = s_chk[r0 * nf + nj[b]];
+                            nb[b] = e.x;
+                            nn[b] = in ? e.y - e.x : 0u;
+                            nw[b] = ov[b] = 0;
+                        }
+                        tail_overlap<2>(g.nbr, rows, d, cols, nj, nw, nb, nn, ov);
+#pragma unroll
+                        for (uint32_t b = 0; b < 2; b++)
+                            if (j0 + b * T < nf) s_ovl[o * nf + nj[b]] = ov[b];
+                    }
+                    o++;
+                }
+                __syncthreads();
+            }
+        }
         // Phase 2: injectivity against the placed vertices a candidate of this
         // depth can coincide with, one placed column at a time for all items,
         // so I reads are in flight together.
@@ -1087,7 +1139,7 @@ DEV void expand_tile(const DevGraphView &g, const DP &dp, CP col, CP dcol,
             seg_contains_n<I>(g.nbr, sg, w, keep);
         }
 
-        if (INNER) {
+        if (KIND == EXPAND_MID) {
             // Phase 4: the survivor's next generator segment; no children, no node.
             uint2 ns[I];
             if (need_nxt && stage_meta) {
@@ -1228,20 +1280,140 @@ DEV void expand_tile(const DevGraphView &g, const DP &dp, CP col, CP dcol,
                 if (KIND == EXPAND_MID && sm.tot[0] <= io.cap) out_off[sm.tot[0]] = sm.tot[1];
             }
         } else if constexpr (TAIL) {
-            // Every entry of the survivor's next segment is an embedding, but
-            // for the placed vertices among them.
-            uint32_t ov[I];
-            const bool by_node = need_nxt && stage_meta;
+            // The survivor's completions: c injective choices of the leaves so
+            // far, each with (candidates - placed vertices and twins among them)
+            // choices of the next; two leaves that meet multiply and take the
+            // common choices off.
+            // Four candidates per thread at a time (two with sets compared entry
+            // by entry): more would spill.
+            constexpr uint32_t P = I < (WIDE ? 2 : 4) ? I : (WIDE ? 2 : 4);
+            static_assert(I <= 2 * P, "two parts");
+            const auto leaves = [&](auto part) {
+            constexpr uint32_t K0 = decltype(part)::value * P;
+            uint64_t c[P], pc[WIDE ? P : 1];
+            uint32_t pn[WIDE ? P : 1], pj[P], pw[P];
 #pragma unroll
-            for (uint32_t k = 0; k < I; k++) ov[k] = by_node ? s_ovl[jj[k]] : 0u;
-            const uint32_t cols = by_node ? linj & (1u << d) : linj;
-            if (cols) tail_overlap<I>(g.nbr, rows, d, cols, jj, w, gb, cnt, ov);
-#pragma unroll
-            for (uint32_t k = 0; k < I; k++) {
-                acc_h0 += keep[k] ? 1u : 0u;
-                acc_h1 += cnt[k];
-                acc_cnt += keep[k] ? cnt[k] - ov[k] : 0u;
+            for (uint32_t k = 0; k < P; k++) {
+                c[k] = keep[K0 + k] ? 1u : 0u;
+                pj[k] = jj[K0 + k];
+                pw[k] = w[K0 + k];
             }
+            // Segment of (column cc, relation): staged (the next one of the list), or looked up.
+            const auto leaf_seg = [&](uint32_t cc, uint32_t rel, const void *tab, uint32_t &r, uint2 (&o)[P]) {
+                if (cc < d) {
+                    r++;
+                    if (stage_meta) {
+#pragma unroll
+                        for (uint32_t k = 0; k < P; k++) o[k] = c[k] ? s_chk[(r - 1) * nf + pj[k]] : make_uint2(0u, 0u);
+                        return;
+                    }
+                }
+                uint32_t x[P];
+                bool act[P];
+#pragma unroll
+                for (uint32_t k = 0; k < P; k++) {
+                    x[k] = pick_row_or(rows, pj[k], cc, d, pw[k]);
+                    act[k] = c[k] != 0;
+                }
+                if (tab) {
+                    const auto t = gp(reinterpret_cast<const uint64_t *>(tab));
+#pragma unroll
+                    for (uint32_t k = 0; k < P; k++) {
+                        const uint64_t v = act[k] ? t[x[k]] : 0ull;
+                        o[k] = make_uint2((uint32_t)v, (uint32_t)(v >> 32));
+                    }
+                } else {
+                    seg_lookup_n<P>(g, x, rel, act, o);
+                }
+            };
+            uint32_t r = nchk, o = 0, pr = 0;
+            for (uint32_t i = 0; i < tl.m; i++) {
+                const uint32_t lc = tl.leaf[i].col, linj = tl.leaf[i].inj, twins = tl.leaf[i].twins;
+                const uint32_t ln = WIDE ? tl.leaf[i].nchk : 0u;
+                const bool pair = WIDE && tl.leaf[i].pair;
+                const uint32_t r0 = r;
+                uint2 sg[P];
+                leaf_seg(lc, tl.leaf[i].rel, tl.leaf[i].tab, r, sg);
+                uint32_t len[P], beg[P], ov[P];
+                uint64_t kept = 0, cand = 0;
+#pragma unroll
+                for (uint32_t k = 0; k < P; k++) {
+                    beg[k] = sg[k].x;
+                    len[k] = sg[k].y - sg[k].x;
+                    kept += len[k] ? c[k] : 0ull;
+                    cand += c[k] * len[k];
+                    ov[k] = 0;
+                }
+                tail_add(sh.tsum, 2 * i, kept);
+                tail_add(sh.tsum, 2 * i + 1, cand);
+                if (!(WIDE && (ln || pair))) {
+                    uint32_t cols = linj;
+                    if (lc < d && (linj & row_mask) && stage_meta) {
+#pragma unroll
+                        for (uint32_t k = 0; k < P; k++) ov[k] = s_ovl[o * nf + pj[k]];
+                        cols = linj & ~row_mask;
+                    }
+                    o += lc < d && (linj & row_mask) ? 1u : 0u;
+                    if (cols) tail_overlap<P>(g.nbr, rows, d, cols, pj, pw, beg, len, ov);
+#pragma unroll
+                    for (uint32_t k = 0; k < P; k++) {
+                        if constexpr (WIDE) {
+                            pc[k] = c[k];
+                            pn[k] = len[k] - ov[k];
+                        }
+                        c[k] = len[k] ? c[k] * (uint64_t)(int64_t)(int32_t)(len[k] - ov[k] - twins) : 0ull;
+                    }
+                } else if constexpr (WIDE) {
+                    uint2 cs[GFSM_TAILCHK][P], ps[1 + GFSM_TAILCHK][P];
+                    for (uint32_t q = 0; q < GFSM_TAILCHK; q++)
+                        if (q < ln) leaf_seg(tl.leaf[i].chk_col[q], tl.leaf[i].chk_rel[q], tl.leaf[i].chk_tab[q], r, cs[q]);
+                    const uint32_t pq = pair ? tl.leaf[i - 1].nchk : 0u;
+                    if (pair) {
+                        uint32_t rr = pr;
+                        leaf_seg(tl.leaf[i - 1].col, tl.leaf[i - 1].rel, tl.leaf[i - 1].tab, rr, ps[0]);
+                        for (uint32_t q = 0; q < GFSM_TAILCHK; q++)
+                            if (q < pq)
+                                leaf_seg(tl.leaf[i - 1].chk_col[q], tl.leaf[i - 1].chk_rel[q], tl.leaf[i - 1].chk_tab[q],
+                                         rr, ps[1 + q]);
+                    }
+#pragma unroll
+                    for (uint32_t k = 0; k < P; k++) {
+                        uint32_t n = 0, both = 0;
+                        for (uint32_t e0 = 0; __any(e0 < len[k]); e0 += 8) {
+                            uint32_t e[8];
+                            load8(g.nbr, beg[k] + e0, e0 < len[k] ? len[k] - e0 : 0u, kSegEmpty, e);
+                            for (uint32_t im = linj; im; im &= im - 1) {
+                                const uint32_t kk = (uint32_t)__builtin_ctz(im);
+                                const uint32_t x = kk == d ? pw[k] : rows.at(pj[k], kk == d ? 0u : kk);
+#pragma unroll
+                                for (uint32_t b = 0; b < 8; b++) e[b] = e[b] == x ? kSegEmpty : e[b];
+                            }
+                            for (uint32_t q = 0; q < GFSM_TAILCHK; q++)
+                                if (q < ln) keep_in(g.nbr, cs[q][k], e);
+#pragma unroll
+                            for (uint32_t b = 0; b < 8; b++) n += e[b] != kSegEmpty ? 1u : 0u;
+                            if (pair) {
+                                for (uint32_t q = 0; q < GFSM_TAILCHK; q++)
+                                    if (q < pq) keep_in(g.nbr, ps[1 + q][k], e);
+                                both += equal_in(g.nbr, ps[0][k], e);
+                            }
+                        }
+                        const uint64_t pc0 = pc[k], c0_ = c[k];
+                        const uint32_t pn0 = pn[k];
+                        pc[k] = c0_;
+                        pn[k] = n;
+                        c[k] = pair ? (c0_ ? pc0 * ((uint64_t)pn0 * n - both) : 0ull) : c0_ * n;
+                    }
+                }
+                pr = r0;
+            }
+            uint64_t sum = 0;
+#pragma unroll
+            for (uint32_t k = 0; k < P; k++) sum += c[k];
+            tail_add(sh.tsum, 2 * tl.m, sum);
+            };
+            leaves(std::integral_constant<uint32_t, 0>{});
+            if constexpr (I > P) leaves(std::integral_constant<uint32_t, 1>{});
         } else {
 #pragma unroll
             for (uint32_t k = 0; k < I; k++) acc_cnt += keep[k] ? 1u : 0u;
@@ -1278,6 +1450,16 @@ DEV void expand_tile(const DevGraphView &g, const DP &dp, CP col, CP dcol,
         tail(LevelRows{in_rows, d});
 }
 
+
+// A tail tile's sums go to sums[kTailWords * t], and start again from zero.
+DEV void tail_tile_end(uint64_t *sums, uint64_t t, uint64_t *tsum)
+{
+    __syncthreads();
+    if (threadIdx.x < 2 * GFSM_MAXTAIL + 1) {
+        gp(sums)[kTailWords * t + threadIdx.x] = tsum[threadIdx.x];
+        tsum[threadIdx.x] = 0;
+    }
+}
 
 // Tiles of the kinds without a look-back, dealt so that runs of kXcdRun
 // consecutive tiles go to workgroups of one XCD: consecutive tiles expand
@@ -1322,7 +1504,7 @@ __global__ __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(4))) void
         for (TileDeal dl; dl.tile() < a.io.ntiles; dl.next()) {
             const uint64_t t = dl.tile();
             __syncthreads();  // the previous tile's readers of the tile LDS are done
-            expand_tile<KIND, I>(a.g, a.dp, a.col, a.dcol, a.io, t, t, 0, a.ws, ep, a.dp.inj, a.linj, a.pool_words, sh, smem, acc_cnt,
+            expand_tile<KIND, I>(a.g, a.dp, a.tail, a.col, a.dcol, a.io, t, t, 0, a.ws, ep, a.dp.inj, a.pool_words, sh, smem, acc_cnt,
                                  acc_h0, acc_h1, false);
         }
     } else {
@@ -1330,7 +1512,7 @@ __global__ __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(4))) void
         for (;;) {
             const uint64_t t = tickets_take(&sh.next);
             if (t >= a.io.ntiles) break;
-            expand_tile<KIND, I>(a.g, a.dp, a.col, a.dcol, a.io, t, t, 0, a.ws, ep, a.dp.inj, a.linj, a.pool_words, sh, smem, acc_cnt,
+            expand_tile<KIND, I>(a.g, a.dp, a.tail, a.col, a.dcol, a.io, t, t, 0, a.ws, ep, a.dp.inj, a.pool_words, sh, smem, acc_cnt,
                                  acc_h0, acc_h1);
         }
     }
@@ -1338,120 +1520,113 @@ __global__ __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(4))) void
     finish_launch(a.ws);
 }
 
-// The tail kernel: depth q-2, whose survivors' children are counted without a
-// level in between, from each survivor's segment of the last generator.  Under
-// a cap (host_kc set) the tiles' sums stay apart for k_tail_cut; otherwise they
-// are added to the totals.
-// The last two depths held most of a count's candidates and nearly all of its
-// level traffic (7-vertex path on the 1400 x 1400 grid: 420 M nodes of 36 bytes
-// written and read back).  The step is bound by the loads of a candidate, of its
-// next segment's bounds and of that segment's entries, so it keeps 8 candidates
-// per thread and four waves per SIMD as k_expand, and deals its tiles without
-// tickets.  Measured, two steps against this one: that path 23.9 -> 12.2 ms; a
-// 7-vertex count on a 200,000-vertex labelled graph 8.0 -> 2.9 ms, a 6-vertex one
-// inside 60 MiB of levels 1.26 -> 0.45 ms; nine capped queries on R-MAT 18, where
-// the tile with the cap's candidate still takes the two steps, 6.7 -> 5.5 ms.
-template <uint32_t I>
+// The tail kernel: the last depth before the leaves, whose survivors'
+// completions are counted from the leaves' segments, with no level in between.
+// Under a cap (host_kc set) every tile's sums stay apart for k_tail_cut;
+// otherwise they are added to the totals.
+// The last depths hold most of a count's candidates and nearly all of its level
+// traffic, and in the matching order (by degree) they are mostly leaves.  The
+// step is bound by the loads of a candidate, of its leaves' segment bounds and
+// of their entries; it keeps 8 candidates per thread (4 with sets compared entry
+// by entry) and four waves per SIMD, and deals its tiles without tickets.
+// Measured, every depth expanded / one leaf / up to three leaves: 7-vertex path
+// on the 1400 x 1400 grid 23.9 / 12.2 / 8.0 ms; its 6-cycle, a checked leaf, 10.9
+// / 10.6 / 6.8 ms; a 7-vertex count on a 200,000-vertex labelled graph 8.0 / 2.5 /
+// 1.0 ms, a 6-vertex one inside 60 MiB of levels 1.26 / 0.43 / 0.20 ms; nine
+// capped queries on R-MAT 18, where the tile with the cap's candidate is still
+// expanded level by level, 6.7 / 4.7 / 4.5 ms.
+template <uint32_t KIND, uint32_t I>
 __global__ __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(4))) void k_expand_tail(ExpandArgs a)
 {
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ TileShared<I> sh;
     const uint32_t ep = read_epoch(a.ws);
     const bool capped = a.io.host_kc != nullptr;
-    uint64_t cnt = 0, kept = 0, cand = 0;
+    if (threadIdx.x < kTailWords) sh.tsum[threadIdx.x] = 0;
+    uint64_t c = 0, h0 = 0, h1 = 0;
     for (TileDeal dl; dl.tile() < a.io.ntiles; dl.next()) {
         const uint64_t t = dl.tile();
         __syncthreads();
-        expand_tile<EXPAND_TAIL, I>(a.g, a.dp, a.col, a.dcol, a.io, t, t, 0, a.ws, ep, a.dp.inj, a.linj, a.pool_words,
-                                    sh, smem, cnt, kept, cand, false);
-        if (capped) {
-            tail_tile_sums(a.tail_sums, t, cnt, kept, cand, sh.red);
-            cnt = kept = cand = 0;
-        }
+        expand_tile<KIND, I>(a.g, a.dp, a.tail, a.col, a.dcol, a.io, t, t, 0, a.ws, ep, a.dp.inj, a.pool_words, sh, smem,
+                             c, h0, h1, false);
+        if (capped) tail_tile_end(a.tail_sums, t, sh.tsum);
     }
-    if (!capped) flush_tail(cnt, kept, cand, a.io.tot, sh.red);
+    __syncthreads();
+    if (!capped && threadIdx.x < 2 * a.tail.m + 1)
+        __hip_atomic_fetch_add(&gp(a.io.tot)->tail[threadIdx.x], sh.tsum[threadIdx.x], __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
     finish_launch(a.ws);
 }
 
+DEV uint64_t add_sat(uint64_t a, uint64_t b) { return a + b < a ? ~0ull : a + b; }
+
 // After a capped tail step (one workgroup): sums the tiles in order up to the
-// first one whose last-depth candidates no longer fit `room`, and tells the
-// host how far it came and the sums so far: {nodes kept, candidates,
-// embeddings, tiles}, the polled first word last.  A kernel of its own: inside
-// the tail kernel its registers would be spilled by every tile.
-__global__ __launch_bounds__(kTile) void k_tail_cut(const uint64_t *tile_sums, uint64_t ntiles, uint64_t room,
-                                                    uint64_t *kc)
+// first one whose candidates no longer fit the rooms of the leaves' depths, and
+// tells the host {tiles, their sums}, the polled first word last.  A kernel of
+// its own: inside the tail kernel its registers would be spilled by every tile.
+constexpr uint32_t kCutThreads = 1024;
+__global__ __launch_bounds__(kCutThreads) void k_tail_cut(const uint64_t *tile_sums, uint64_t ntiles, uint32_t m,
+                                                          uint64_t room0, uint64_t room1, uint64_t room2,
+                                                          uint64_t room_all, uint64_t *kc)
 {
-    constexpr uint32_t B = 8;
-    __shared__ uint64_t s_red[3][kWaves];
+    static_assert(GFSM_MAXTAIL == 3, "rooms");
+    constexpr uint32_t W = kCutThreads / 64;
+    __shared__ uint64_t s_w[W][kTailWords];
+    __shared__ uint64_t s_base[kTailWords];  // sums of the tiles taken so far
+    __shared__ uint32_t s_fit[W];
     const uint32_t lane = lane_id(), wave = threadIdx.x >> 6;
-    uint64_t kept = 0, cand = 0, cnt = 0, tiles = ntiles;
-    for (uint64_t t0 = 0; t0 < ntiles; t0 += kTile * B) {
-        // this thread's B consecutive tiles: their sums, then the prefix before them
-        uint64_t c[B], k[B], e[B], mine = 0;
+    const uint64_t room[3] = {room0, room1, room2};
+    if (threadIdx.x < kTailWords) s_base[threadIdx.x] = 0;
+    uint64_t tiles = 0;
+    for (uint64_t t0 = 0; t0 < ntiles; t0 += kCutThreads) {
+        const uint64_t t = t0 + threadIdx.x;
+        uint64_t v[3], inc[3];
 #pragma unroll
-        for (uint32_t b = 0; b < B; b++) {
-            const uint64_t t = t0 + threadIdx.x * B + b;
-            e[b] = t < ntiles ? tile_sums[2 * t] : 0ull;
-            c[b] = t < ntiles ? tile_sums[2 * t + 1] : 0ull;
-        }
-#pragma unroll
-        for (uint32_t b = 0; b < B; b++) {
-            k[b] = c[b] >> kTailKeptShift;
-            c[b] &= (1ull << kTailKeptShift) - 1;
-            mine += c[b];
-        }
-        uint64_t inc = mine;
-        for (uint32_t o = 1; o < 64; o <<= 1) {
-            const uint64_t v = __shfl_up(inc, o, 64);
-            if (lane >= o) inc += v;
-        }
-        if (lane == 63) s_red[0][wave] = inc;
-        __syncthreads();
-        uint64_t run = cand + inc - mine, all = cand;
-        for (uint32_t w = 0; w < kWaves; w++) {
-            if (w < wave) run += s_red[0][w];
-            all += s_red[0][w];
-        }
-        // this thread's tiles that fit
-        uint64_t my_k = 0, my_e = 0, my_c = 0, fit = 0;
-#pragma unroll
-        for (uint32_t b = 0; b < B; b++) {
-            run += c[b];
-            if (run <= room) {
-                my_k += k[b];
-                my_e += e[b];
-                my_c += c[b];
-                fit += t0 + threadIdx.x * B + b < ntiles ? 1 : 0;
+        for (uint32_t i = 0; i < 3; i++) {
+            v[i] = i < m && t < ntiles ? tile_sums[kTailWords * t + 1 + 2 * i] : 0ull;
+            inc[i] = v[i];
+            for (uint32_t o = 1; o < 64; o <<= 1) {
+                const uint64_t u = __shfl_up(inc[i], o, 64);
+                if (lane >= o) inc[i] = add_sat(inc[i], u);
             }
-        }
-        my_k = wave_sum64(my_k << 32 | fit);
-        my_e = wave_sum64(my_e);
-        my_c = wave_sum64(my_c);
-        __syncthreads();
-        if (lane == 0) {
-            s_red[0][wave] = my_k;
-            s_red[1][wave] = my_e;
-            s_red[2][wave] = my_c;
+            if (lane == 63) s_w[wave][i] = inc[i];
         }
         __syncthreads();
-        uint64_t fits = 0;
-        for (uint32_t w = 0; w < kWaves; w++) {
-            kept += s_red[0][w] >> 32;
-            fits += s_red[0][w] & 0xFFFFFFFFull;
-            cnt += s_red[1][w];
-            cand += s_red[2][w];
+        bool fit = t < ntiles;
+        uint64_t all = 0;
+#pragma unroll
+        for (uint32_t i = 0; i < 3; i++) {
+            uint64_t p = s_base[1 + 2 * i];
+            for (uint32_t w = 0; w < wave; w++) p = add_sat(p, s_w[w][i]);
+            p = i < m ? add_sat(p, inc[i]) : 0ull;
+            fit = fit && p <= room[i];
+            all = add_sat(all, p);
+        }
+        fit = fit && all <= room_all;
+        // prefixes only grow: the tiles that fit are the first ones
+        const uint64_t mask = __ballot(fit);
+        __syncthreads();
+        if (lane == 0) s_fit[wave] = (uint32_t)__popcll(mask);
+        for (uint32_t i = 0; i < 2 * m + 1; i++) {
+            const uint64_t x = wave_sum64(fit ? tile_sums[kTailWords * t + i] : 0ull);
+            if (lane == 0) s_w[wave][i] = x;
         }
         __syncthreads();
-        if (all > room) {  // candidate counts only grow: the tiles that fit are the first ones
-            tiles = t0 + fits;
-            break;
+        if (threadIdx.x < 2 * m + 1) {
+            uint64_t x = s_base[threadIdx.x];
+            for (uint32_t w = 0; w < W; w++) x += s_w[w][threadIdx.x];
+            s_base[threadIdx.x] = x;
         }
+        uint32_t n = 0;
+        for (uint32_t w = 0; w < W; w++) n += s_fit[w];
+        tiles += n;
+        __syncthreads();
+        if (n < kCutThreads) break;
     }
     if (threadIdx.x == 0) {
-        __hip_atomic_store(kc + 1, cand, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        __hip_atomic_store(kc + 2, cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        __hip_atomic_store(kc + 3, tiles, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        __hip_atomic_store(kc, kept, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+        for (uint32_t i = 0; i < 2 * m + 1; i++)
+            __hip_atomic_store(kc + 1 + i, s_base[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        __hip_atomic_store(kc, tiles, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 
@@ -1468,7 +1643,7 @@ __global__ __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(8))) void
     for (TileDeal dl; dl.tile() < a.io.ntiles; dl.next()) {  // dealt by XCD, as for LAST_COUNT
         const uint64_t t = dl.tile();
         __syncthreads();
-        expand_tile<EXPAND_LAST_BARE, I>(a.g, a.dp, a.col, a.dcol, a.io, t, t, 0, a.ws, ep, a.dp.inj, a.linj, a.pool_words, sh, smem,
+        expand_tile<EXPAND_LAST_BARE, I>(a.g, a.dp, a.tail, a.col, a.dcol, a.io, t, t, 0, a.ws, ep, a.dp.inj, a.pool_words, sh, smem,
                                          acc_cnt, acc_h0, acc_h1, false);
     }
     flush_sums(acc_cnt, 0, 0, a.io.tot, sh.red);
@@ -1502,44 +1677,39 @@ DEV uint64_t capped_chunk(const BatchSlot &B, uint32_t d, uint64_t n, uint64_t c
 }
 
 // What a slot's finished tail step counted: the sums over its first tiles whose
-// last-depth candidates fit the cap, and how many tiles those are.
+// candidates fit the caps, and how many tiles those are.
 struct TailSums {
-    uint64_t kept, cand, cnt, tiles;
+    uint64_t sum[2 * GFSM_MAXTAIL + 1], tiles;
 };
 
-// Last-depth candidates that the caps of slot B leave for its running tail step.
-DEV uint64_t tail_room(const BatchSlot &B)
+// The sums of the tail step of slot B, by all 64 lanes of one wave.
+DEV TailSums wave_tail_sums(gptr_t<const uint64_t> sums, const BatchSlot &B)
 {
-    uint64_t room = ~0ull;
-    if (B.max_depth_cand) room = B.max_depth_cand - umin64(B.max_depth_cand, B.cand[B.q - 1]);
-    if (B.max_cand) room = umin64(room, B.max_cand - umin64(B.max_cand, B.cand_done));
-    return room;
-}
-
-// The sums of a slot's `n` tail tiles, by all 64 lanes of one wave.
-DEV TailSums wave_tail_sums(gptr_t<const uint64_t> sums, uint64_t n, uint64_t room)
-{
-    const uint32_t lane = lane_id();
-    TailSums r{0, 0, 0, n};
+    const uint32_t lane = lane_id(), m = B.tail;
+    const uint64_t n = B.io.ntiles;
+    TailSums r{};
     for (uint64_t t0 = 0; t0 < n; t0 += 64) {
         const uint64_t t = t0 + lane;
-        const uint64_t e = t < n ? sums[2 * t] : 0ull, p = t < n ? sums[2 * t + 1] : 0ull;
-        const uint64_t c = p & ((1ull << kTailKeptShift) - 1);
-        uint64_t inc = c;
-        for (uint32_t o = 1; o < 64; o <<= 1) {
-            const uint64_t v = __shfl_up(inc, o, 64);
-            if (lane >= o) inc += v;
+        bool fit = t < n;
+        uint64_t all = 0;
+        for (uint32_t i = 0; i < m; i++) {
+            uint64_t inc = t < n ? sums[kTailWords * t + 1 + 2 * i] : 0ull;
+            for (uint32_t o = 1; o < 64; o <<= 1) {
+                const uint64_t v = __shfl_up(inc, o, 64);
+                if (lane >= o) inc = add_sat(inc, v);
+            }
+            inc = add_sat(inc, r.sum[1 + 2 * i]);
+            if (B.max_depth_cand)
+                fit = fit && inc <= B.max_depth_cand - umin64(B.max_depth_cand, B.cand[B.d + 1 + i]);
+            all = add_sat(all, inc);
         }
-        const bool fit = r.cand + inc <= room;
-        r.kept += wave_sum64(fit ? p >> kTailKeptShift : 0ull);
-        r.cnt += wave_sum64(fit ? e : 0ull);
-        const uint64_t cand = wave_sum64(fit ? c : 0ull);
-        const uint64_t m = __ballot(fit);
-        r.cand += cand;
-        if (m != ~0ull) {
-            r.tiles = t0 + (uint64_t)__builtin_ctzll(~m);
-            break;
-        }
+        if (B.max_cand) fit = fit && all <= B.max_cand - umin64(B.max_cand, B.cand_done);
+        const uint64_t mask = __ballot(fit);
+#pragma unroll
+        for (uint32_t i = 0; i < 2 * GFSM_MAXTAIL + 1; i++)
+            if (i < 2 * m + 1) r.sum[i] += wave_sum64(fit ? sums[kTailWords * t + i] : 0ull);
+        r.tiles += (uint64_t)__popcll(mask);
+        if (mask != ~0ull) break;  // the tiles that fit are the first ones
     }
     return r;
 }
@@ -1568,7 +1738,7 @@ DEV uint32_t schedule_slot(const BatchCfg &cfg, BatchSlot &B, Totals *tot, const
             B.chunk[k] = (k + 1 < q) ? umin64(B.cap[k], limit) : limit;
         }
         B.chunk[0] = umax64(TC, umin64(B.cap[0], limit));
-        if (B.tail && q >= 3) B.chunk[q - 2] = limit;  // writes no level
+        if (B.tail) B.chunk[q - 1 - B.tail] = limit;  // writes no level
         if (B.max_depth_cand) {  // capped: start small, grow from the observed fan-out
             B.chunk[0] = umax64(TC, umin64(B.chunk[0], umax64(B.max_depth_cand / 64, floor)));
             for (uint32_t k = 1; k < GFSM_MAXQ; k++) B.chunk[k] = 0;  // set at the depth's first step
@@ -1616,24 +1786,30 @@ DEV uint32_t schedule_slot(const BatchCfg &cfg, BatchSlot &B, Totals *tot, const
             }
         } else if (B.step == EXPAND_TAIL) {
             B.steps++;
+            const uint32_t m = B.tail;
             uint64_t to = e;
             if (ts.tiles < B.io.ntiles) {
                 // The cap's last candidate falls in the next tile, which is
                 // expanded level by level and ends the match.
                 to = b + ts.tiles * TC;
                 B.cand_done -= e - to;
-                B.tail = 0;
+                B.tail = m - 1;
+                B.chunk[d] = TC;
+            } else if (B.max_depth_cand) {
+                uint64_t ch = limit;
+                for (uint32_t i = 0; i < m; i++)
+                    ch = capped_chunk(B, d + i, to - b, ts.sum[1 + 2 * i], ch, TC, limit, floor);
+                B.chunk[d] = ch;
             }
-            if (B.max_depth_cand && to > b)
-                B.chunk[d] = capped_chunk(B, d, to - b, ts.cand, limit, TC, limit, floor);
-            if (!B.tail) B.chunk[d] = TC;
             B.lo[d] = to;
             B.cand[d] += to - b;
-            B.level[d] += ts.kept;
-            B.cand[d + 1] += ts.cand;
-            B.level[d + 1] += ts.cnt;
-            B.cand_done += ts.cand;
-            B.count += ts.cnt;
+            B.level[d] += ts.sum[0];
+            for (uint32_t i = 0; i < m; i++) {
+                B.cand[d + 1 + i] += ts.sum[1 + 2 * i];
+                B.level[d + 1 + i] += ts.sum[2 + 2 * i];
+                B.cand_done += ts.sum[1 + 2 * i];
+            }
+            B.count += ts.sum[2 * m];
         } else if (B.step == EXPAND_LAST_COUNT) {
             B.steps++;
             B.lo[d] = e;
@@ -1675,8 +1851,8 @@ DEV uint32_t schedule_slot(const BatchCfg &cfg, BatchSlot &B, Totals *tot, const
     }
     if (d >= 1) {
         const uint32_t kind = (d == (int32_t)q - 1)                ? (uint32_t)EXPAND_LAST_COUNT
-                              : (B.tail && d == (int32_t)q - 2) ? (uint32_t)EXPAND_TAIL
-                                                                : (uint32_t)EXPAND_MID;
+                              : (d + 1 + (int32_t)B.tail >= (int32_t)q) ? (uint32_t)EXPAND_TAIL
+                                                                        : (uint32_t)EXPAND_MID;
         const uint64_t b = B.lo[d];
         if (!B.chunk[d])
             B.chunk[d] = umax64(TC, umin64(umin64(kind == EXPAND_MID ? B.cap[d] : limit, limit),
@@ -1709,7 +1885,7 @@ DEV uint32_t schedule_slot(const BatchCfg &cfg, BatchSlot &B, Totals *tot, const
             io.out_gbeg = B.gbeg[d];
             io.cap = B.cap[d];
         }
-        io.need_nxt = kind != EXPAND_LAST_COUNT && dp.nxt_dist > 1 ? 1u : 0u;
+        io.need_nxt = kind == EXPAND_MID && dp.nxt_dist > 1 ? 1u : 0u;
         io.tot = tot;
         io.ntiles = (e - b + TC - 1) / TC;
         io.d = (uint32_t)d;
@@ -1826,9 +2002,9 @@ __global__ __launch_bounds__(kTile) void k_batch_schedule(BatchCfg cfg)
         wave_sync_lds();
         BatchSlot &B = *reinterpret_cast<BatchSlot *>(lw);
         uint32_t fin = 0;
-        TailSums ts{0, 0, 0, 0};
+        TailSums ts{};
         if (B.state == SLOT_RUN && B.step == EXPAND_TAIL)
-            ts = wave_tail_sums(gp((const uint64_t *)cfg.tile_node) + 2 * B.tile0, B.io.ntiles, tail_room(B));
+            ts = wave_tail_sums(gp((const uint64_t *)cfg.tail_sums) + kTailWords * B.tile0, B);
         if (lane == 0) {
             const uint32_t before = B.state;
             const uint32_t nt = schedule_slot(cfg, B, &cfg.slots[s].tot, ts);
@@ -1991,22 +2167,22 @@ __global__ __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(4))) void
             uint64_t c = 0, h0 = 0, h1 = 0;
             const StepIO io = uniform_copy(B.io);
             const uint32_t inj = (uint32_t)__builtin_amdgcn_readfirstlane((int)plan->depth[B.d].inj);
-            expand_tile<EXPAND_MID, I>(cfg.g, plan->depth[B.d], plan->col, plan->dcol, io, t - t0, t, t0, ws,
-                                       ep, inj, 0u, cfg.pool_words, sh, smem, c, h0, h1);
+            expand_tile<EXPAND_MID, I>(cfg.g, plan->depth[B.d], plan->tail[0], plan->col, plan->dcol, io, t - t0, t, t0, ws,
+                                       ep, inj, cfg.pool_words, sh, smem, c, h0, h1);
         } else if (step == EXPAND_TAIL) {
-            uint64_t c = 0, kept = 0, cand = 0;
+            uint64_t c = 0, h0 = 0, h1 = 0;
             const StepIO io = uniform_copy(B.io);
             const uint32_t inj = (uint32_t)__builtin_amdgcn_readfirstlane((int)plan->depth[B.d].inj);
-            const uint32_t linj = (uint32_t)__builtin_amdgcn_readfirstlane((int)plan->depth[B.d + 1].inj);
-            expand_tile<EXPAND_TAIL, I>(cfg.g, plan->depth[B.d], plan->col, plan->dcol, io, t - t0, t, t0, ws, ep, inj,
-                                        linj, cfg.pool_words, sh, smem, c, kept, cand);
-            tail_tile_sums(cfg.tile_node, t, c, kept, cand, sh.red);
+            if (threadIdx.x < kTailWords) sh.tsum[threadIdx.x] = 0;
+            expand_tile<EXPAND_TAIL, I>(cfg.g, plan->depth[B.d], plan->tail[B.tail - 1], plan->col, plan->dcol, io,
+                                        t - t0, t, t0, ws, ep, inj, cfg.pool_words, sh, smem, c, h0, h1);
+            tail_tile_end(cfg.tail_sums, t, sh.tsum);
         } else {
             uint64_t c = 0, h0 = 0, h1 = 0;
             const StepIO io = uniform_copy(B.io);
             const uint32_t inj = (uint32_t)__builtin_amdgcn_readfirstlane((int)plan->depth[B.d].inj);
-            expand_tile<EXPAND_LAST_COUNT, I>(cfg.g, plan->depth[B.d], plan->col, plan->dcol, io, t - t0, t, t0,
-                                              ws, ep, inj, 0u, cfg.pool_words, sh, smem, c, h0, h1);
+            expand_tile<EXPAND_LAST_COUNT, I>(cfg.g, plan->depth[B.d], plan->tail[0], plan->col, plan->dcol, io, t - t0, t, t0,
+                                              ws, ep, inj, cfg.pool_words, sh, smem, c, h0, h1);
             flush_sums(c, h0, h1, io.tot, sh.red);
         }
     }
@@ -2172,28 +2348,38 @@ static hipError_t launch_expand_bare_t(const ExpandArgs &a, uint32_t grid, hipSt
     return hipGetLastError();
 }
 
-template <uint32_t I>
+template <uint32_t KIND, uint32_t I>
 static hipError_t launch_expand_tail_t(const ExpandArgs &a, uint32_t grid, hipStream_t s)
 {
     static bool attr = false;
     const size_t lds = expand_lds_bytes(I, a.pool_words);
-    if (lds > kMaxDynLds) return hipErrorInvalidValue;
-    hipError_t e = allow_lds(&k_expand_tail<I>, attr);
+    if (lds > kMaxDynLds || a.tail.m == 0 || a.tail.m > GFSM_MAXTAIL) return hipErrorInvalidValue;
+    hipError_t e = allow_lds(&k_expand_tail<KIND, I>, attr);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((k_expand_tail<I>), dim3(grid), dim3(kTile), lds, s, a);
+    hipLaunchKernelGGL((k_expand_tail<KIND, I>), dim3(grid), dim3(kTile), lds, s, a);
     e = hipGetLastError();
     if (e != hipSuccess || !a.io.host_kc) return e;
-    hipLaunchKernelGGL(k_tail_cut, dim3(1), dim3(kTile), 0, s, a.tail_sums, a.io.ntiles, a.room, a.io.host_kc);
+    hipLaunchKernelGGL(k_tail_cut, dim3(1), dim3(kCutThreads), 0, s, a.tail_sums, a.io.ntiles, a.tail.m, a.room[0],
+                       a.room[1], a.room[2], a.room_all, a.io.host_kc);
     return hipGetLastError();
 }
 
 static hipError_t launch_expand_tail(const ExpandArgs &a, uint32_t grid, hipStream_t s)
 {
+    if (a.tail.wide) {
+        static_assert(kWideItems == 4, "widest wide tail");
+        switch (a.items) {
+        case 1: return launch_expand_tail_t<EXPAND_TAIL_WIDE, 1>(a, grid, s);
+        case 2: return launch_expand_tail_t<EXPAND_TAIL_WIDE, 2>(a, grid, s);
+        case 4: return launch_expand_tail_t<EXPAND_TAIL_WIDE, 4>(a, grid, s);
+        default: return hipErrorInvalidValue;
+        }
+    }
     switch (a.items) {
-    case 1: return launch_expand_tail_t<1>(a, grid, s);
-    case 2: return launch_expand_tail_t<2>(a, grid, s);
-    case 4: return launch_expand_tail_t<4>(a, grid, s);
-    case 8: return launch_expand_tail_t<8>(a, grid, s);
+    case 1: return launch_expand_tail_t<EXPAND_TAIL, 1>(a, grid, s);
+    case 2: return launch_expand_tail_t<EXPAND_TAIL, 2>(a, grid, s);
+    case 4: return launch_expand_tail_t<EXPAND_TAIL, 4>(a, grid, s);
+    case 8: return launch_expand_tail_t<EXPAND_TAIL, 8>(a, grid, s);
     default: return hipErrorInvalidValue;
     }
 }

@@ -108,6 +108,63 @@ void set_injectivity(const HostGraph &data, Plan &plan)
     }
 }
 
+// Graphs whose largest degree is at most this have no hubs: a candidate's sets
+// are compared entry by entry on one thread (checks, pairs), 64 x 64 at worst.
+// Past it such a leaf is placed, its candidates spread over the threads.
+static constexpr uint32_t kWideDegree = 64;
+
+void set_tails(const HostGraph &data, Plan &plan, bool wide)
+{
+    const uint32_t q = plan.q;
+    const bool by_label = data.mode == GFSM_MODE_VLABEL;
+    wide = wide && data.max_degree <= kWideDegree && data.V < 0xFFFFFFFEu;
+    auto label = [&](uint32_t k) { return by_label ? (plan.dev.depth[k].gen_rel >> 10) & 0x7FFu : 0u; };
+    uint32_t bits = 1;  // of a segment's length
+    while (bits < 32 && (data.max_degree >> bits)) bits++;
+    for (uint32_t m = 1; m <= GFSM_MAXTAIL; m++) {
+        TailPlanDev &tp = plan.dev.tail[m - 1];
+        tp = TailPlanDev{};
+        // A tile keeps at most 2^11 nodes; its number of completions fits 62 bits.
+        if (q < m + 2 || m * bits + 11 > 62) continue;
+        const uint32_t d = q - 1 - m;
+        bool ok = true, any_wide = false;
+        for (uint32_t i = 0; i < m && ok; i++) {
+            const uint32_t k = d + 1 + i;
+            const DepthPlanDev &dp = plan.dev.depth[k];
+            TailLeafDev &l = tp.leaf[i];
+            l.col = k - dp.gen_dist;
+            l.rel = dp.gen_rel;
+            l.inj = dp.inj & (uint32_t)((1ull << (d + 1)) - 1);
+            l.nchk = dp.nchk;
+            ok = l.col <= d && (dp.nchk == 0 || (wide && dp.nchk <= GFSM_TAILCHK));
+            for (uint32_t r = 0; r < dp.nchk && ok; r++) {
+                ok = dp.chk_dist[r] && k - dp.chk_dist[r] <= d;
+                l.chk_col[r] = k - dp.chk_dist[r];
+                l.chk_rel[r] = dp.chk_rel[r];
+            }
+            // Earlier leaves with the same label: all this very set, or one
+            // other set, the leaf before it, that meets nothing else.
+            uint32_t same = 0, twin = 0;
+            for (uint32_t j = 0; j < i && ok; j++) {
+                if (label(d + 1 + j) != label(k)) continue;
+                same++;
+                const TailLeafDev &o = tp.leaf[j];
+                if (o.col == l.col && o.rel == l.rel && !o.nchk && !l.nchk && !o.pair && !data.has_dups) twin++;
+            }
+            if (same == twin)
+                l.twins = twin;
+            else if (wide && same == 1 && label(k - 1) == label(k) && !tp.leaf[i - 1].pair)
+                l.pair = 1;
+            else
+                ok = false;
+            any_wide = any_wide || l.nchk || l.pair;
+        }
+        if (!ok) continue;
+        tp.m = m;
+        tp.wide = any_wide ? 1u : 0u;
+    }
+}
+
 Status plan_query(const HostGraph &qg, Plan &out, const HostGraph *by_cost)
 {
     out = Plan{};

@@ -34,6 +34,29 @@ struct DepthPlanDev {
     const void *chk_seg[4];
 };
 
+// The last depths of a query as leaves: each generated from, and checked
+// against, vertices placed at depths <= d only, so that a node of depth d has a
+// number of completions that is counted from the leaves' candidate sets (the
+// entries of the generator's segment that pass the checks and are no placed
+// vertex) without placing them.
+#define GFSM_MAXTAIL 3
+#define GFSM_TAILCHK 2
+struct TailLeafDev {
+    uint32_t col, rel;  // generator: depth of its ancestor (<= d), relation
+    uint32_t inj;       // placed columns (bits 0..d) its candidates can equal
+    uint32_t twins;     // earlier leaves of the tail with this very set
+    uint32_t pair;      // 1: may also meet the leaf before it, whose set is another
+    uint32_t nchk;
+    uint32_t chk_col[GFSM_TAILCHK], chk_rel[GFSM_TAILCHK];
+    const void *tab;    // dense segment tables, as in DepthPlanDev
+    const void *chk_tab[GFSM_TAILCHK];
+};
+struct TailPlanDev {
+    uint32_t m;         // leaves: depths d + 1 .. q - 1 (0: not countable this way)
+    uint32_t wide;      // some leaf has checks or a pair
+    TailLeafDev leaf[GFSM_MAXTAIL];
+};
+
 struct QueryPlanDev {
     uint32_t q;
     uint32_t root_rel;                   // generator relation of depth 1
@@ -42,4 +65,5 @@ struct QueryPlanDev {
     uint32_t col[GFSM_MAXQ];             // original query id placed at depth d
     uint32_t dcol[GFSM_MAXQ];            // depth whose vertex is column c
     DepthPlanDev depth[GFSM_MAXQ];
+    TailPlanDev tail[GFSM_MAXTAIL];      // tail[m - 1]: the last m depths as leaves of depth q - 1 - m
 };

@@ -235,7 +235,7 @@ Status server_submit(Server &s, const HostGraph &query, const gfsm_match_opts *o
     job->query = &query;
     if (opts) job->opts = *opts;
     job->opts.flags |= s.opts.flags;
-    Status plan_st = (query.mode == s.data->mode) ? plan_for(*s.data, query, job->opts, job->plan)
+    Status plan_st = (query.mode == s.data->mode) ? plan_for(*s.data, query, job->opts, job->plan, false)
                                                    : Status::err(GFSM_ERR_ARG, "query and data graph use different modes");
     // The level model is worked out here, on the submitting thread, so the
     // worker's admission loop only compares sizes.

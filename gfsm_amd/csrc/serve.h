@@ -125,6 +125,7 @@ private:
     std::vector<std::unique_ptr<BatchJob>> jobs_;  // per slot
     uint32_t running_ = 0;
     uint64_t steps_ = 0, since_clear_ = 0;
+    uint64_t step_limit_ = 0;            // candidates of a slot's step that the tile words allow every slot
     uint64_t step_cand_ = 0;             // per-slot step size last written to the device
     double calib_ = 1, calib_log_ = 0;   // projection calibration (see calibrate)
     uint64_t calib_n_ = 0;

@@ -1,6 +1,6 @@
-"""Counts whose last depth has no checks: the last two depths are counted from
-the one before (no level between them), against the digest run, which expands
-every level, and the oracle."""
+"""Counts whose last depths are leaves (each generated from and checked against
+earlier depths only): the leaves are counted without being placed, against the
+digest run, which expands every level, and the oracle."""
 import numpy as np
 import pytest
 
@@ -35,9 +35,15 @@ def _query(edges, labels, mode):
 
 
 def _queries(mode, rng):
-    shapes = [  # path (last vertex hangs off the new one), star and comb (off an older one), cycle with a tail
-        [(0, 1), (1, 2)], [(0, 1), (1, 2), (2, 3)], [(0, 1), (0, 2), (0, 3)], [(0, 1), (1, 2), (0, 3), (1, 4)],
-        [(0, 1), (1, 2), (2, 0), (2, 3)], [(0, 1), (1, 2), (2, 3), (3, 4)],
+    shapes = [
+        [(0, 1), (1, 2)], [(0, 1), (1, 2), (2, 3)], [(0, 1), (1, 2), (2, 3), (3, 4)],  # paths: two leaves that meet
+        [(0, 1), (0, 2), (0, 3)], [(0, 1), (0, 2), (0, 3), (0, 4)],  # stars: leaves with one set
+        [(0, 1), (1, 2), (0, 3), (1, 4)], [(0, 1), (0, 2), (0, 3), (1, 4), (1, 5)],  # comb, double star
+        [(0, 1), (1, 2), (2, 0), (2, 3)], [(0, 1), (1, 2), (2, 0), (0, 3), (1, 4)],  # triangle with one, two tails
+        [(0, 1), (1, 2), (2, 3), (3, 0)], [(0, 1), (1, 2), (2, 3), (3, 4), (4, 0)],  # cycles: a checked leaf
+        [(0, 1), (1, 2), (3, 4), (4, 5), (0, 3), (1, 4), (2, 5)],  # 2 x 3 patch: checked leaves
+        [(0, 1), (0, 2), (0, 3), (1, 4), (2, 4), (2, 5), (3, 5)],  # two checked leaves that meet
+        [(0, 1), (1, 2), (2, 0), (0, 3), (1, 3), (2, 3)],  # K4: a leaf with two checks
     ]
     return [_query(s, [1] * (max(map(max, s)) + 1) if k % 2 else rng.integers(1, 4, size=max(map(max, s)) + 1), mode)
             for s in shapes for k in (0, 1)]
@@ -57,9 +63,12 @@ def test_counts_equal_the_expanded_run(ctx, kind, mode):
             assert m.count == full.count, (i, kw)
             assert m.stats["level"] == full.stats["level"] and m.stats["cand"] == full.stats["cand"], (i, kw)
         assert ctx.match_batch(data, [q])[0].count == full.count, i
-        # caps before, inside and past the last depth's candidates, and one that is exactly enough
+        # caps before, inside and past every depth's candidates, and some that are exactly enough
         last = full.stats["cand"][-1]
-        for cap in {1, max(1, last // 3), max(1, last - 1), max(1, last), last + 1, 1 << 40}:
+        caps = {1, max(1, last // 3), max(1, last - 1), max(1, last), last + 1, 1 << 40}
+        for c in full.stats["cand"][1:]:
+            caps |= {max(1, c - 1), max(1, c), c + 1}
+        for cap in sorted(caps):
             a = ctx.match(data, q, max_depth_cand=cap, allow_partial=True, digest=True)
             for kw in (dict(), dict(tile=256), dict(mem_budget=2 << 20)):
                 b = ctx.match(data, q, max_depth_cand=cap, allow_partial=True, **kw)
