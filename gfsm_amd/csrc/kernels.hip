@@ -307,14 +307,9 @@ DEV void tile_prefix(uint64_t t, uint64_t t0, const ScanWS &ws, uint32_t ep, Sca
 {
     const uint32_t lane = lane_id(), wave = threadIdx.x >> 6;
     if (wave == 0) {
-        uint64_t ak = 0, ac = 0;
-#pragma unroll
-        for (uint32_t k = 0; k < I; k++)
-#pragma unroll
-            for (uint32_t w = 0; w < kWaves; w++) {
-                ak += sm.wk[k][w];
-                ac += sm.wc[k][w];
-            }
+        static_assert(I * kWaves <= 64, "one count per lane");
+        const uint64_t ak = wave_sum64(lane < I * kWaves ? (&sm.wk[0][0])[lane] : 0u);
+        const uint64_t ac = wave_sum64(lane < I * kWaves ? (&sm.wc[0][0])[lane] : 0ull);
         uint64_t ek = 0, ec = 0;
         if (t != t0) {
             if (lane == 0) {
@@ -1187,51 +1182,57 @@ DEV void expand_tile(const DevGraphView &g, const DP &dp, const TP &tl, CP col, 
                 }
             }
             __syncthreads();
+            // Kept nodes and candidates before this wave's part of every item:
+            // lane l holds count l of the tile (item l / kWaves, wave l % kWaves);
+            // the prefixes come from wave scans, formed while the look-back waits,
+            // and go to scalar registers (measured against every lane summing all
+            // counts from LDS: 3 x 3 patch of the grid 10.6 -> 10.5 ms, 256-query
+            // batch 12.1 -> 11.1 ms; after the look-back they cost 0.6%).  (A
+            // wave's candidates of one item stay under 2^32: in two halves their
+            // 32-bit prefixes cannot wrap.)
+            const uint32_t ck = lane < I * kWaves ? (&sm.wk[0][0])[lane] : 0u;
+            const uint32_t cc = lane < I * kWaves ? (uint32_t)(&sm.wc[0][0])[lane] : 0u;
+            const uint32_t sk = wave_incl_scan(ck) - ck;
+            const uint32_t sl = wave_incl_scan(cc & 0xFFFFu) - (cc & 0xFFFFu);
+            const uint32_t sh16 = wave_incl_scan(cc >> 16) - (cc >> 16);
             tile_prefix<I>(gt, gt0, ws, ep, sm, &sh.next);
-            uint64_t bk = sm.ex[0], bc = sm.ex[1];
-            uint64_t idx[I];
+            const uint32_t wv = (uint32_t)__builtin_amdgcn_readfirstlane((int)wave);
+            const uint64_t bk = uniform_copy(sm.ex[0]), bc = uniform_copy(sm.ex[1]);
             bool put[I];
-            // MID rows of one wave and item are consecutive in the next
-            // level: staged in this wave's share of s_seg (free after phase
+            // The rows of one wave and item are consecutive in the next level
+            // (or, of q = d + 1 words in original ids, in the output): staged in this wave's share of s_seg (free after phase
             // 1) and written out as whole words by all lanes, instead of
             // each lane storing its row with a stride of d + 1 words.
             const uint32_t row_w = d + 1;
-            const bool coalesce = KIND == EXPAND_MID && row_w * 64 <= TC / kWaves;
+            const bool coalesce = row_w * 64 <= TC / kWaves;
             uint32_t *wst = s_seg + wave * (TC / kWaves);
 #pragma unroll
             for (uint32_t k = 0; k < I; k++) {
-                uint64_t ok_ = bk, oc_ = bc;
-#pragma unroll
-                for (uint32_t ww = 0; ww < kWaves; ww++) {
-                    if (ww < wave) {
-                        ok_ += sm.wk[k][ww];
-                        oc_ += sm.wc[k][ww];
-                    }
-                    bk += sm.wk[k][ww];
-                    bc += sm.wc[k][ww];
-                }
-                idx[k] = ok_ + kpre[k];
-                put[k] = keep[k] && idx[k] < io.cap;
+                const uint32_t at = k * kWaves + wv;
+                const uint64_t ok_ = bk + (uint32_t)__builtin_amdgcn_readlane(sk, at);
+                const uint64_t oc_ = bc + (uint32_t)__builtin_amdgcn_readlane(sl, at) +
+                                     ((uint64_t)(uint32_t)__builtin_amdgcn_readlane(sh16, at) << 16);
+                // rows of this wave and item that the level holds
+                const uint64_t left = ok_ < io.cap ? io.cap - ok_ : 0u;
+                const uint32_t room = left < 64u ? (uint32_t)left : 64u;
+                put[k] = keep[k] && kpre[k] < room;
                 if (KIND == EXPAND_MID && put[k]) {
-                    out_off[idx[k]] = oc_ + cpre[k];
-                    out_gbeg[idx[k]] = gb[k];
-                } else if (KIND == EXPAND_LAST_ROWS && put[k]) {
-                    out_rows[idx[k] * io.q + col[d]] = w[k];
+                    (out_off + ok_)[kpre[k]] = oc_ + cpre[k];
+                    (out_gbeg + ok_)[kpre[k]] = gb[k];
                 }
-                if (KIND == EXPAND_MID && coalesce) {
+                if (coalesce) {
                     if (put[k]) {
                         uint32_t *sr = wst + kpre[k] * row_w;
-                        for (uint32_t kk = 0; kk < d; kk++) sr[kk] = rows.at(jj[k], kk);
-                        sr[d] = w[k];
+                        for (uint32_t kk = 0; kk < d; kk++) sr[KIND == EXPAND_MID ? kk : col[kk]] = rows.at(jj[k], kk);
+                        sr[KIND == EXPAND_MID ? d : col[d]] = w[k];
                     }
                     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
                     __builtin_amdgcn_wave_barrier();
                     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
                     // rows [ok_, ok_ + nrow) of the level, capped at its capacity
-                    uint64_t nrow = (uint64_t)__popcll(__ballot(keep[k]));
-                    nrow = ok_ >= io.cap ? 0 : (nrow < io.cap - ok_ ? nrow : io.cap - ok_);
-                    const uint32_t words = (uint32_t)nrow * row_w;  // at most 64 * I
-                    const auto dst = out_vec + ok_ * row_w;
+                    const uint32_t kept = (uint32_t)__popcll(__ballot(keep[k]));
+                    const uint32_t words = (kept < room ? kept : room) * row_w;  // at most 64 * I
+                    const auto dst = (KIND == EXPAND_MID ? out_vec : out_rows) + ok_ * row_w;
                     // 16-byte stores for the body (a quarter of the store
                     // instructions; the level is 256-byte aligned), single
                     // words for the head before the first 16-byte boundary
@@ -1258,19 +1259,11 @@ DEV void expand_tile(const DevGraphView &g, const DP &dp, const TP &tl, CP col, 
                     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
                     __builtin_amdgcn_wave_barrier();
                     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                } else if (KIND == EXPAND_MID && put[k]) {
-                    out_vec[idx[k] * row_w + d] = w[k];
-                }
-            }
-            // Otherwise the placed vertices, one column at a time for all items.
-            if (!(KIND == EXPAND_MID && coalesce)) {
-                for (uint32_t kk = 0; kk < d; kk++) {
-                    const uint32_t ck = (KIND == EXPAND_MID) ? kk : col[kk];
-                    const uint64_t wd = (KIND == EXPAND_MID) ? d + 1 : io.q;
-                    const auto out = (KIND == EXPAND_MID) ? out_vec : out_rows;
-#pragma unroll
-                    for (uint32_t k = 0; k < I; k++)
-                        if (put[k]) out[idx[k] * wd + ck] = rows.at(jj[k], kk);
+                } else if (put[k]) {
+                    // the placed vertices by each lane's own stores
+                    const auto out = (KIND == EXPAND_MID ? out_vec : out_rows) + ok_ * row_w + kpre[k] * row_w;
+                    out[KIND == EXPAND_MID ? d : col[d]] = w[k];
+                    for (uint32_t kk = 0; kk < d; kk++) out[KIND == EXPAND_MID ? kk : col[kk]] = rows.at(jj[k], kk);
                 }
             }
             if (lt == io.ntiles - 1 && tid == 0) {
