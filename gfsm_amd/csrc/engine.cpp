@@ -430,6 +430,9 @@ struct Runner {
     uint64_t chunk[GFSM_MAXQ] = {};
     uint32_t *rows_d = nullptr;
     uint64_t rows_cap = 0;
+    uint64_t rows_kept = 0;     // rows of the one chunk so far, still in rows_d (sorted runs)
+    char *level_base = nullptr; // the levels' part of the arena: free once the walk has ended
+    uint64_t level_bytes = 0;
     uint32_t grid_cap = 0;
     uint64_t max_cand = 0;      // work cap (0 = none)
     uint64_t cand_total = 0;    // candidates launched so far
@@ -538,7 +541,10 @@ struct Runner {
             p += round256(b);
             return r;
         };
+        const char *end = p + (fixed ? fixed->bytes : ctx.arena.bytes);
         if (rows_mode) rows_d = reinterpret_cast<uint32_t *>(take(rows_cap * q * 4));
+        level_base = p;
+        level_bytes = (uint64_t)(end - p);
         for (uint32_t k = 0; k + 1 < q; k++) {
             vec[k] = reinterpret_cast<uint32_t *>(take(cap[k] * 4 * (k + 1)));
             off[k] = reinterpret_cast<uint64_t *>(take((cap[k] + 1) * 8));
@@ -708,6 +714,51 @@ struct Runner {
         return Status::ok();
     }
 
+    // Appends the first `n` rows at `from` (device) to the result.
+    Status copy_rows(const uint32_t *from, uint64_t n)
+    {
+        const size_t at = res.rows.size();
+        res.rows.resize(at + n * q);
+        if (n) HIP_TRY(hipMemcpy(res.rows.data() + at, from, n * q * sizeof(uint32_t), hipMemcpyDeviceToHost));
+        return Status::ok();
+    }
+    Status copy_kept()
+    {
+        const uint64_t n = rows_kept;
+        rows_kept = 0;
+        return n ? copy_rows(rows_d, n) : Status::ok();
+    }
+
+    // Columns that a sorted run still has to be sorted by: its rows come ordered
+    // by the vertices in placement order, so once the first `n` columns are in
+    // order the others are too where their placement order is the column order.
+    uint32_t sort_columns() const
+    {
+        uint32_t n = q - 1;
+        while (n > 0 && plan.dev.dcol[n - 1] < plan.dev.dcol[n]) n--;
+        return n;
+    }
+
+    // The result's rows in sorted order: on the device where one chunk holds
+    // them all and the levels' memory has room for the sort, else on the host.
+    Status finish_sorted()
+    {
+        const uint32_t ncol = sort_columns();
+        uint32_t bits = 1;
+        while (bits < 32 && ((data.V - 1) >> bits)) bits++;
+        if (ncol && rows_kept && sort_rows_bytes(rows_kept, q) <= level_bytes) {
+            uint32_t *sorted = nullptr;
+            HIP_TRY(launch_sort_rows(rows_d, rows_kept, q, ncol, bits, level_base, &sorted, lane.stream));
+            HIP_TRY(hipStreamSynchronize(lane.stream));
+            const uint64_t n = rows_kept;
+            rows_kept = 0;
+            return copy_rows(sorted, n);
+        }
+        Status st = copy_kept();
+        if (st.good() && ncol) sort_rows(res.rows, q);
+        return st;
+    }
+
     // Expand depth d over candidates [g0, g1) of level d-1 (S_prev nodes).
     Status descend(uint32_t d, uint64_t g0, uint64_t g1, uint64_t S_prev)
     {
@@ -813,6 +864,10 @@ struct Runner {
                 HIP_TRY(launch_tile_index(io.in_off, S_prev, c, e, tc, io.ntiles, lane.tile_node, lane.stream));
                 io.tile_node = lane.tile_node;
             }
+            if (kind == EXPAND_LAST_ROWS && rows_kept) {  // the step overwrites them
+                Status cs = copy_kept();
+                if (!cs.good()) return cs;
+            }
             HIP_TRY(lane.before_launch());
             {
                 Status ks = kbegin();
@@ -915,11 +970,12 @@ struct Runner {
                     c = e;
                     continue;
                 }
-                size_t at = res.rows.size();
-                res.rows.resize(at + keep * q);
-                if (keep)
-                    HIP_TRY(hipMemcpy(res.rows.data() + at, rows_d, keep * q * sizeof(uint32_t),
-                                      hipMemcpyDeviceToHost));
+                if ((flags & GFSM_SORTED) && res.rows.empty()) {
+                    rows_kept = keep;
+                } else {
+                    st = copy_rows(rows_d, keep);
+                    if (!st.good()) return st;
+                }
             }
             c = e;
         }
@@ -1103,6 +1159,10 @@ Status run_match(Ctx &ctx, const HostGraph &data, const DevGraph &dg, const Plan
         res.digest[0] = run.sdg[0];
         res.digest[1] = run.sdg[1];
     } else if (run.rows_mode) {
+        if (o.flags & GFSM_SORTED) {
+            st = run.finish_sorted();
+            if (!st.good()) return st;
+        }
         res.count = res.rows.size() / q;
         res.stats.level[q - 1] = res.count;
         if (o.flags & GFSM_DIGEST) {
@@ -1116,7 +1176,6 @@ Status run_match(Ctx &ctx, const HostGraph &data, const DevGraph &dg, const Plan
             res.digest[0] = d0;
             res.digest[1] = d1;
         }
-        if (o.flags & GFSM_SORTED) sort_rows(res.rows, q);
     } else {
         res.count = L.tot_h->count + run.tail_count;
         if (run.leaves && !o.max_depth_cand && !o.max_cand) {

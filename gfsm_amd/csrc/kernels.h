@@ -339,6 +339,13 @@ static_assert(512 + 32 * kNoAllocTiles + 8 * kTailWords * kNoAllocTailTiles <= k
 // current; its workspace part cleared on `s`), then cached.
 hipError_t noalloc_scratch(int device, hipStream_t s, char **ptr);
 
+// Rows sorted by their first `ncol` columns (values of `bits` bits), equal ones
+// in their present order, into scratch `tmp` of sort_rows_bytes(n, q); *sorted =
+// the sorted rows there.
+uint64_t sort_rows_bytes(uint64_t n, uint32_t q);
+hipError_t launch_sort_rows(const uint32_t *rows, uint64_t n, uint32_t q, uint32_t ncol, uint32_t bits, void *tmp,
+                            uint32_t **sorted, hipStream_t s);
+
 // Traffic calibration (kernels of known footprint).  mode 0: dst[i] =
 // src[i] + 1 over n words (n words read and written); mode 1: one word from
 // each of n distinct 128-byte lines of src (n a power of two, src holding 32n

@@ -2297,8 +2297,179 @@ __global__ void k_ws_clear(ScanWS ws)
 }
 
 // ---------------------------------------------------------------------------
+// sorting an embedding table
+// ---------------------------------------------------------------------------
+
+// Stable radix sort of the rows' indices by the first `ncol` columns, eight bits
+// of the concatenated columns (`bits` each) a pass, least significant first:
+// per-block digit counts, their scan in (digit, block) order, and a scatter that
+// ranks equal digits of a wave with ballots.  A pass reads one or two words of
+// each row, a cache line in random order, and is otherwise a few microseconds of
+// launches.  Measured against the host's comparison sort (one thread below 100,000
+// rows, merged blocks above), whole calls: 12,288 rows of five columns 0.98 ->
+// 0.25 ms, 480,000 rows 5.2 -> 1.8 ms, 1,920,000 rows of seven 76 -> 20 ms.
+constexpr uint32_t kSortItems = 8, kSortBlock = kTile * kSortItems, kSortBins = 256;
+
+DEV uint32_t sort_digit(const uint32_t *__restrict__ rows, uint64_t row, uint32_t q, uint32_t ncol, uint32_t bits,
+                        uint32_t off)
+{
+    uint32_t d = 0, got = 0, sh = off % bits;
+    for (int32_t c = (int32_t)(ncol - 1 - off / bits); c >= 0 && got < 8; c--) {
+        const uint32_t take = 8 - got < bits - sh ? 8 - got : bits - sh;
+        d |= ((rows[row * q + (uint32_t)c] >> sh) & ((1u << take) - 1u)) << got;
+        got += take;
+        sh = 0;
+    }
+    return d;
+}
+
+__global__ __launch_bounds__(kTile) void k_sort_hist(const uint32_t *rows, const uint32_t *idx, uint64_t n, uint32_t q,
+                                                     uint32_t ncol, uint32_t bits, uint32_t off, uint32_t *hist)
+{
+    __shared__ uint32_t s_cnt[kSortBins];
+    s_cnt[threadIdx.x] = 0;
+    __syncthreads();
+#pragma unroll
+    for (uint32_t r = 0; r < kSortItems; r++) {
+        const uint64_t e = (uint64_t)blockIdx.x * kSortBlock + r * kTile + threadIdx.x;
+        if (e < n) atomicAdd(&s_cnt[sort_digit(rows, idx ? idx[e] : e, q, ncol, bits, off)], 1u);
+    }
+    __syncthreads();
+    hist[(uint64_t)threadIdx.x * gridDim.x + blockIdx.x] = s_cnt[threadIdx.x];
+}
+
+// Exclusive scan of `m` counts in place, one workgroup.
+constexpr uint32_t kSortScanThreads = 1024;
+__global__ __launch_bounds__(kSortScanThreads) void k_sort_scan(uint32_t *v, uint64_t m)
+{
+    constexpr uint32_t W = kSortScanThreads / 64, B = 4;
+    __shared__ uint32_t s_w[W];
+    const uint32_t lane = lane_id(), wave = threadIdx.x >> 6;
+    uint32_t carry = 0;
+    for (uint64_t i0 = 0; i0 < m; i0 += kSortScanThreads * B) {
+        const uint64_t i = i0 + threadIdx.x * B;
+        uint32_t x[B], sum = 0;
+#pragma unroll
+        for (uint32_t b = 0; b < B; b++) x[b] = i + b < m ? v[i + b] : 0u;
+#pragma unroll
+        for (uint32_t b = 0; b < B; b++) {
+            const uint32_t t = x[b];
+            x[b] = sum;
+            sum += t;
+        }
+        const uint32_t inc = wave_incl_scan(sum);
+        if (lane == 63) s_w[wave] = inc;
+        __syncthreads();
+        uint32_t base = carry + inc - sum, all = 0;
+        for (uint32_t w = 0; w < W; w++) {
+            if (w < wave) base += s_w[w];
+            all += s_w[w];
+        }
+        carry += all;
+#pragma unroll
+        for (uint32_t b = 0; b < B; b++)
+            if (i + b < m) v[i + b] = base + x[b];
+        __syncthreads();
+    }
+}
+
+__global__ __launch_bounds__(kTile) void k_sort_scatter(const uint32_t *rows, const uint32_t *idx, uint64_t n, uint32_t q,
+                                                        uint32_t ncol, uint32_t bits, uint32_t off,
+                                                        const uint32_t *hist, uint32_t *out)
+{
+    __shared__ uint32_t s_cnt[kWaves][kSortBins];
+    const uint32_t lane = lane_id(), wave = threadIdx.x >> 6;
+#pragma unroll
+    for (uint32_t w = 0; w < kWaves; w++) s_cnt[w][threadIdx.x] = 0;
+    __syncthreads();
+    // This wave's rows in order: 64 a round.
+    const uint64_t e0 = (uint64_t)blockIdx.x * kSortBlock + wave * (64 * kSortItems) + lane;
+    uint32_t id[kSortItems], dig[kSortItems], rank[kSortItems];
+#pragma unroll
+    for (uint32_t r = 0; r < kSortItems; r++) {
+        const uint64_t e = e0 + 64 * r;
+        id[r] = e < n ? (idx ? idx[e] : (uint32_t)e) : 0u;
+        dig[r] = e < n ? sort_digit(rows, id[r], q, ncol, bits, off) : 0u;
+    }
+#pragma unroll
+    for (uint32_t r = 0; r < kSortItems; r++) {
+        const bool in = e0 + 64 * r < n;
+        uint64_t same = __ballot(in);
+#pragma unroll
+        for (uint32_t b = 0; b < 8; b++) {
+            const bool one = (dig[r] >> b) & 1u;
+            const uint64_t m = __ballot(one);
+            same &= one ? m : ~m;
+        }
+        const uint32_t before = mask_prefix(same);
+        rank[r] = s_cnt[wave][dig[r]] + before;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (in && before == 0) s_cnt[wave][dig[r]] += (uint32_t)__popcll(same);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+    __syncthreads();
+    uint32_t at = hist[(uint64_t)threadIdx.x * gridDim.x + blockIdx.x];
+#pragma unroll
+    for (uint32_t w = 0; w < kWaves; w++) {
+        const uint32_t c = s_cnt[w][threadIdx.x];
+        s_cnt[w][threadIdx.x] = at;
+        at += c;
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t r = 0; r < kSortItems; r++)
+        if (e0 + 64 * r < n) out[s_cnt[wave][dig[r]] + rank[r]] = id[r];
+}
+
+__global__ void k_sort_gather(const uint32_t *rows, const uint32_t *idx, uint64_t words, uint32_t q, uint32_t *out)
+{
+    for (uint64_t u = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; u < words; u += (uint64_t)gridDim.x * blockDim.x) {
+        const uint64_t r = u / q;
+        out[u] = rows[(uint64_t)idx[r] * q + (u - r * q)];
+    }
+}
+
+// ---------------------------------------------------------------------------
 // launch wrappers
 // ---------------------------------------------------------------------------
+
+static uint64_t sort_blocks(uint64_t n) { return (n + kSortBlock - 1) / kSortBlock; }
+static uint64_t up256(uint64_t b) { return (b + 255) / 256 * 256; }
+
+uint64_t sort_rows_bytes(uint64_t n, uint32_t q)
+{
+    return up256(4 * n * q) + 2 * up256(4 * n) + up256(4 * kSortBins * sort_blocks(n));
+}
+
+hipError_t launch_sort_rows(const uint32_t *rows, uint64_t n, uint32_t q, uint32_t ncol, uint32_t bits, void *tmp,
+                            uint32_t **sorted, hipStream_t s)
+{
+    if (n == 0 || n > 0xFFFFFFFFull || q == 0 || ncol == 0 || ncol > q || bits == 0 || bits > 32)
+        return hipErrorInvalidValue;
+    const uint64_t nb = sort_blocks(n);
+    char *p = static_cast<char *>(tmp);
+    uint32_t *out = reinterpret_cast<uint32_t *>(p);
+    uint32_t *ia = reinterpret_cast<uint32_t *>(p += up256(4 * n * q));
+    uint32_t *ib = reinterpret_cast<uint32_t *>(p += up256(4 * n));
+    uint32_t *hist = reinterpret_cast<uint32_t *>(p += up256(4 * n));
+    const uint32_t *from = nullptr;  // the rows' own order
+    uint32_t *to = ia;
+    for (uint32_t off = 0; off < ncol * bits; off += 8) {
+        hipLaunchKernelGGL(k_sort_hist, dim3((uint32_t)nb), dim3(kTile), 0, s, rows, from, n, q, ncol, bits, off, hist);
+        hipLaunchKernelGGL(k_sort_scan, dim3(1), dim3(kSortScanThreads), 0, s, hist, kSortBins * nb);
+        hipLaunchKernelGGL(k_sort_scatter, dim3((uint32_t)nb), dim3(kTile), 0, s, rows, from, n, q, ncol, bits, off, hist,
+                           to);
+        from = to;
+        to = to == ia ? ib : ia;
+    }
+    const uint64_t words = n * q, wg = (words + 255) / 256;
+    hipLaunchKernelGGL(k_sort_gather, dim3((uint32_t)(wg < 65536 ? wg : 65536)), dim3(256), 0, s, rows, from, words, q,
+                       out);
+    *sorted = out;
+    return hipGetLastError();
+}
 
 size_t expand_lds_bytes(uint32_t items, uint32_t pool_words)
 {
