@@ -360,11 +360,24 @@ class Graph:
         return col, hdr, req[: 2 * mv.value * q.value]
 
 
+class _Result:
+    """Owns a result handle; the Match and a view of its rows both hold it."""
+
+    def __init__(self, handle):
+        self.h = handle
+
+    def __del__(self):
+        if self.h and self.h.value:
+            lib().gfsm_result_free(self.h)
+            self.h = C.c_void_p()
+
+
 class Match:
     """Result of one match: count, digest, optional rows and kernel statistics."""
 
     def __init__(self, handle):
         self._h = handle
+        self._own = _Result(handle)
         L = lib()
         n = C.c_uint64()
         _check(L.gfsm_result_count(handle, C.byref(n)))
@@ -378,7 +391,12 @@ class Match:
         w, nr = C.c_uint32(), C.c_uint64()
         _check(L.gfsm_result_rows(handle, C.byref(p), C.byref(w), C.byref(nr)))
         self.width = w.value
-        self.rows = _view(p, nr.value * w.value).reshape(nr.value, w.value) if nr.value else None
+        self.rows = None
+        if nr.value:
+            # the result's own memory, no copy: the array keeps the result alive
+            buf = (C.c_uint32 * (nr.value * w.value)).from_address(C.addressof(p.contents))
+            buf._own = self._own
+            self.rows = np.frombuffer(buf, dtype=np.uint32).reshape(nr.value, w.value)
 
     @property
     def stats(self):
@@ -391,11 +409,6 @@ class Match:
 
     def write_fs(self, path):
         _check(lib().gfsm_result_write_fs(self._h, str(path).encode()), "write_fs")
-
-    def __del__(self):
-        if getattr(self, "_h", None) and self._h.value:
-            lib().gfsm_result_free(self._h)
-            self._h = C.c_void_p()
 
 
 def _opts(rows=False, sorted=False, digest=False, profile=False, root_lo=0, root_hi=0, max_rows=0,

@@ -16,8 +16,10 @@
 #include <algorithm>
 #include <chrono>
 #include <cmath>
+#include <cstdlib>
 #include <cstring>
 #include <functional>
+#include <new>
 
 namespace gfsm {
 
@@ -34,6 +36,87 @@ static double now_ms()
         hipError_t e_ = (expr);                                          \
         if (e_ != hipSuccess) return hip_status(e_, #expr);              \
     } while (0)
+
+// Pinned blocks that results gave back, kept for the next ones (any thread, any
+// context): at most kPoolBlocks of them and kPoolBytes in all.  Measured, a call
+// returning 1,920,000 rows of seven: pageable rows, filled with zeros, copied into
+// and copied once more for the caller, 6-17 ms; straight into pinned memory that the
+// caller views, 1.25 ms.  With an allocation per call instead of the pool a call
+// with 12,288 rows took 0.29 ms, with it 0.24.
+namespace {
+struct RowHead {  // precedes the memory handed out
+    uint64_t bytes;  // handed out at most
+    uint64_t pinned;
+    uint64_t pad[6];
+};
+constexpr size_t kRowPinMin = 64u << 10, kRowPinMax = 1u << 30;  // past it pageable: pinned memory is the machine's
+constexpr size_t kPoolBlocks = 16, kPoolBytes = 512u << 20;
+struct RowPool {
+    std::mutex mu;
+    std::vector<RowHead *> free;
+    size_t bytes = 0;
+};
+RowPool &row_pool()
+{
+    static RowPool *p = new RowPool;  // never destroyed: results may be freed at exit
+    return *p;
+}
+}  // namespace
+
+void *row_alloc(size_t bytes)
+{
+    if (bytes >= kRowPinMin && bytes <= kRowPinMax) {
+        RowPool &pool = row_pool();
+        {
+            std::lock_guard<std::mutex> lk(pool.mu);
+            size_t best = pool.free.size();
+            for (size_t i = 0; i < pool.free.size(); i++) {
+                const uint64_t b = pool.free[i]->bytes;
+                if (b >= bytes && b / 4 <= bytes && (best == pool.free.size() || b < pool.free[best]->bytes)) best = i;
+            }
+            if (best < pool.free.size()) {
+                RowHead *h = pool.free[best];
+                pool.free.erase(pool.free.begin() + best);
+                pool.bytes -= h->bytes;
+                return h + 1;
+            }
+        }
+        const size_t grain = bytes < (2u << 20) ? kRowPinMin : (2u << 20);  // near sizes share blocks
+        const size_t room = (bytes + grain - 1) / grain * grain;
+        void *p = nullptr;
+        if (hipHostMalloc(&p, room + sizeof(RowHead), hipHostMallocPortable) == hipSuccess) {
+            RowHead *h = static_cast<RowHead *>(p);
+            h->bytes = room;
+            h->pinned = 1;
+            return h + 1;
+        }
+        (void)hipGetLastError();
+    }
+    RowHead *h = static_cast<RowHead *>(std::malloc(bytes + sizeof(RowHead)));
+    if (!h) throw std::bad_alloc();
+    h->bytes = bytes;
+    h->pinned = 0;
+    return h + 1;
+}
+
+void row_free(void *q)
+{
+    RowHead *h = static_cast<RowHead *>(q) - 1;
+    if (!h->pinned) {
+        std::free(h);
+        return;
+    }
+    RowPool &pool = row_pool();
+    {
+        std::lock_guard<std::mutex> lk(pool.mu);
+        if (pool.free.size() < kPoolBlocks && pool.bytes + h->bytes <= kPoolBytes) {
+            pool.free.push_back(h);
+            pool.bytes += h->bytes;
+            return;
+        }
+    }
+    (void)hipHostFree(h);
+}
 
 Status Lane::init(uint64_t max_tiles, bool tile_index, uint64_t tail)
 {
@@ -443,7 +526,7 @@ struct Runner {
     // host memory stays one chunk, whatever the result size.
     FILE *stream = nullptr;
     uint64_t streamed = 0, sdg[2] = {0, 0};
-    std::vector<uint32_t> stage;
+    RowVec stage;
 
     // The lane (stream, scan workspace, totals); optionally a fixed level
     // arena, with which nothing is allocated (dense tables only if cached).
@@ -755,7 +838,7 @@ struct Runner {
             return copy_rows(sorted, n);
         }
         Status st = copy_kept();
-        if (st.good() && ncol) sort_rows(res.rows, q);
+        if (st.good() && ncol) sort_rows(res.rows.data(), res.rows.size() / q, q);
         return st;
     }
 

@@ -396,14 +396,13 @@ Status write_tve(const HostGraph &g, const char *path)
 // Lexicographic row sort: LSD over columns with a stable counting pass per
 // 16-bit digit would touch the rows many times; a comparison sort on row
 // indices keeps it simple and is only used for host-side SORTED output.
-void sort_rows(std::vector<uint32_t> &rows, uint32_t width)
+void sort_rows(uint32_t *rows, size_t n, uint32_t width)
 {
     if (!width) return;
-    size_t n = rows.size() / width;
     if (n > 0xFFFFFFFFull) return;  // callers cap host-side sorting far below this
     std::vector<uint32_t> idx(n);
     for (size_t i = 0; i < n; i++) idx[i] = (uint32_t)i;
-    const uint32_t *R = rows.data();
+    const uint32_t *R = rows;
     auto less = [R, width](uint32_t a, uint32_t b) {
         const uint32_t *x = R + (size_t)a * width, *y = R + (size_t)b * width;
         for (uint32_t c = 0; c < width; c++)
@@ -429,12 +428,12 @@ void sort_rows(std::vector<uint32_t> &rows, uint32_t width)
         }
         for (auto &t : ts) t.join();
     }
-    std::vector<uint32_t> out(rows.size());
+    std::vector<uint32_t> out(n * width);
     parallel_for(n, [&](uint64_t b, uint64_t e) {
         for (uint64_t i = b; i < e; i++)
             std::memcpy(out.data() + i * width, R + (size_t)idx[i] * width, width * sizeof(uint32_t));
     });
-    rows.swap(out);
+    std::copy(out.begin(), out.end(), rows);
 }
 
 }  // namespace gfsm

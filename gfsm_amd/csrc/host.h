@@ -133,16 +133,46 @@ Status gen_grid(uint32_t rows, uint32_t cols, double del_frac, double diag_frac,
                 HostGraph *&out);
 Status gen_query_walk(const HostGraph &data, uint32_t qsize, uint32_t kind, uint64_t seed, HostGraph *&out);
 
+// Host memory of embedding tables: pinned where the runtime gives it (the
+// device copies straight into it; a copy into pageable memory goes through the
+// runtime's staging), never filled before it is written.
+void *row_alloc(size_t bytes);
+void row_free(void *p);
+template <class T>
+struct RowAlloc {
+    using value_type = T;
+    RowAlloc() = default;
+    template <class U>
+    RowAlloc(const RowAlloc<U> &) {}
+    T *allocate(size_t n) { return static_cast<T *>(row_alloc(n * sizeof(T))); }
+    void deallocate(T *p, size_t) { row_free(p); }
+    template <class U>
+    void construct(U *p)
+    {
+        ::new (static_cast<void *>(p)) U;  // not value-initialised: resize() leaves new rows unwritten
+    }
+    template <class U, class... A>
+    void construct(U *p, A &&...a)
+    {
+        ::new (static_cast<void *>(p)) U(static_cast<A &&>(a)...);
+    }
+    template <class U>
+    bool operator==(const RowAlloc<U> &) const { return true; }
+    template <class U>
+    bool operator!=(const RowAlloc<U> &) const { return false; }
+};
+using RowVec = std::vector<uint32_t, RowAlloc<uint32_t>>;
+
 struct Result {
     gfsm_status status = GFSM_OK;
     uint64_t count = 0;
     uint64_t digest[2] = {0, 0};
     uint32_t width = 0;
-    std::vector<uint32_t> rows;
+    RowVec rows;
     gfsm_stats stats{};
 };
 
-void sort_rows(std::vector<uint32_t> &rows, uint32_t width);
+void sort_rows(uint32_t *rows, size_t n, uint32_t width);
 uint64_t mix64(uint64_t z);
 void row_hash(const uint32_t *row, uint32_t width, uint64_t h[2]);
 

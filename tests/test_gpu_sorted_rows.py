@@ -43,3 +43,20 @@ def test_sorted_rows_under_caps(ctx):
     assert ctx.match(data, query, rows=True, sorted=True, max_rows=full.count).count == full.count
     with pytest.raises(G.GfsmError):
         ctx.match(data, query, rows=True, sorted=True, max_rows=full.count - 1)
+
+
+@pytest.mark.parametrize("n", [50, 5000, 60000])  # below and above the size from which the table is pinned
+def test_rows_outlive_match_and_context(n):
+    """The rows are a view of the result's memory: they stay valid, and can be
+    written, after the match, the graphs and the context are gone."""
+    ctx = G.Context(0)
+    data = G.Graph.er(n, 6.0, nvlabels=1, nelabels=1, seed=9200, mode=G.MODE_REF)
+    query = _path([1] * 3, (0, 1, 2), G.MODE_REF)
+    m = ctx.match(data, query, rows=True)
+    rows, copy = m.rows, m.rows.copy()
+    again = ctx.match(data, query, rows=True).rows  # another result in between
+    del m, data, query
+    ctx.close()
+    assert np.array_equal(rows, copy) and np.array_equal(again, copy)
+    rows[0, 0] += 1
+    assert rows[0, 0] == copy[0, 0] + 1 and np.array_equal(again, copy)
