@@ -389,8 +389,8 @@ bool BatchEngine::try_admit(std::unique_ptr<BatchJob> &job, Status &st)
     s.max_depth_cand = job->opts.max_depth_cand;
     s.q = plan.q;
     s.digest = (job->opts.flags & GFSM_DIGEST) ? 1u : 0u;
-    s.tail = 0;
-    for (uint32_t m = 1; !s.digest && m <= GFSM_MAXTAIL && plan.dev.tail[m - 1].m; m++) s.tail = m;
+    s.tail = s.digest ? 0u
+                      : usable_leaves(data_, plan, job->opts.max_depth_cand, (uint64_t)kTile * shape_.items);
     s.state = SLOT_NEW;
     s.step = STEP_NONE;
     n_admit_++;  // installed by the next replay's first scheduler launch

@@ -584,7 +584,7 @@ struct Runner {
         prof = flags & GFSM_PROFILE;
         leaves = 0;
         if (!rows_mode && !digest && lane.kc_h && lane.tail_sums)
-            for (uint32_t m = 1; m <= GFSM_MAXTAIL && plan.dev.tail[m - 1].m; m++) leaves = m;
+            leaves = usable_leaves(data, plan, max_depth_cand, kTile * kItems);
         grid_cap = std::max<uint32_t>(ctx.num_cus, 1) * ctx.tune.wgs_per_cu;
         const uint64_t min_nodes = 8 * kTile;  // a level must hold one launch tile's survivors
         uint64_t row_bytes = 0;
@@ -983,6 +983,7 @@ struct Runner {
                         // is expanded level by level, which stops there.
                         const uint64_t to = c + tiles * tc;
                         untailed = std::min(e, to + tc);
+                        leaves = 0;
                         cand_total -= e - to;
                         e = to;
                     }

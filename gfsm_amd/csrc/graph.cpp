@@ -76,14 +76,29 @@ bool relation_sources(const HostGraph &g, uint32_t rel, uint64_t &sources, uint6
         std::lock_guard<std::mutex> lk(g.stats_mu);
         if (g.rel_entries.size() != g.rel_keys.size()) {
             std::vector<uint64_t> e(g.rel_keys.size(), 0);
-            for (size_t r = 0; r < e.size(); r++)
-                for (uint64_t i = g.rel_off[r]; i < g.rel_off[r + 1]; i++) e[r] += g.rel_cnt[i];
+            std::vector<double> b(g.rel_keys.size(), 0);
+            for (size_t r = 0; r < e.size(); r++) {
+                for (uint64_t i = g.rel_off[r]; i < g.rel_off[r + 1]; i++) {
+                    e[r] += g.rel_cnt[i];
+                    b[r] += (double)g.rel_cnt[i] * g.rel_cnt[i];
+                }
+                b[r] /= (double)std::max<uint64_t>(e[r], 1);
+            }
             g.rel_entries.swap(e);
+            g.rel_biased.swap(b);
         }
         entries = g.rel_entries[k];
     }
     sources = g.rel_off[k + 1] - g.rel_off[k];
     return true;
+}
+
+double relation_biased_mean(const HostGraph &g, uint32_t rel)
+{
+    uint64_t src, ent;
+    if (!relation_sources(g, rel, src, ent)) return 0;
+    std::lock_guard<std::mutex> lk(g.stats_mu);
+    return g.rel_biased[(size_t)g.rel_index(rel)];
 }
 
 uint64_t relation_pool(const HostGraph &g, uint32_t rel)

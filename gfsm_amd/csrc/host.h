@@ -78,6 +78,7 @@ struct HostGraph {
     mutable bool free_pending = false;
     mutable std::mutex stats_mu;
     mutable std::vector<uint64_t> rel_entries;  // per rel_keys index, filled on first use
+    mutable std::vector<double> rel_biased;     // likewise (relation_biased_mean)
     mutable std::vector<uint64_t> label_count;  // vertices per vertex label, filled on first use
 };
 
@@ -88,6 +89,10 @@ uint64_t relation_pool(const HostGraph &g, uint32_t rel);
 // Vertices owning a segment of `rel` and the entries of those segments
 // (false when the graph has no such relation).  Computed once per graph.
 bool relation_sources(const HostGraph &g, uint32_t rel, uint64_t &sources, uint64_t &entries);
+
+// Mean segment length of `rel` over its entries rather than its vertices (sum of
+// squares over sum): what a vertex reached along an edge is likely to have.
+double relation_biased_mean(const HostGraph &g, uint32_t rel);
 
 // Relation of an entry: REF = edge label; VLABEL = (lu << 21) | (lv << 10) | l.
 bool relation_of(uint32_t mode, uint32_t lu, uint32_t lv, uint32_t l, uint32_t &rel);
@@ -113,6 +118,10 @@ void set_injectivity(const HostGraph &data, Plan &plan);
 // Fill the plan's tails (QueryPlanDev::tail) for a data graph; `wide`: leaves
 // with checks and pairs too, where the graph allows them.  After set_injectivity.
 void set_tails(const HostGraph &data, Plan &plan, bool wide);
+// How many leaves to count without placing them: as many as the plan allows, and
+// under a per-depth cap (0: none) only while a few tiles of `tc` candidates are
+// expected to have no more leaf candidates than the cap.
+uint32_t usable_leaves(const HostGraph &data, const Plan &plan, uint64_t max_depth_cand, uint64_t tc);
 // The reference's matching order, or with `by_cost` (a data graph) the
 // order chosen from its relation statistics.
 Status plan_query(const HostGraph &query, Plan &out, const HostGraph *by_cost = nullptr);

@@ -235,8 +235,8 @@ struct BatchSlot {
     uint64_t max_cand;            // work cap (0 = none)
     uint64_t max_depth_cand;      // deterministic per-depth cap (0 = none)
     uint32_t q, digest;
-    uint32_t tail, pad;           // leaves counted without being placed (EXPAND_TAIL); the scheduler takes
-                                  // one off once a cap ends inside a tail step
+    uint32_t tail, pad;           // leaves counted without being placed (EXPAND_TAIL); the scheduler
+                                  // clears it once a cap ends inside a tail step
     uint32_t state;               // SLOT_NEW at admission
     uint32_t error;
     // Depth-first chunk walk, maintained by the scheduler.

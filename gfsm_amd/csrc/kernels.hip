@@ -1828,7 +1828,7 @@ DEV uint32_t schedule_slot(const BatchCfg &cfg, BatchSlot &B, Totals *tot, const
                 // expanded level by level and ends the match.
                 to = b + ts.tiles * TC;
                 B.cand_done -= e - to;
-                B.tail = m - 1;
+                B.tail = 0;
                 B.chunk[d] = TC;
             } else if (B.max_depth_cand) {
                 uint64_t ch = limit;
