@@ -469,6 +469,9 @@ namespace {
 // the power-law hub and middle windows, cap 2^25: 1/8 -> 1/64 cut their time
 // by 30% and 15%; 1/128 gained nothing more).
 constexpr uint64_t kCapStartDiv = 64;
+// ... but no fewer than fill half the GPU's workgroups with a tile each (nine
+// queries on R-MAT 16 under a cap of 2^23, digests: 2.59 -> 2.26 ms).
+constexpr uint64_t kCapStartMin = 1ull << 20;
 
 
 // Steps of at least this many tiles get their frontier nodes from k_tile_index.
@@ -1206,7 +1209,8 @@ Status run_match(Ctx &ctx, const HostGraph &data, const DevGraph &dg, const Plan
     // needs no level buffer, and its ranges are trimmed to the cap exactly.
     if (o.max_depth_cand)
         for (uint32_t k = 0; k + 1 < plan.q; k++)
-            run.chunk[k] = std::max<uint64_t>(2048, std::min<uint64_t>(run.chunk[k], o.max_depth_cand / kCapStartDiv));
+            run.chunk[k] = std::max<uint64_t>(
+                2048, std::min<uint64_t>(run.chunk[k], std::max(kCapStartMin, o.max_depth_cand / kCapStartDiv)));
     uint64_t rlo, rhi;
     root_range(data, plan, o.root_lo, o.root_hi, rlo, rhi);
 
