@@ -261,6 +261,8 @@ Status BatchEngine::init(const BatchShape &shape, uint64_t arena_bytes, char *ar
     cfg_.ctl = ctl_d_;
     cfg_.nslots = n;
     cfg_.items = shape_.items;
+    cfg_.small_items = std::max<uint32_t>(1, shape_.items / 4);
+    cfg_.tile_room = lane_.tail_tiles - n;
     cfg_.pool_words = shape_.pool_words;
     cfg_.max_step_cand = shape_.step_budget;
     cfg_.max_degree = std::max<uint32_t>(data_.max_degree, 1);

@@ -235,8 +235,9 @@ struct BatchSlot {
     uint64_t max_cand;            // work cap (0 = none)
     uint64_t max_depth_cand;      // deterministic per-depth cap (0 = none)
     uint32_t q, digest;
-    uint32_t tail, pad;           // leaves counted without being placed (EXPAND_TAIL); the scheduler
+    uint32_t tail;                // leaves counted without being placed (EXPAND_TAIL); the scheduler
                                   // clears it once a cap ends inside a tail step
+    uint32_t tc;                  // candidates of a tile of the scheduled step
     uint32_t state;               // SLOT_NEW at admission
     uint32_t error;
     // Depth-first chunk walk, maintained by the scheduler.
@@ -266,7 +267,8 @@ struct BatchCtl {
     uint32_t n_admit;             // admission entries waiting (set by the host, cleared by the scheduler)
     uint32_t sched_done;          // scheduler workgroups finished (the last one lays out the tiles
                                   // and resets it)
-    uint32_t pad;
+    uint32_t step_items;          // candidates per thread of the scheduled step (0 before the first)
+    uint32_t next_items, pad;     // ... and of the one after it
 };
 
 // One admission, written by the host into a contiguous queue between
@@ -291,7 +293,11 @@ struct BatchCfg {
     BatchCtl *ctl;
     uint32_t nslots;
     uint32_t items;               // candidates per thread (tile = 256 * items)
+    uint32_t small_items;         // ... of steps that would leave most of the GPU idle (may be items)
     uint32_t pool_words;
+    uint32_t pad;
+    uint64_t tile_room;           // tiles of one step (tail_sums)
+    uint32_t pad2;
     uint32_t fill_tiles;          // tiles that fill the GPU (the step kernel's workgroups)
     uint64_t max_step_cand;       // upper bound of BatchCtl::step_cand (workspace size)
     uint64_t max_degree;          // of the data graph (scan value bound)

@@ -1758,11 +1758,14 @@ DEV TailSums wave_tail_sums(gptr_t<const uint64_t> sums, const BatchSlot &B)
 // re-estimated from the observed selectivity.
 DEV uint32_t schedule_slot(const BatchCfg &cfg, BatchSlot &B, Totals *tot, const TailSums &ts)
 {
-    const uint64_t TC = (uint64_t)kTile * cfg.items;
+    const uint32_t items = cfg.ctl->next_items ? cfg.ctl->next_items : cfg.items;
+    const uint64_t TC = (uint64_t)kTile * items;
     const uint64_t by_val = kValueMask / umax64(cfg.max_degree, 1);
     const uint64_t step = cfg.ctl->step_cand ? umin64(cfg.ctl->step_cand, cfg.max_step_cand) : cfg.max_step_cand;
-    const uint64_t limit = umax64(TC, umin64(step, by_val));
-    const uint64_t floor = cfg.fill_tiles / umax64(cfg.ctl->running, 1) * TC;
+    uint64_t limit = umax64(TC, umin64(step, by_val));
+    if (items < cfg.items)  // all slots' tiles have to fit the tile words
+        limit = umax64(TC, umin64(limit, cfg.tile_room / umax64(cfg.ctl->running + cfg.ctl->n_admit, 1) * TC));
+    const uint64_t floor = cfg.fill_tiles / umax64(cfg.ctl->running, 1) * ((uint64_t)kTile * cfg.items);
     const uint32_t q = B.q;
     uint32_t state = B.state;
     if (state == SLOT_NEW) {
@@ -1826,7 +1829,7 @@ DEV uint32_t schedule_slot(const BatchCfg &cfg, BatchSlot &B, Totals *tot, const
             if (ts.tiles < B.io.ntiles) {
                 // The cap's last candidate falls in the next tile, which is
                 // expanded level by level and ends the match.
-                to = b + ts.tiles * TC;
+                to = b + ts.tiles * B.tc;
                 B.cand_done -= e - to;
                 B.tail = 0;
                 B.chunk[d] = TC;
@@ -1923,6 +1926,7 @@ DEV uint32_t schedule_slot(const BatchCfg &cfg, BatchSlot &B, Totals *tot, const
         io.need_nxt = kind == EXPAND_MID && dp.nxt_dist > 1 ? 1u : 0u;
         io.tot = tot;
         io.ntiles = (e - b + TC - 1) / TC;
+        B.tc = (uint32_t)TC;
         io.d = (uint32_t)d;
         io.q = q;
         io.kind = kind;
@@ -2115,6 +2119,15 @@ __global__ __launch_bounds__(kTile) void k_batch_schedule(BatchCfg cfg)
         tile_start[cfg.nslots] = total;
         gp(cfg.ctl)->total_tiles = total;
         gp(cfg.ctl)->running = running;
+        // The scheduled step's tile size, and the next one's: small tiles while
+        // the large ones would not give an eighth of the workgroups one each (a
+        // lone slot's step 50 -> 33 us; 256-query batch 11.1 -> 10.9 ms, 1,000
+        // served queries 14.6-16.1 -> 14.4 ms; at half the workgroups the batch
+        // loses 1%).
+        const uint32_t items = gp(cfg.ctl)->next_items ? gp(cfg.ctl)->next_items : cfg.items;
+        gp(cfg.ctl)->step_items = items;
+        gp(cfg.ctl)->next_items =
+            (uint64_t)total * items < (uint64_t)cfg.fill_tiles * cfg.items / 8 ? cfg.small_items : cfg.items;
         gp(cfg.ctl)->n_admit = 0;     // every workgroup has read it
         gp(cfg.ctl)->sched_done = 0;  // for the next launch
     }
@@ -2145,7 +2158,7 @@ DEV uint32_t slot_search(const uint64_t *__restrict__ start, uint32_t nslots, ui
 __global__ __launch_bounds__(kTile) void k_batch_tile_index(BatchCfg cfg)
 {
     const uint64_t total = cfg.ctl->total_tiles;
-    const uint64_t TC = (uint64_t)kTile * cfg.items;
+    const uint64_t TC = (uint64_t)kTile * cfg.ctl->step_items;
     const uint32_t lane = lane_id();
     const uint64_t nwaves = ((uint64_t)gridDim.x * kTile) >> 6;
     for (uint64_t t = ((uint64_t)blockIdx.x * kTile + threadIdx.x) >> 6; t < total; t += nwaves) {
@@ -2176,7 +2189,7 @@ __global__ __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(4))) void
     // cost 79 us with all 1,024 in them and the release above; the 256-query
     // batch 16.4 -> 11.9 ms, 1,000 served queries 22.5 -> 17.0 ms by both).
     const uint32_t nwg = total < gridDim.x ? (uint32_t)total : gridDim.x;
-    if (blockIdx.x >= nwg) return;
+    if (blockIdx.x >= nwg || cfg.ctl->step_items != I) return;
     ScanWS ws = cfg.ws;
     ws.brief = total <= gridDim.x;
     const uint32_t ep = read_epoch(ws);
@@ -2686,16 +2699,23 @@ hipError_t launch_batch_tile_index(const BatchCfg &cfg, hipStream_t s)
     return hipGetLastError();
 }
 
-hipError_t launch_batch_step(const BatchCfg &cfg, uint32_t grid, hipStream_t s)
+static hipError_t launch_batch_step_i(const BatchCfg &cfg, uint32_t items, uint32_t grid, hipStream_t s)
 {
-    if (cfg.nslots == 0 || cfg.nslots > kMaxSlots) return hipErrorInvalidValue;
-    switch (cfg.items) {
+    switch (items) {
     case 1: return launch_batch_step_t<1>(cfg, grid, s);
     case 2: return launch_batch_step_t<2>(cfg, grid, s);
     case 4: return launch_batch_step_t<4>(cfg, grid, s);
     case 8: return launch_batch_step_t<8>(cfg, grid, s);
     default: return hipErrorInvalidValue;
     }
+}
+
+hipError_t launch_batch_step(const BatchCfg &cfg, uint32_t grid, hipStream_t s)
+{
+    if (cfg.nslots == 0 || cfg.nslots > kMaxSlots || cfg.small_items > cfg.items) return hipErrorInvalidValue;
+    hipError_t e = launch_batch_step_i(cfg, cfg.items, grid, s);
+    if (e == hipSuccess && cfg.small_items != cfg.items) e = launch_batch_step_i(cfg, cfg.small_items, grid, s);
+    return e;
 }
 
 hipError_t launch_scan_test(const uint32_t *vals, uint64_t n, uint64_t *out, uint32_t *idx, ScanWS ws,
