@@ -53,6 +53,7 @@ struct Lane {
     uint64_t *kc_h = nullptr;
     hipEvent_t ev[2] = {nullptr, nullptr};
     std::vector<hipEvent_t> kev;  // begin/end pairs of timed launches (grown on demand)
+    uint64_t matches = 0;   // matches whose totals were published (kHostFinal)
     uint64_t launches = 0;  // chained-scan launches issued on this lane
     uint64_t *tile_node = nullptr;  // [2*max_tiles] per-tile frontier nodes (single-query lane only)
     uint64_t *tail_sums = nullptr;  // [kTailWords*tail_tiles] sums of a capped tail step's tiles
@@ -92,6 +93,7 @@ struct Ctx {
     int device = 0;
     uint64_t budget = 0;
     uint32_t num_cus = 0;
+    uint32_t clock_khz = 100000;  // of the device clock (wall_clock64)
     uint64_t max_tiles = 0;
     Lane lane;
     Arena arena;

@@ -52,6 +52,7 @@ struct Totals {
     uint64_t count;   // last level, count-only: embeddings
     uint64_t dg0, dg1;// digest sums
     uint64_t tail[2 * GFSM_MAXTAIL + 1]; // tail steps: sums of nodes kept, then {candidates, nodes kept} per leaf
+    uint64_t t0;      // device clock at the match's first root step
 };
 
 enum ExpandKind : uint32_t {
@@ -99,7 +100,8 @@ struct StepIO {
 };
 constexpr uint32_t kTailWords = 8;  // words of a tail tile's sums (2 * GFSM_MAXTAIL + 1 used)
 constexpr uint32_t kTailTiles = 1u << 18;  // tiles of a capped tail step (sums buffer)
-constexpr uint32_t kHostWords = 16;        // host words of a step's totals (Lane::kc_h)
+constexpr uint32_t kHostWords = 32;        // host words of a step's totals and, from kHostFinal on, a
+constexpr uint32_t kHostFinal = 16;        // match's {sequence number, clock ticks, Totals} (Lane::kc_h)
 constexpr uint32_t kNbrPad = 4;     // words allocated past nbr's end (four-word loads of a segment's end)
 constexpr uint32_t kDenseChk = 4;  // checked relations per depth with a dense-table slot (DepthPlanDev)
 
@@ -116,6 +118,7 @@ struct RootIO {
     Totals *tot;
     uint64_t ntiles;
     uint64_t *host_kc;         // as StepIO::host_kc
+    uint32_t first, pad;       // the match's first step: clears the sums in tot and stamps t0
 };
 
 struct ExpandArgs {
@@ -358,6 +361,10 @@ hipError_t launch_sort_rows(const uint32_t *rows, uint64_t n, uint32_t q, uint32
 // words) written to dst[0..n); mode 2: words 0 and 16 of each of those lines
 // (both 64-byte halves) written to dst[0..2n).
 hipError_t launch_calibrate(uint32_t mode, const uint32_t *src, uint32_t *dst, uint64_t n, hipStream_t s);
+
+// The end of a match: its totals and the device clock's ticks since t0 go to
+// host words kc[kHostFinal..], the polled sequence number last.
+hipError_t launch_publish(const Totals *tot, uint64_t *kc, uint64_t seq, hipStream_t s);
 
 // Zero the control block of a workspace (device kernel; safe under capture).
 hipError_t launch_ws_reset(ScanWS ws, Totals *tot, hipStream_t s);

@@ -26,6 +26,7 @@
 // persistent step kernel takes (query, tile) work items by ticket.
 #include <hip/hip_runtime.h>
 
+#include <cstddef>
 #include <mutex>
 #include <type_traits>
 
@@ -520,6 +521,12 @@ template <uint32_t I>
 __global__ __launch_bounds__(kTile) void k_root(RootArgs a)
 {
     __shared__ TileShared<I> sh;
+    // The sums of the match that starts here (keep and cnt are this step's own).
+    if (a.io.first && blockIdx.x == 0) {
+        constexpr uint32_t from = offsetof(Totals, count) / 8, to = offsetof(Totals, t0) / 8;
+        if (threadIdx.x < to - from) reinterpret_cast<uint64_t *>(a.io.tot)[from + threadIdx.x] = 0;
+        if (threadIdx.x == 0) a.io.tot->t0 = wall_clock64();
+    }
     const uint32_t ep = read_epoch(a.ws);
     tickets_init(a.ws, &sh.next);
     for (;;) {
@@ -2336,6 +2343,20 @@ __global__ void k_seg_insert(const uint32_t *dir_ptr, const uint32_t *dir, uint3
     }
 }
 
+__global__ __launch_bounds__(64) void k_publish(const Totals *tot, uint64_t *kc, uint64_t seq)
+{
+    constexpr uint32_t n = sizeof(Totals) / 8;
+    static_assert(kHostFinal + 2 + n <= kHostWords, "host words");
+    const uint64_t *w = reinterpret_cast<const uint64_t *>(tot);
+    const uint64_t v = threadIdx.x < n ? w[threadIdx.x] : 0ull;
+    if (threadIdx.x < n)
+        __hip_atomic_store(kc + kHostFinal + 2 + threadIdx.x, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (threadIdx.x == 0)
+        __hip_atomic_store(kc + kHostFinal + 1, wall_clock64() - tot->t0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __threadfence_system();
+    if (threadIdx.x == 0) __hip_atomic_store(kc + kHostFinal, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 __global__ void k_ws_reset(ScanWS ws, Totals *tot)
 {
     if (threadIdx.x < 4) ws.ctl[threadIdx.x] = 0u;
@@ -2820,6 +2841,12 @@ hipError_t noalloc_scratch(int device, hipStream_t s, char **ptr)
     }
     *ptr = addr[device];
     return hipSuccess;
+}
+
+hipError_t launch_publish(const Totals *tot, uint64_t *kc, uint64_t seq, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_publish, dim3(1), dim3(64), 0, s, tot, kc, seq);
+    return hipGetLastError();
 }
 
 hipError_t launch_ws_reset(ScanWS ws, Totals *tot, hipStream_t s)

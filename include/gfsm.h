@@ -112,7 +112,7 @@ typedef struct gfsm_stats {
     uint64_t alg_bytes;         /* algorithmic HBM bytes: 4 per root candidate; per depth k, */
                                 /* 8 per frontier node, 4 per candidate and per probe, 8 per */
                                 /* kept inner node; rows mode adds 4 q per embedding         */
-    double device_ms;           /* first matcher kernel -> result ready (HIP events)         */
+    double device_ms;           /* first matcher kernel -> totals final (device clock)       */
     double kernel_ms;           /* sum of matcher kernel durations (GFSM_PROFILE only)       */
     double expand_ms;           /* sum of expand-kernel durations (GFSM_PROFILE only)        */
     uint32_t expand_launches;   /* expand-kernel launches timed in expand_ms                 */
