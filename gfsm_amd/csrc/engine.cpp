@@ -120,19 +120,24 @@ void row_free(void *q)
 
 Status Lane::init(uint64_t max_tiles, bool tile_index, uint64_t tail)
 {
-    if (tile_index) HIP_TRY(hipMalloc(&tile_node, 2 * max_tiles * sizeof(uint64_t)));
-    tail_tiles = tail;
-    HIP_TRY(hipMalloc(&tail_sums, kTailWords * tail_tiles * sizeof(uint64_t)));
-    HIP_TRY(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
+    // One allocation: control block, totals, tile words (cleared), tile index,
+    // tail sums.
+    const uint64_t words = max_tiles * sizeof(uint64_t), index = tile_index ? 2 * words : 0;
+    const uint64_t sums = kTailWords * tail * sizeof(uint64_t);
+    static_assert(sizeof(Totals) <= 256, "totals block");
+    char *p = nullptr;
+    HIP_TRY(hipMalloc(reinterpret_cast<void **>(&p), 512 + 2 * words + index + sums));
+    mem = p;
     ws.max_tiles = max_tiles;
-    HIP_TRY(hipMalloc(&ws.wk, max_tiles * sizeof(uint64_t)));
-    HIP_TRY(hipMalloc(&ws.wc, max_tiles * sizeof(uint64_t)));
-    HIP_TRY(hipMalloc(&ws.ctl, 4 * sizeof(uint32_t)));
-    HIP_TRY(hipMemset(ws.wk, 0, max_tiles * sizeof(uint64_t)));
-    HIP_TRY(hipMemset(ws.wc, 0, max_tiles * sizeof(uint64_t)));
-    HIP_TRY(hipMemset(ws.ctl, 0, 4 * sizeof(uint32_t)));
-    HIP_TRY(hipMalloc(&tot_d, sizeof(Totals)));
-    HIP_TRY(hipMemset(tot_d, 0, sizeof(Totals)));
+    ws.ctl = reinterpret_cast<uint32_t *>(p);
+    tot_d = reinterpret_cast<Totals *>(p + 256);
+    ws.wk = reinterpret_cast<uint64_t *>(p + 512);
+    ws.wc = ws.wk + max_tiles;
+    if (tile_index) tile_node = ws.wc + max_tiles;
+    tail_sums = reinterpret_cast<uint64_t *>(p + 512 + 2 * words + index);
+    tail_tiles = tail;
+    HIP_TRY(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
+    HIP_TRY(hipMemset(p, 0, 512 + 2 * words));
     HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&tot_h), sizeof(Totals), hipHostMallocDefault));
     std::memset(tot_h, 0, sizeof(Totals));
     HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&kc_h), kHostWords * sizeof(uint64_t), hipHostMallocCoherent));
@@ -154,13 +159,7 @@ hipError_t Lane::before_launch()
 void Lane::destroy()
 {
     if (stream) (void)hipStreamSynchronize(stream);
-    (void)hipFree(ws.wk);
-    (void)hipFree(ws.wc);
-    (void)hipFree(ws.ctl);
-    (void)hipFree(tile_node);
-    tile_node = nullptr;
-    (void)hipFree(tail_sums);
-    (void)hipFree(tot_d);
+    (void)hipFree(mem);
     if (tot_h) (void)hipHostFree(tot_h);
     if (kc_h) (void)hipHostFree(kc_h);
     kc_h = nullptr;

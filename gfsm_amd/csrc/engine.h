@@ -43,6 +43,7 @@ const uint2 *dense_segments_cached(DevGraph &dg, uint32_t rel);
 // launches at once.
 struct Lane {
     hipStream_t stream = nullptr;
+    void *mem = nullptr;  // the device arrays below, when this lane owns them
     ScanWS ws{};
     Totals *tot_d = nullptr;
     Totals *tot_h = nullptr;  // pinned

@@ -99,7 +99,7 @@ struct StepIO {
                                // EXPAND_TAIL: see ExpandArgs::room)
 };
 constexpr uint32_t kTailWords = 8;  // words of a tail tile's sums (2 * GFSM_MAXTAIL + 1 used)
-constexpr uint32_t kTailTiles = 1u << 18;  // tiles of a capped tail step (sums buffer)
+constexpr uint32_t kTailTiles = 1u << 16;  // tiles of a capped tail step (sums buffer)
 constexpr uint32_t kHostWords = 32;        // host words of a step's totals and, from kHostFinal on, a
 constexpr uint32_t kHostFinal = 16;        // match's {sequence number, clock ticks, Totals} (Lane::kc_h)
 constexpr uint32_t kNbrPad = 4;     // words allocated past nbr's end (four-word loads of a segment's end)
