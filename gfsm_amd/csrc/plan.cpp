@@ -112,6 +112,14 @@ void set_injectivity(const HostGraph &data, Plan &plan)
 // are compared entry by entry on one thread (checks, pairs), 64 x 64 at worst.
 // Past it such a leaf is placed, its candidates spread over the threads.
 static constexpr uint32_t kWideDegree = 64;
+// The relations compared have segments of at most this mean length (over entries),
+// and the step itself checks nothing: behind a check few lanes of a wave hold a
+// survivor, and one's comparing holds up all.  Measured, all depths expanded /
+// compared: checked step: 3 x 3 patch of the 1400 x 1400 grid 10.0 / 11.9 ms, cliques
+// of four at mean degree 30 1.34 / 2.46 ms.  Unchecked, 4-cycles / triangles with a
+// tail-free step: degree 12, 20,000 vertices 0.36 / 0.24 and 0.088 / 0.089 ms; degree 20
+// 1.20 / 0.86 and 0.117 / 0.198 ms; degree 36 6.98 / 5.34 and 0.24 / 0.38 ms.
+static constexpr double kWideMean = 16;
 
 void set_tails(const HostGraph &data, Plan &plan, bool wide)
 {
@@ -119,6 +127,7 @@ void set_tails(const HostGraph &data, Plan &plan, bool wide)
     const bool by_label = data.mode == GFSM_MODE_VLABEL;
     wide = wide && data.max_degree <= kWideDegree && data.V < 0xFFFFFFFEu;
     auto label = [&](uint32_t k) { return by_label ? (plan.dev.depth[k].gen_rel >> 10) & 0x7FFu : 0u; };
+    auto brief = [&](uint32_t rel) { return relation_biased_mean(data, rel) <= kWideMean; };
     uint32_t bits = 1;  // of a segment's length
     while (bits < 32 && (data.max_degree >> bits)) bits++;
     for (uint32_t m = 1; m <= GFSM_MAXTAIL; m++) {
@@ -128,6 +137,7 @@ void set_tails(const HostGraph &data, Plan &plan, bool wide)
         if (q < m + 2 || m * bits + 11 > 62) continue;
         const uint32_t d = q - 1 - m;
         bool ok = true, any_wide = false;
+        const bool compare = wide && plan.dev.depth[d].nchk == 0;
         for (uint32_t i = 0; i < m && ok; i++) {
             const uint32_t k = d + 1 + i;
             const DepthPlanDev &dp = plan.dev.depth[k];
@@ -136,9 +146,9 @@ void set_tails(const HostGraph &data, Plan &plan, bool wide)
             l.rel = dp.gen_rel;
             l.inj = dp.inj & (uint32_t)((1ull << (d + 1)) - 1);
             l.nchk = dp.nchk;
-            ok = l.col <= d && (dp.nchk == 0 || (wide && dp.nchk <= GFSM_TAILCHK));
+            ok = l.col <= d && (dp.nchk == 0 || (compare && dp.nchk <= GFSM_TAILCHK && brief(dp.gen_rel)));
             for (uint32_t r = 0; r < dp.nchk && ok; r++) {
-                ok = dp.chk_dist[r] && k - dp.chk_dist[r] <= d;
+                ok = dp.chk_dist[r] && k - dp.chk_dist[r] <= d && brief(dp.chk_rel[r]);
                 l.chk_col[r] = k - dp.chk_dist[r];
                 l.chk_rel[r] = dp.chk_rel[r];
             }
@@ -153,7 +163,8 @@ void set_tails(const HostGraph &data, Plan &plan, bool wide)
             }
             if (same == twin)
                 l.twins = twin;
-            else if (wide && same == 1 && label(k - 1) == label(k) && !tp.leaf[i - 1].pair)
+            else if (compare && same == 1 && label(k - 1) == label(k) && !tp.leaf[i - 1].pair && brief(l.rel) &&
+                     brief(tp.leaf[i - 1].rel))
                 l.pair = 1;
             else
                 ok = false;
@@ -176,7 +187,8 @@ static constexpr double kCapTiles = 4;
 uint32_t usable_leaves(const HostGraph &data, const Plan &plan, uint64_t max_depth_cand, uint64_t tc)
 {
     uint32_t best = 0;
-    for (uint32_t m = 1; m <= GFSM_MAXTAIL && plan.dev.tail[m - 1].m; m++) {
+    for (uint32_t m = 1; m <= GFSM_MAXTAIL; m++) {
+        if (!plan.dev.tail[m - 1].m) continue;
         if (max_depth_cand) {
             double per = kCapTiles * (double)tc;
             for (uint32_t i = 0; i < m; i++) per *= std::max(1.0, relation_biased_mean(data, plan.dev.tail[m - 1].leaf[i].rel));

@@ -93,3 +93,21 @@ def test_many_tiles_under_a_cap(ctx):
         a = ctx.match(data, q, max_depth_cand=cap, allow_partial=True, digest=True)
         b = ctx.match(data, q, max_depth_cand=cap, allow_partial=True)
         assert (a.count, a.status) == (b.count, b.status), cap
+
+
+@pytest.mark.parametrize("degree", [10, 14, 18])
+def test_checked_leaves_by_mean_length(ctx, degree):
+    """Around the mean segment length up to which checked leaves are compared, and
+    where only a larger or a smaller number of leaves qualifies."""
+    data = G.Graph.er(300, degree, seed=degree)
+    ctx.upload(data)
+    shapes = [
+        [(0, 1), (1, 2), (2, 0)], [(0, 1), (0, 2), (0, 3), (1, 2), (1, 3), (2, 3)],  # triangle, clique
+        [(0, 1), (1, 2), (2, 0), (0, 3), (1, 4)],  # a pair behind a check
+        [(0, 1), (1, 2), (2, 3), (3, 0)], [(0, 1), (1, 2), (3, 4), (4, 5), (0, 3), (1, 4), (2, 5)],
+    ]
+    for edges in shapes:
+        q = _query(edges, [1] * (max(map(max, edges)) + 1), G.MODE_REF)
+        full, m = ctx.match(data, q, digest=True), ctx.match(data, q)
+        assert m.count == full.count == oracle_solve(data, q, G.MODE_REF, rows=False).count, edges
+        assert m.stats["level"] == full.stats["level"] and m.stats["cand"] == full.stats["cand"], edges
