@@ -473,7 +473,8 @@ def main():
             "unit": "GB/s",
             "frac": achieved / HBM_PEAK_GBS,
             "traffic": None,
-            "kernel": "gfsm::k_expand (inner depths) + gfsm::k_expand_bare (last depth)",
+            "kernel": "gfsm::k_expand (inner depths) + gfsm::k_expand_tail (counted leaves) + "
+                      "gfsm::k_expand_bare (last depth)",
             "launches": launches // K,
             "mean_launch_ms": mean_ms,
         },
