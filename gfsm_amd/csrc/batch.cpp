@@ -4,9 +4,10 @@
 //
 // Every query admitted to the engine owns a slot (its plan, its level
 // buffers and its depth-first chunk walk, all in device memory).  One step is
-// a scheduler launch (one workgroup: consume each slot's finished step,
-// choose its next one, lay all slots' tiles end to end) followed by one
-// persistent step launch that hands out (slot, tile) work items by ticket.
+// a scheduler launch (one wave per slot: consume each slot's finished step,
+// choose its next one, lay all slots' tiles end to end) followed by a
+// persistent step launch in each of two tile sizes, the one the scheduler chose
+// handing out (slot, tile) work items by ticket, the other returning at once.
 // Steps need no host round trip, so K of them are captured once in a hipGraph
 // and replayed; between replays the host harvests finished slots and admits
 // waiting queries into them.  The arena is shared by the slots' regions,

@@ -308,7 +308,7 @@ struct BatchCfg {
     ScanWS ws;
 };
 
-// One batch step: the scheduler (one workgroup) consumes every slot's last
+// One batch step: the scheduler (one wave per slot) consumes every slot's last
 // step, schedules its next one and lays out the tiles; the step kernel
 // (`grid` persistent workgroups) runs them.  Both read only `cfg` and device
 // memory, so the pair can be captured and replayed.
