@@ -36,6 +36,7 @@ ORDER_COST = 16  # matching order from the data graph's relation statistics
 WALK_DENSE = 0
 WALK_SPARSE = 1
 ERR_PENDING = 6
+ERR_OVERFLOW = 7  # 2^64 embeddings or more
 MAX_Q = 32
 NOALLOC_SCRATCH_BYTES = 64 << 20  # GFSM_NOALLOC_SCRATCH_BYTES
 NOALLOC_LEVEL_BYTES = 60 << 20    # its level part (the rest holds the scan workspace)
@@ -501,7 +502,8 @@ class Context:
         """Batched matching: every query of the list in flight together.
         windows: optional per-query (root_lo, root_hi); caps / depth_caps:
         optional per-query max_cand / max_depth_cand.  Returns one Match per query;
-        check each Match's status (5 = capped, partial count)."""
+        check each Match's status (5 = capped, partial count; 7 = 2^64 embeddings or
+        more, no count)."""
         n = len(queries)
         if windows is None and caps is None and depth_caps is None:
             os_ = (MatchOpts * 1)(_opts(**kw))

@@ -472,7 +472,7 @@ Status BatchEngine::harvest(const std::function<void(std::unique_ptr<BatchJob>, 
     for (uint32_t s = 0; s < shape_.slots; s++) {
         if (!jobs_[s]) continue;
         const uint32_t st = report_h_[s].state;
-        if (st == SLOT_DONE || st == SLOT_CAP || st == SLOT_ERROR) fin.push_back(s);
+        if (st == SLOT_DONE || st == SLOT_CAP || st == SLOT_ERROR || st == SLOT_OVER) fin.push_back(s);
     }
     if (fin.empty()) return Status::ok();
     const double t = now_ms();
@@ -499,6 +499,10 @@ Status BatchEngine::harvest(const std::function<void(std::unique_ptr<BatchJob>, 
         r.stats.device_ms = t - job->t_admit;
         if (b.state == SLOT_CAP) r.status = GFSM_ERR_CAP;
         if (b.state == SLOT_ERROR) r.status = GFSM_ERR_ARG;
+        if (b.state == SLOT_OVER) {
+            r.status = GFSM_ERR_OVERFLOW;
+            r.count = 0;
+        }
         regions_.give(job->region_off, job->region_bytes);
         running_--;
         calibrate(job->model_bytes, r, q);

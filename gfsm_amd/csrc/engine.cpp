@@ -453,14 +453,14 @@ void root_range(const HostGraph &data, const Plan &plan, uint32_t root_lo, uint3
 uint64_t alg_bytes(const Plan &plan, const gfsm_stats &st, uint32_t flags)
 {
     const uint32_t q = plan.q;
-    uint64_t b = 4ull * st.roots;
+    unsigned __int128 b = 4ull * st.roots;  // 32 depths of at most 2^64 x 2^37
     for (uint32_t k = 1; k < q; k++) {
-        b += 8ull * st.level[k - 1];
-        b += 4ull * st.cand[k] * (1ull + plan.dev.depth[k].nchk);
-        if (k + 1 < q) b += 8ull * st.level[k];
+        b += (unsigned __int128)8 * st.level[k - 1];
+        b += (unsigned __int128)4 * st.cand[k] * (1ull + plan.dev.depth[k].nchk);
+        if (k + 1 < q) b += (unsigned __int128)8 * st.level[k];
     }
     if (flags & (GFSM_ROWS | GFSM_SORTED)) b += 4ull * q * st.level[q - 1];
-    return b;
+    return b >> 64 ? ~0ull : (uint64_t)b;
 }
 
 namespace {
@@ -583,6 +583,20 @@ struct Runner {
         const uint64_t by_ws = lane.ws.max_tiles * kTile;  // enough tiles at any tile size
         const uint64_t by_val = kValueMask / std::max<uint64_t>(1, data.max_degree);
         return std::max<uint64_t>(kTile * 8, std::min(by_ws, by_val));
+    }
+
+    // Tiles of an uncapped tail step of m leaves: few enough for every workgroup to
+    // add its tiles' sums in 64 bits.  A tile of tc candidates has at most tc *
+    // degree^m completions, under 2^62 (set_tails); of n tiles dealt by XCD (kernels.hip,
+    // TileDeal) a workgroup takes at most (n + 128) / grid + 1, and one where every
+    // tile has a workgroup.
+    uint64_t tail_step_tiles(uint64_t tc, uint32_t m) const
+    {
+        uint64_t most = tc;
+        for (uint32_t i = 0; i < m; i++) most *= std::max<uint64_t>(data.max_degree, 1);
+        const uint64_t tiles = std::min<uint64_t>(~0ull / most, 1u << 30);  // at least 3
+        const uint64_t grid = grid_cap >= 8 ? grid_cap & ~7u : grid_cap;
+        return std::max<uint64_t>(grid_cap, std::max<uint64_t>((tiles - 1) * grid, 128) - 128);
     }
 
     uint32_t grid_for(uint64_t ntiles) const
@@ -916,7 +930,7 @@ struct Runner {
                 if (depth_done[d] >= max_depth_cand) return Status::err(GFSM_ERR_CAP, "per-depth candidate cap reached");
                 e = std::min(e, c + (max_depth_cand - depth_done[d]));
             }
-            if (kind == EXPAND_TAIL && capped) e = std::min(e, c + lane.tail_tiles * tc);
+            if (kind == EXPAND_TAIL) e = std::min(e, c + (capped ? lane.tail_tiles : tail_step_tiles(tc, m)) * tc);
             if (at_tail && kind == EXPAND_MID)  // writes the level, up to the range's end
                 e = std::min(e, std::min(untailed, c + std::max<uint64_t>(tc, cap[d])));
             ExpandArgs a{};
@@ -1309,11 +1323,16 @@ Status run_match(Ctx &ctx, const HostGraph &data, const DevGraph &dg, const Plan
     } else {
         res.count = L.tot_h->count + run.tail_count;
         if (run.leaves && !o.max_depth_cand && !o.max_cand) {
+            // Counted leaves reach numbers that no enumeration would: a count past
+            // 2^64 - 1 is an error, a statistic stays at the largest number.
             const uint32_t m = run.leaves, d = q - 1 - m;
-            res.stats.level[d] = L.tot_h->tail[0];
+            const auto sum = [&](uint32_t i) { return (L.tot_h->tail_over >> i) & 1 ? ~0ull : L.tot_h->tail[i]; };
+            if ((L.tot_h->tail_over >> (2 * m)) & 1)
+                return Status::err(GFSM_ERR_OVERFLOW, "the query has 2^64 embeddings or more");
+            res.stats.level[d] = sum(0);
             for (uint32_t i = 0; i < m; i++) {
-                res.stats.cand[d + 1 + i] = L.tot_h->tail[1 + 2 * i];
-                res.stats.level[d + 1 + i] = L.tot_h->tail[2 + 2 * i];
+                res.stats.cand[d + 1 + i] = sum(1 + 2 * i);
+                res.stats.level[d + 1 + i] = sum(2 + 2 * i);
             }
             res.count = L.tot_h->tail[2 * m];
         }

@@ -52,6 +52,7 @@ struct Totals {
     uint64_t count;   // last level, count-only: embeddings
     uint64_t dg0, dg1;// digest sums
     uint64_t tail[2 * GFSM_MAXTAIL + 1]; // tail steps: sums of nodes kept, then {candidates, nodes kept} per leaf
+    uint64_t tail_over; // bit i: tail[i] passed 2^64
     uint64_t t0;      // device clock at the match's first root step
 };
 
@@ -206,6 +207,7 @@ enum SlotState : uint32_t {
     SLOT_DONE = 3,      // finished: count and digest are final
     SLOT_CAP = 4,       // the work cap was reached: partial count
     SLOT_ERROR = 5,     // a step shape check failed (see error)
+    SLOT_OVER = 6,      // the count passed 2^64 - 1
 };
 constexpr uint32_t STEP_NONE = 7;
 constexpr uint32_t STEP_ROOT = 8;

@@ -1552,9 +1552,16 @@ __global__ __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(4))) void
         if (capped) tail_tile_end(a.tail_sums, t, sh.tsum);
     }
     __syncthreads();
-    if (!capped && threadIdx.x < 2 * a.tail.m + 1)
-        __hip_atomic_fetch_add(&gp(a.io.tot)->tail[threadIdx.x], sh.tsum[threadIdx.x], __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
+    // A workgroup's own sums fit 64 bits (the launch has few enough tiles); a total
+    // that carries past them is marked.
+    if (!capped && threadIdx.x < 2 * a.tail.m + 1) {
+        const uint64_t x = sh.tsum[threadIdx.x];
+        const uint64_t old = __hip_atomic_fetch_add(&gp(a.io.tot)->tail[threadIdx.x], x, __ATOMIC_RELAXED,
+                                                    __HIP_MEMORY_SCOPE_AGENT);
+        if (old + x < old)
+            __hip_atomic_fetch_or(&gp(a.io.tot)->tail_over, 1ull << threadIdx.x, __ATOMIC_RELAXED,
+                                  __HIP_MEMORY_SCOPE_AGENT);
+    }
     finish_launch(a.ws);
 }
 
@@ -1643,7 +1650,7 @@ __global__ __launch_bounds__(kCutThreads) void k_tail_cut(const uint64_t *tile_s
                 fit = fit && p <= room.leaf[i];
                 all = add_sat(all, p);
             }
-            fit = fit && all <= room.all;
+            fit = fit && all <= room.all && all != ~0ull;  // (a saturated sum fits no room)
             // prefixes only grow: the tiles that fit are the first ones
             const uint64_t mask = __ballot(fit);
             __syncthreads();
@@ -1722,7 +1729,18 @@ DEV uint64_t capped_chunk(const BatchSlot &B, uint32_t d, uint64_t n, uint64_t c
 // candidates fit the caps, and how many tiles those are.
 struct TailSums {
     uint64_t sum[2 * GFSM_MAXTAIL + 1], tiles;
+    uint32_t over;  // bit i: sum[i] passed 2^64
 };
+
+// The sum of v (at most 2^62) over a wave; *over: it passed 2^64.
+DEV uint64_t wave_sum_over(uint64_t v, bool *over)
+{
+    *over = false;
+    if (!__any((v >> 57) != 0)) return wave_sum64(v);
+    const uint64_t lo = wave_sum64(v & 0xFFFFFFFFull), hi = wave_sum64(v >> 32) + (lo >> 32);
+    *over = hi >> 32;
+    return hi << 32 | (lo & 0xFFFFFFFFull);
+}
 
 // The sums of the tail step of slot B, by all 64 lanes of one wave.
 DEV TailSums wave_tail_sums(gptr_t<const uint64_t> sums, const BatchSlot &B)
@@ -1746,10 +1764,16 @@ DEV TailSums wave_tail_sums(gptr_t<const uint64_t> sums, const BatchSlot &B)
             all = add_sat(all, inc);
         }
         if (B.max_cand) fit = fit && all <= B.max_cand - umin64(B.max_cand, B.cand_done);
+        if (B.max_depth_cand || B.max_cand) fit = fit && all != ~0ull;  // (a saturated sum fits no cap)
         const uint64_t mask = __ballot(fit);
 #pragma unroll
         for (uint32_t i = 0; i < 2 * GFSM_MAXTAIL + 1; i++)
-            if (i < 2 * m + 1) r.sum[i] += wave_sum64(fit ? sums[kTailWords * t + i] : 0ull);
+            if (i < 2 * m + 1) {
+                bool over;
+                const uint64_t v = wave_sum_over(fit ? sums[kTailWords * t + i] : 0ull, &over);
+                r.sum[i] += v;
+                r.over |= (over || r.sum[i] < v) ? 1u << i : 0u;
+            }
         r.tiles += (uint64_t)__popcll(mask);
         if (mask != ~0ull) break;  // the tiles that fit are the first ones
     }
@@ -1854,12 +1878,20 @@ DEV uint32_t schedule_slot(const BatchCfg &cfg, BatchSlot &B, Totals *tot, const
             B.lo[d] = to;
             B.cand[d] += to - b;
             B.level[d] += ts.sum[0];
+            // Statistics past 2^64 stay at the largest number; a count there ends
+            // the match.
+            const auto sum = [&](uint32_t i) { return (ts.over >> i) & 1u ? ~0ull : ts.sum[i]; };
             for (uint32_t i = 0; i < m; i++) {
-                B.cand[d + 1 + i] += ts.sum[1 + 2 * i];
-                B.level[d + 1 + i] += ts.sum[2 + 2 * i];
-                B.cand_done += ts.sum[1 + 2 * i];
+                B.cand[d + 1 + i] = add_sat(B.cand[d + 1 + i], sum(1 + 2 * i));
+                B.level[d + 1 + i] = add_sat(B.level[d + 1 + i], sum(2 + 2 * i));
+                B.cand_done = add_sat(B.cand_done, sum(1 + 2 * i));
             }
             B.count += ts.sum[2 * m];
+            if (((ts.over >> (2 * m)) & 1u) || B.count < ts.sum[2 * m]) {
+                B.state = SLOT_OVER;
+                B.step = STEP_NONE;
+                return 0;
+            }
         } else if (B.step == EXPAND_LAST_COUNT) {
             B.steps++;
             B.lo[d] = e;

@@ -60,6 +60,7 @@ typedef int32_t gfsm_status;
 #define GFSM_ERR_DEVICE 4         /* HIP runtime error                                       */
 #define GFSM_ERR_CAP 5            /* a cap was reached (max_rows, max_cand, max_depth_cand)  */
 #define GFSM_ERR_PENDING 6        /* server: result not ready yet                            */
+#define GFSM_ERR_OVERFLOW 7       /* a match with 2^64 embeddings or more: no count          */
 #define GFSM_ERR_MISSING_FILE 232 /* HnHelper.cuh:16 */
 #define GFSM_ERR_INVALID_DATA 233 /* HnHelper.cuh:17 */
 #define GFSM_ERR_MISSING_DATA 234 /* HnHelper.cuh:18 */
@@ -106,7 +107,8 @@ typedef struct gfsm_stats {
     uint32_t chunks;            /* expand launches beyond one per depth (chunked expansion)  */
     uint32_t overflows;         /* launches discarded because a level overflowed its buffer  */
     uint64_t roots;             /* root candidates read                                      */
-    uint64_t level[GFSM_MAX_Q]; /* nodes kept per depth (last depth: embeddings)             */
+    uint64_t level[GFSM_MAX_Q]; /* nodes kept per depth (last depth: embeddings); 2^64 - 1:  */
+                                /* that many or more (as in cand and alg_bytes)              */
     uint64_t cand[GFSM_MAX_Q];  /* candidates tested per depth (depth 0: root candidates)     */
     uint32_t checks[GFSM_MAX_Q];/* membership probes per candidate at each depth             */
     uint64_t alg_bytes;         /* algorithmic HBM bytes: 4 per root candidate; per depth k, */

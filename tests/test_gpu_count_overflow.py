@@ -74,8 +74,9 @@ def test_capped_counts_stay_exact(ctx):
     assert ctx.match(data, q, max_depth_cand=1 << 30, allow_partial=True).status == 5
 
 
-def test_several_tiles_of_a_workgroup():
-    """Sums past 2^62 in a workgroup's own words, over seven tiles each."""
+def test_tiles_of_almost_2_to_62():
+    """More tiles than workgroups, each near the most that a tile may count: launches
+    of few enough for a workgroup's own sum."""
     with G.Context(0) as ctx:
         ctx.set_tuning(wgs_per_cu=1)
         data = _biclique(25, 130000)
