@@ -394,7 +394,8 @@ class Match:
         self.width = w.value
         self.rows = None
         if nr.value:
-            # the result's own memory, no copy: the array keeps the result alive
+            # the result's own memory, no copy: the array keeps the result alive, and
+            # write_fs writes what it holds
             buf = (C.c_uint32 * (nr.value * w.value)).from_address(C.addressof(p.contents))
             buf._own = self._own
             self.rows = np.frombuffer(buf, dtype=np.uint32).reshape(nr.value, w.value)

@@ -553,7 +553,8 @@ Status match_batch_shaped(Ctx &ctx, const HostGraph &data, const std::vector<con
                           double *device_ms)
 {
     const size_t n = queries.size();
-    out.assign(n, Result{});
+    out.clear();
+    out.resize(n);
     if (opts.size() != 1 && opts.size() != n) return Status::err(GFSM_ERR_ARG, "opts must have 1 or n entries");
     auto opt = [&](size_t i) -> const gfsm_match_opts & { return opts.size() == 1 ? opts[0] : opts[i]; };
     std::deque<std::unique_ptr<BatchJob>> pending;

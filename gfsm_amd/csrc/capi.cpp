@@ -350,7 +350,7 @@ gfsm_status gfsm_match_write_fs(gfsm_ctx *ctx, const gfsm_graph *data, const gfs
     const bool partial = st.code == GFSM_ERR_CAP && res->r.status == GFSM_ERR_CAP;
     if (!st.good() && !partial) return fail(st);
     Result &m = res->r;
-    const RowVec &rows = m.rows;  // one-vertex queries and sorted rows
+    const RowBuf &rows = m.rows;  // one-vertex queries and sorted rows
     if (!rows.empty() && std::fwrite(rows.data(), sizeof(uint32_t), rows.size(), f.get()) != rows.size())
         return fail(Status::err(GFSM_ERR_MISSING_FILE, "short write to output.fs"));
     if (m.count > 0xFFFFFFFFull) return fail(Status::err(GFSM_ERR_CAP, "output.fs holds at most 2^32-1 rows"));
@@ -359,7 +359,7 @@ gfsm_status gfsm_match_write_fs(gfsm_ctx *ctx, const gfsm_graph *data, const gfs
     if (std::fseek(f.get(), 0, SEEK_SET) != 0 || std::fwrite(hdr, sizeof(uint32_t), 2, f.get()) != 2 ||
         std::fflush(f.get()) != 0)
         return fail(Status::err(GFSM_ERR_MISSING_FILE, "short write to output.fs"));
-    RowVec().swap(m.rows);  // the rows live in the file
+    m.rows.clear();  // the rows live in the file
     *r = res.release();
     return partial ? fail(st) : ok();
     GUARD_END

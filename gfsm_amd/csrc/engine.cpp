@@ -20,6 +20,7 @@
 #include <cstring>
 #include <functional>
 #include <new>
+#include <thread>
 
 namespace gfsm {
 
@@ -37,85 +38,112 @@ static double now_ms()
         if (e_ != hipSuccess) return hip_status(e_, #expr);              \
     } while (0)
 
-// Pinned blocks that results gave back, kept for the next ones (any thread, any
-// context): at most kPoolBlocks of them and kPoolBytes in all.  Measured, a call
-// returning 1,920,000 rows of seven: pageable rows, filled with zeros, copied into
-// and copied once more for the caller, 6-17 ms; straight into pinned memory that the
-// caller views, 1.25 ms.  With an allocation per call instead of the pool a call
-// with 12,288 rows took 0.29 ms, with it 0.24.
-namespace {
-struct RowHead {  // precedes the memory handed out
-    uint64_t bytes;  // handed out at most
-    uint64_t pinned;
-    uint64_t pad[6];
-};
-constexpr size_t kRowPinMin = 64u << 10, kRowPinMax = 1u << 30;  // past it pageable: pinned memory is the machine's
-constexpr size_t kPoolBlocks = 16, kPoolBytes = 512u << 20;
-struct RowPool {
-    std::mutex mu;
-    std::vector<RowHead *> free;
-    size_t bytes = 0;
-};
-RowPool &row_pool()
+Status CopyRing::init(size_t bytes)
 {
-    static RowPool *p = new RowPool;  // never destroyed: results may be freed at exit
-    return *p;
-}
-}  // namespace
-
-void *row_alloc(size_t bytes)
-{
-    if (bytes >= kRowPinMin && bytes <= kRowPinMax) {
-        RowPool &pool = row_pool();
-        {
-            std::lock_guard<std::mutex> lk(pool.mu);
-            size_t best = pool.free.size();
-            for (size_t i = 0; i < pool.free.size(); i++) {
-                const uint64_t b = pool.free[i]->bytes;
-                if (b >= bytes && b / 4 <= bytes && (best == pool.free.size() || b < pool.free[best]->bytes)) best = i;
-            }
-            if (best < pool.free.size()) {
-                RowHead *h = pool.free[best];
-                pool.free.erase(pool.free.begin() + best);
-                pool.bytes -= h->bytes;
-                return h + 1;
-            }
-        }
-        const size_t grain = bytes < (2u << 20) ? kRowPinMin : (2u << 20);  // near sizes share blocks
-        const size_t room = (bytes + grain - 1) / grain * grain;
-        void *p = nullptr;
-        if (hipHostMalloc(&p, room + sizeof(RowHead), hipHostMallocPortable) == hipSuccess) {
-            RowHead *h = static_cast<RowHead *>(p);
-            h->bytes = room;
-            h->pinned = 1;
-            return h + 1;
-        }
-        (void)hipGetLastError();
-    }
-    RowHead *h = static_cast<RowHead *>(std::malloc(bytes + sizeof(RowHead)));
-    if (!h) throw std::bad_alloc();
-    h->bytes = bytes;
-    h->pinned = 0;
-    return h + 1;
+    if (bytes <= size) return Status::ok();
+    destroy();
+    HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&mem), bytes, hipHostMallocDefault));
+    size = bytes;
+    HIP_TRY(hipStreamCreateWithFlags(&second, hipStreamNonBlocking));
+    for (auto &e : ev) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    return Status::ok();
 }
 
-void row_free(void *q)
+void CopyRing::destroy()
 {
-    RowHead *h = static_cast<RowHead *>(q) - 1;
-    if (!h->pinned) {
-        std::free(h);
-        return;
+    if (mem) (void)hipHostFree(mem);
+    if (second) (void)hipStreamDestroy(second);
+    for (auto &e : ev) {
+        if (e) (void)hipEventDestroy(e);
+        e = nullptr;
     }
-    RowPool &pool = row_pool();
-    {
-        std::lock_guard<std::mutex> lk(pool.mu);
-        if (pool.free.size() < kPoolBlocks && pool.bytes + h->bytes <= kPoolBytes) {
-            pool.free.push_back(h);
-            pool.bytes += h->bytes;
-            return;
+    mem = nullptr;
+    second = nullptr;
+    size = 0;
+}
+
+Status CopyRing::to_host(hipStream_t s, void *dst, const void *src, size_t n)
+{
+    if (!n) {
+        HIP_TRY(hipStreamSynchronize(s));
+        return Status::ok();
+    }
+    Status st = init(n <= kSmall ? kSmall : kSlots * kPiece);
+    if (!st.good()) return st;
+    char *const to = static_cast<char *>(dst);
+    const char *const from = static_cast<const char *>(src);
+    if (n <= kPiece) {
+        HIP_TRY(launch_copy_out(reinterpret_cast<const uint32_t *>(from), reinterpret_cast<uint32_t *>(mem), n / 4, s));
+        HIP_TRY(hipStreamSynchronize(s));
+        std::memcpy(to, mem, n);
+        return Status::ok();
+    }
+    HIP_TRY(hipStreamSynchronize(s));  // the copies run on two streams
+    // Pieces end at multiples of their size in the table's memory, give or take the
+    // 16 bytes that the source is read by: two threads' pieces share no huge page.
+    size_t head = (kPiece - reinterpret_cast<uintptr_t>(to) % kPiece) & ~(size_t)15;
+    if (!head) head = kPiece;
+    std::vector<size_t> at{0};
+    for (size_t e = head; e < n; e += kPiece) at.push_back(e);
+    // The last one in quarters: nothing overlaps its way out of the ring.
+    for (size_t e = at.back() + kPiece / 4; e < n; e += kPiece / 4) at.push_back(e);
+    at.push_back(n);
+    const size_t np = at.size() - 1;
+    std::atomic<size_t> ready{0}, next{0}, freed[kSlots];  // pieces landed; taken; per slot, past its last piece done
+    std::atomic<bool> stop{false};
+    for (auto &f : freed) f.store(0, std::memory_order_relaxed);
+    const auto out = [&](size_t k) {
+        std::memcpy(to + at[k], mem + k % kSlots * kPiece, at[k + 1] - at[k]);
+        freed[k % kSlots].store(k + 1, std::memory_order_release);
+    };
+    const auto work = [&] {
+        for (size_t k; (k = next.fetch_add(1, std::memory_order_relaxed)) < np;) {
+            for (uint32_t i = 1; ready.load(std::memory_order_acquire) <= k; i++) {
+                if (stop.load(std::memory_order_relaxed)) return;
+                __builtin_ia32_pause();
+                if ((i & 1023) == 0) std::this_thread::yield();
+            }
+            out(k);
+        }
+    };
+    size_t issued = 0;
+    const auto slot_free = [&](size_t k) {
+        return k < kSlots || freed[k % kSlots].load(std::memory_order_acquire) == k - kSlots + 1;
+    };
+    const auto issue = [&]() -> hipError_t {
+        const size_t k = issued++, sl = k % kSlots;
+        const hipStream_t q = k & 1 ? second : s;
+        const hipError_t e = launch_copy_out(reinterpret_cast<const uint32_t *>(from + at[k]),
+                                             reinterpret_cast<uint32_t *>(mem + sl * kPiece), (at[k + 1] - at[k]) / 4, q);
+        return e == hipSuccess ? hipEventRecord(ev[sl], q) : e;
+    };
+    hipError_t err = hipSuccess;
+    while (err == hipSuccess && issued < np && issued < kSlots) err = issue();
+    std::vector<std::thread> th;
+    try {
+        th.reserve(kThreads);
+        while (th.size() < std::min<size_t>(kThreads, np)) th.emplace_back(work);
+    } catch (const std::exception &) {  // no more threads: those there are, or this one
+    }
+    for (size_t k = 0; k < np && err == hipSuccess; k++) {
+        err = hipEventSynchronize(ev[k % kSlots]);
+        if (err != hipSuccess) break;
+        ready.store(k + 1, std::memory_order_release);
+        if (th.empty()) out(k);
+        while (err == hipSuccess && issued < np && issued <= k + kSlots) {
+            if (slot_free(issued)) err = issue();
+            else if (issued > k + 1) break;  // others are on their way
+            else __builtin_ia32_pause();
         }
     }
-    (void)hipHostFree(h);
+    if (err != hipSuccess) stop = true;
+    for (auto &t : th) t.join();
+    if (err != hipSuccess) {
+        (void)hipStreamSynchronize(s);
+        (void)hipStreamSynchronize(second);
+        return hip_status(err, "copy of the rows");
+    }
+    return Status::ok();
 }
 
 Status Lane::init(uint64_t max_tiles, bool tile_index, uint64_t tail)
@@ -206,6 +234,7 @@ Status ctx_open(int device, uint64_t budget, Ctx *&out)
         c->lane.destroy();
         return hip_status(se, "device scratch of the allocation-free match");
     }
+    row_pool_open();
     out = c.release();
     return Status::ok();
 }
@@ -249,6 +278,8 @@ void ctx_close(Ctx *ctx)
         ctx->graphs.clear();
     }
     ctx->lane.destroy();
+    ctx->ring.destroy();
+    row_pool_close();
     if (ctx->arena.base) (void)hipFree(ctx->arena.base);
     if (ctx->batch_arena.base) (void)hipFree(ctx->batch_arena.base);
     delete ctx;
@@ -527,7 +558,7 @@ struct Runner {
     // host memory stays one chunk, whatever the result size.
     FILE *stream = nullptr;
     uint64_t streamed = 0, sdg[2] = {0, 0};
-    RowVec stage;
+    RowBuf stage;
 
     // The lane (stream, scan workspace, totals); optionally a fixed level
     // arena, with which nothing is allocated (dense tables only if cached).
@@ -852,8 +883,7 @@ struct Runner {
     {
         const size_t at = res.rows.size();
         res.rows.resize(at + n * q);
-        if (n) HIP_TRY(hipMemcpy(res.rows.data() + at, from, n * q * sizeof(uint32_t), hipMemcpyDeviceToHost));
-        return Status::ok();
+        return ctx.ring.to_host(lane.stream, res.rows.data() + at, from, n * q * sizeof(uint32_t));
     }
     Status copy_kept()
     {
@@ -882,7 +912,6 @@ struct Runner {
         if (ncol && rows_kept && sort_rows_bytes(rows_kept, q) <= level_bytes) {
             uint32_t *sorted = nullptr;
             HIP_TRY(launch_sort_rows(rows_d, rows_kept, q, ncol, bits, level_base, &sorted, lane.stream));
-            HIP_TRY(hipStreamSynchronize(lane.stream));
             const uint64_t n = rows_kept;
             rows_kept = 0;
             return copy_rows(sorted, n);
@@ -1102,9 +1131,10 @@ struct Runner {
                 if (max_rows && res.rows.size() / q + streamed + keep > max_rows)
                     return Status::err(GFSM_ERR_CAP, "more rows than max_rows");
                 if (stream) {
+                    if (keep * q > stage.capacity()) stage.clear();
                     stage.resize(keep * q);
-                    if (keep)
-                        HIP_TRY(hipMemcpy(stage.data(), rows_d, keep * q * sizeof(uint32_t), hipMemcpyDeviceToHost));
+                    st = ctx.ring.to_host(lane.stream, stage.data(), rows_d, keep * q * sizeof(uint32_t));
+                    if (!st.good()) return st;
                     if (flags & GFSM_DIGEST)
                         for (uint64_t r = 0; r < keep; r++) {
                             uint64_t h[2];
@@ -1224,12 +1254,12 @@ Status run_single(Ctx &ctx, const HostGraph &data, const DevGraph &dg, const Pla
     if (rows) {
         res.count = L.tot_h->keep;
         res.rows.resize(res.count);
-        if (res.count)
-            HIP_TRY(hipMemcpy(res.rows.data(), a.rows, res.count * sizeof(uint32_t), hipMemcpyDeviceToHost));
+        Status st = ctx.ring.to_host(L.stream, res.rows.data(), a.rows, res.count * sizeof(uint32_t));
+        if (!st.good()) return st;
         if (o.flags & GFSM_DIGEST)
-            for (uint32_t x : res.rows) {
+            for (uint64_t r = 0; r < res.count; r++) {
                 uint64_t h[2];
-                row_hash(&x, 1, h);
+                row_hash(res.rows.data() + r, 1, h);
                 res.digest[0] += h[0];
                 res.digest[1] += h[1];
             }

@@ -90,6 +90,24 @@ struct Tuning {
     Tuning();
 };
 
+// Rows' way from the device into ordinary memory: through a few pinned pieces that
+// kernels on two streams fill and host threads empty.  (The runtime's own copy into
+// ordinary memory takes turns with itself: 54 MB 3.1 ms, into fresh pages 6.4,
+// against 1.1 and 1.9.  Pieces of 1, 2, 4 MiB: 1.14, 1.13, 1.29 ms; one stream 1.24; six
+// threads no faster, and two threads' pieces should not share a huge page.)
+struct CopyRing {
+    static constexpr size_t kSmall = 1u << 20, kPiece = 2u << 20, kSlots = 8, kThreads = 4;
+    char *mem = nullptr;  // pinned: kSmall bytes, or kSlots pieces once a table passes them
+    size_t size = 0;
+    hipStream_t second = nullptr;
+    hipEvent_t ev[kSlots] = {};
+    Status init(size_t bytes);
+    void destroy();
+    // dst[0, n) = src on the device (whole words, on a 16-byte boundary), after the
+    // work queued on `s`, which is idle on return.
+    Status to_host(hipStream_t s, void *dst, const void *src, size_t n);
+};
+
 struct Ctx {
     int device = 0;
     uint64_t budget = 0;
@@ -97,6 +115,7 @@ struct Ctx {
     uint32_t clock_khz = 100000;  // of the device clock (wall_clock64)
     uint64_t max_tiles = 0;
     Lane lane;
+    CopyRing ring;  // rows' way to the host
     Arena arena;
     Arena batch_arena;  // level regions of the batched path (grow-only, shared by its engines)
     Tuning tune;

@@ -5,6 +5,7 @@
 #include <atomic>
 #include <cstdint>
 #include <string>
+#include <utility>
 #include <vector>
 #include <mutex>
 #include <unordered_map>
@@ -142,42 +143,49 @@ Status gen_grid(uint32_t rows, uint32_t cols, double del_frac, double diag_frac,
                 HostGraph *&out);
 Status gen_query_walk(const HostGraph &data, uint32_t qsize, uint32_t kind, uint64_t seed, HostGraph *&out);
 
-// Host memory of embedding tables: pinned where the runtime gives it (the
-// device copies straight into it; a copy into pageable memory goes through the
-// runtime's staging), never filled before it is written.
-void *row_alloc(size_t bytes);
-void row_free(void *p);
-template <class T>
-struct RowAlloc {
-    using value_type = T;
-    RowAlloc() = default;
-    template <class U>
-    RowAlloc(const RowAlloc<U> &) {}
-    T *allocate(size_t n) { return static_cast<T *>(row_alloc(n * sizeof(T))); }
-    void deallocate(T *p, size_t) { row_free(p); }
-    template <class U>
-    void construct(U *p)
+// Words of an embedding table: grown without being filled (new ones are
+// unwritten), in place where large.
+class RowBuf {
+public:
+    RowBuf() = default;
+    RowBuf(RowBuf &&o) noexcept { swap(o); }
+    RowBuf &operator=(RowBuf &&o) noexcept
     {
-        ::new (static_cast<void *>(p)) U;  // not value-initialised: resize() leaves new rows unwritten
+        if (this != &o) {
+            clear();
+            swap(o);
+        }
+        return *this;
     }
-    template <class U, class... A>
-    void construct(U *p, A &&...a)
+    ~RowBuf() { clear(); }
+    void resize(size_t n);
+    void clear();  // gives the memory back
+    void swap(RowBuf &o) noexcept
     {
-        ::new (static_cast<void *>(p)) U(static_cast<A &&>(a)...);
+        std::swap(p_, o.p_);
+        std::swap(n_, o.n_);
+        std::swap(cap_, o.cap_);
     }
-    template <class U>
-    bool operator==(const RowAlloc<U> &) const { return true; }
-    template <class U>
-    bool operator!=(const RowAlloc<U> &) const { return false; }
+    uint32_t *data() { return p_; }
+    const uint32_t *data() const { return p_; }
+    size_t size() const { return n_; }
+    size_t capacity() const { return cap_; }
+    bool empty() const { return n_ == 0; }
+
+private:
+    uint32_t *p_ = nullptr;
+    size_t n_ = 0, cap_ = 0;
 };
-using RowVec = std::vector<uint32_t, RowAlloc<uint32_t>>;
+// Contexts open and close; memory kept for the next tables goes with the last.
+void row_pool_open();
+void row_pool_close();
 
 struct Result {
     gfsm_status status = GFSM_OK;
     uint64_t count = 0;
     uint64_t digest[2] = {0, 0};
     uint32_t width = 0;
-    RowVec rows;
+    RowBuf rows;
     gfsm_stats stats{};
 };
 

@@ -357,6 +357,10 @@ uint64_t sort_rows_bytes(uint64_t n, uint32_t q);
 hipError_t launch_sort_rows(const uint32_t *rows, uint64_t n, uint32_t q, uint32_t ncol, uint32_t bits, void *tmp,
                             uint32_t **sorted, hipStream_t s);
 
+// `words` words from the device to host memory that the device maps, both on a
+// 16-byte boundary.
+hipError_t launch_copy_out(const uint32_t *src, uint32_t *dst, uint64_t words, hipStream_t s);
+
 // Traffic calibration (kernels of known footprint).  mode 0: dst[i] =
 // src[i] + 1 over n words (n words read and written); mode 1: one word from
 // each of n distinct 128-byte lines of src (n a power of two, src holding 32n

@@ -2565,9 +2565,34 @@ __global__ void k_sort_gather(const uint32_t *rows, const uint32_t *idx, uint64_
     }
 }
 
+// Rows on their way to the host, bound by the link: 54 MiB whole 1.03 ms, in pieces
+// of 2 MiB on two streams with host threads emptying them 1.13 ms, 50 GB/s.  The
+// runtime's copies of the same pieces took 1.25 to 1.31 ms in most processes and 3.1 to
+// 4.7 in some, where whole copies ran at half the rate too.  (32 to 1,024
+// workgroups, and streaming stores: all within 5%.)
+constexpr uint32_t kCopyGrid = 64;
+__global__ __launch_bounds__(kTile) void k_copy_out(const uint32_t *__restrict__ src, uint32_t *__restrict__ dst,
+                                                    uint64_t words)
+{
+    const uint64_t i0 = (uint64_t)blockIdx.x * kTile + threadIdx.x;
+    const auto from = gp(reinterpret_cast<const u32x4 *>(src));
+    const auto to = gp(reinterpret_cast<u32x4 *>(dst));
+    for (uint64_t i = i0; i < words / 4; i += (uint64_t)gridDim.x * kTile) to[i] = from[i];
+    if (i0 < words % 4) dst[words / 4 * 4 + i0] = src[words / 4 * 4 + i0];
+}
+
 // ---------------------------------------------------------------------------
 // launch wrappers
 // ---------------------------------------------------------------------------
+
+hipError_t launch_copy_out(const uint32_t *src, uint32_t *dst, uint64_t words, hipStream_t s)
+{
+    if ((reinterpret_cast<uintptr_t>(src) | reinterpret_cast<uintptr_t>(dst)) & 15) return hipErrorInvalidValue;
+    const uint64_t wg = (words / 4 + kTile - 1) / kTile;
+    hipLaunchKernelGGL(k_copy_out, dim3((uint32_t)(wg < kCopyGrid ? (wg ? wg : 1) : kCopyGrid)), dim3(kTile), 0, s, src,
+                       dst, words);
+    return hipGetLastError();
+}
 
 static uint64_t sort_blocks(uint64_t n) { return (n + kSortBlock - 1) / kSortBlock; }
 static uint64_t up256(uint64_t b) { return (b + 255) / 256 * 256; }
