@@ -525,9 +525,9 @@ class Context:
         return t.as_dict()
 
     def set_tuning(self, **kw):
-        """Change launch shapes: items (int for all kinds/depths, or 3x32 lists),
-        pool_words, wgs_per_cu, batch_items, batch_pool_words, batch_wgs_per_cu,
-        batch_slots."""
+        """Change launch shapes: items (the most candidates per thread, int for all
+        kinds/depths, or 3x32 lists; small steps take fewer), pool_words, wgs_per_cu,
+        batch_items, batch_pool_words, batch_wgs_per_cu, batch_slots."""
         t = Tuning()
         _check(lib().gfsm_tuning_get(self._h, C.byref(t)), "tuning_get")
         for k, v in kw.items():

@@ -749,8 +749,8 @@ struct Runner {
         return lane.kc_h;
     }
 
-    // After a root or non-counting step: take its {keep, cnt} into tot_h,
-    // from the host words it wrote or by a copy.  With `early`, the host
+    // After a root or non-counting step: take its {keep, cnt} into tot_h
+    // from the host words it wrote.  With `early`, the host
     // takes them as soon as the step's last tile has published them, while
     // the step's other workgroups may still be finishing: only for steps whose
     // next use is a launch on the same stream (stream order makes it wait).
@@ -930,9 +930,9 @@ struct Runner {
         // registers under 64 for eight waves per SIMD).
         const bool bare = last && !rows_mode && !digest && plan.dev.depth[d].nchk == 0 &&
                           !(forced_items > kBareItems);
-        // The tail: every later depth is a leaf.  Deeper than its first depth
-        // only where a cap ended inside a tail step.
-        const bool at_tail = !last && d + 1 + leaves >= q;
+        // The tail: every later depth is a leaf.  (Once a cap has ended inside a tail
+        // step, `leaves` is 0 and the rest is expanded level by level.)
+        const bool at_tail = leaves && d + 1 + leaves == q;
         const TailPlanDev *tp = at_tail ? &plan.dev.tail[q - 2 - d] : nullptr;
         const uint32_t m = at_tail ? tp->m : 0u;
         const uint32_t inner_kind =

@@ -2011,7 +2011,7 @@ DEV uint32_t schedule_slot(const BatchCfg &cfg, BatchSlot &B, Totals *tot, const
 }
 
 // N words copied by the 64 lanes of one wave, each lane issuing 16 loads
-// before their stores (a slot is 748 words, a plan 2,594).
+// before their stores (a slot takes one such batch, a plan three).
 template <uint32_t N, class SP, class DP>
 DEV void wave_copy_words(DP dst, SP src, uint32_t lane)
 {
@@ -2046,6 +2046,7 @@ DEV void wave_sync_lds()
 // finish lays the slots' tiles end to end.
 constexpr uint32_t kSlotWords = sizeof(BatchSlot) / 4;
 constexpr uint32_t kPlanWords = sizeof(QueryPlanDev) / 4;
+static_assert(kSlotWords <= 1024 && kPlanWords <= 3 * 1024, "batches of wave_copy_words");
 // tile_start[s] between a slot's scheduling and the layout: its tile count,
 // whether it is running, and whether its step reads the tile index.
 constexpr uint64_t kSchedRun = 1ull << 63, kSchedIndexed = 1ull << 62;

@@ -26,7 +26,6 @@ struct DepthPlanDev {
     uint32_t inj;
     uint32_t chk_dist[GFSM_MAXCHK];
     uint32_t chk_rel[GFSM_MAXCHK];
-    uint32_t pad;
     // Dense segment tables ({begin, end} per data vertex, see DevGraph) of
     // nxt_rel and of the first four chk_rel, filled in per run where one
     // exists; null: the segment hash table.

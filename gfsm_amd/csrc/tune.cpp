@@ -5,6 +5,8 @@
 //   single-query path: candidates per thread x LDS staging pool x
 //                      persistent workgroups per CU,
 //   batch path:        the same three for the batch step kernel.
+// Candidates per thread are the most that a step takes: steps too small to fill the
+// GPU with such tiles take fewer under every shape.
 // Every shape computes the same result; only time is compared, as the best
 // of kRepeats runs per shape (one run is noisy at millisecond scale).
 #include <algorithm>

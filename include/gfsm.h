@@ -316,10 +316,11 @@ gfsm_status gfsm_selftest_traffic(gfsm_ctx *ctx, uint32_t mode, uint64_t n, uint
  * batch_steps: steps per captured replay; batch_step_budget: candidates one
  * step processes over all running queries (split evenly among them). */
 typedef struct gfsm_tuning {
-    uint32_t items[3][GFSM_MAX_Q];
+    uint32_t items[3][GFSM_MAX_Q]; /* most candidates per thread; steps too small to fill the GPU   */
+                                   /* with such tiles take fewer (gfsm_match_opts.tile forces one)  */
     uint32_t pool_words;
     uint32_t wgs_per_cu;
-    uint32_t batch_items;
+    uint32_t batch_items;        /* likewise; a quarter of it while few tiles are scheduled       */
     uint32_t batch_pool_words;
     uint32_t batch_wgs_per_cu;
     uint32_t batch_slots;
