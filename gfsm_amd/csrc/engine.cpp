@@ -72,28 +72,34 @@ Status CopyRing::to_host(hipStream_t s, void *dst, const void *src, size_t n)
     if (!st.good()) return st;
     char *const to = static_cast<char *>(dst);
     const char *const from = static_cast<const char *>(src);
-    if (n <= kPiece) {
+    if (n <= kMinPiece) {
         HIP_TRY(launch_copy_out(reinterpret_cast<const uint32_t *>(from), reinterpret_cast<uint32_t *>(mem), n / 4, s));
         HIP_TRY(hipStreamSynchronize(s));
         std::memcpy(to, mem, n);
         return Status::ok();
     }
-    HIP_TRY(hipStreamSynchronize(s));  // the copies run on two streams
+    // Up to kSmall bytes the calling thread empties the pieces of one stream; past
+    // them two streams and threads (their start costs 40 us, their end as much).
+    const bool small = n <= kSmall;
+    if (!small) HIP_TRY(hipStreamSynchronize(s));
+    size_t piece = kMinPiece;
+    while (piece < kPiece && piece * kSlots < n) piece *= 2;
     // Pieces end at multiples of their size in the table's memory, give or take the
-    // 16 bytes that the source is read by: two threads' pieces share no huge page.
-    size_t head = (kPiece - reinterpret_cast<uintptr_t>(to) % kPiece) & ~(size_t)15;
-    if (!head) head = kPiece;
+    // 16 bytes that the source is read by: large ones of two threads share no huge
+    // page.
+    size_t head = (piece - reinterpret_cast<uintptr_t>(to) % piece) & ~(size_t)15;
+    if (!head) head = piece;
     std::vector<size_t> at{0};
-    for (size_t e = head; e < n; e += kPiece) at.push_back(e);
-    // The last one in quarters: nothing overlaps its way out of the ring.
-    for (size_t e = at.back() + kPiece / 4; e < n; e += kPiece / 4) at.push_back(e);
+    for (size_t e = head; e < n; e += piece) at.push_back(e);
+    // The last large one in quarters: nothing overlaps its way out of the ring.
+    for (size_t e = at.back() + piece / 4; piece == kPiece && e < n; e += piece / 4) at.push_back(e);
     at.push_back(n);
     const size_t np = at.size() - 1;
     std::atomic<size_t> ready{0}, next{0}, freed[kSlots];  // pieces landed; taken; per slot, past its last piece done
     std::atomic<bool> stop{false};
     for (auto &f : freed) f.store(0, std::memory_order_relaxed);
     const auto out = [&](size_t k) {
-        std::memcpy(to + at[k], mem + k % kSlots * kPiece, at[k + 1] - at[k]);
+        std::memcpy(to + at[k], mem + k % kSlots * piece, at[k + 1] - at[k]);
         freed[k % kSlots].store(k + 1, std::memory_order_release);
     };
     const auto work = [&] {
@@ -112,9 +118,9 @@ Status CopyRing::to_host(hipStream_t s, void *dst, const void *src, size_t n)
     };
     const auto issue = [&]() -> hipError_t {
         const size_t k = issued++, sl = k % kSlots;
-        const hipStream_t q = k & 1 ? second : s;
+        const hipStream_t q = k & 1 && !small ? second : s;
         const hipError_t e = launch_copy_out(reinterpret_cast<const uint32_t *>(from + at[k]),
-                                             reinterpret_cast<uint32_t *>(mem + sl * kPiece), (at[k + 1] - at[k]) / 4, q);
+                                             reinterpret_cast<uint32_t *>(mem + sl * piece), (at[k + 1] - at[k]) / 4, q);
         return e == hipSuccess ? hipEventRecord(ev[sl], q) : e;
     };
     hipError_t err = hipSuccess;
@@ -122,7 +128,7 @@ Status CopyRing::to_host(hipStream_t s, void *dst, const void *src, size_t n)
     std::vector<std::thread> th;
     try {
         th.reserve(kThreads);
-        while (th.size() < std::min<size_t>(kThreads, np)) th.emplace_back(work);
+        while (!small && th.size() < kThreads) th.emplace_back(work);
     } catch (const std::exception &) {  // no more threads: those there are, or this one
     }
     for (size_t k = 0; k < np && err == hipSuccess; k++) {

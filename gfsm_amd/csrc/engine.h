@@ -91,13 +91,17 @@ struct Tuning {
 };
 
 // Rows' way from the device into ordinary memory: through a few pinned pieces that
-// kernels on two streams fill and host threads empty.  (The runtime's own copy into
-// ordinary memory takes turns with itself: 54 MB 3.1 ms, into fresh pages 6.4,
-// against 1.1 and 1.9.  Pieces of 1, 2, 4 MiB: 1.14, 1.13, 1.29 ms; one stream 1.24; six
-// threads no faster, and two threads' pieces should not share a huge page.)
+// kernels fill and the host empties, large tables on two streams and with host threads.
+// (The runtime's own copy into ordinary memory takes turns with itself: 54 MB 3.1 ms,
+// into fresh pages 6.4, against 1.1 and 1.9.  Pieces of 1, 2, 4 MiB: 1.14, 1.13, 1.29 ms;
+// one stream 1.24; six threads no faster, and two threads' pieces should not share a
+// huge page.  A call and the first read of its rows, results kept, against pinned
+// blocks: 0.26 MB 0.27 -> 0.11 ms, 2 MB 0.98 -> 0.24, 33 MB 12.9 -> 2.1; dropped 0.11 /
+// 0.11, 0.22 / 0.22, 1.6 / 1.7.)
 struct CopyRing {
-    static constexpr size_t kSmall = 1u << 20, kPiece = 2u << 20, kSlots = 8, kThreads = 4;
-    char *mem = nullptr;  // pinned: kSmall bytes, or kSlots pieces once a table passes them
+    static constexpr size_t kMinPiece = 256u << 10, kPiece = 2u << 20, kSlots = 8, kThreads = 4;
+    static constexpr size_t kSmall = kSlots * kMinPiece;
+    char *mem = nullptr;  // pinned: kSmall bytes, or kSlots large pieces once a table passes them
     size_t size = 0;
     hipStream_t second = nullptr;
     hipEvent_t ev[kSlots] = {};

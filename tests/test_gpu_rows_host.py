@@ -30,8 +30,8 @@ def _want(roots):
     return np.stack([np.stack([a, v, b], 1), np.stack([b, v, a], 1)], 1).reshape(-1, 3).astype(np.uint32)
 
 
-# 24 bytes a root: around the sizes of one small, one and four large pieces, past them
-@pytest.mark.parametrize("bytes_", [24, MIB, 4 * MIB, 8 * MIB, 16 * MIB, 20 * MIB, 90 * MIB])
+# 24 bytes a root: around one and eight small pieces, the pieces between, eight large ones, past them
+@pytest.mark.parametrize("bytes_", [24, MIB // 4, MIB, 2 * MIB, 4 * MIB, 8 * MIB, 16 * MIB, 20 * MIB, 90 * MIB])
 def test_rows(ctx, ring, path3, tmp_path, bytes_):
     for roots in sorted({bytes_ // 24, bytes_ // 24 + 1}):
         want = _want(roots)
