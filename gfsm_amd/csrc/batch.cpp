@@ -267,6 +267,13 @@ Status BatchEngine::init(const BatchShape &shape, uint64_t arena_bytes, char *ar
     cfg_.pool_words = shape_.pool_words;
     cfg_.max_step_cand = shape_.step_budget;
     cfg_.max_degree = std::max<uint32_t>(data_.max_degree, 1);
+    // A step's sums of m leaves: at most its candidates times degree^m.
+    cfg_.big_tails = 0;
+    for (uint32_t m = 1; m <= GFSM_MAXTAIL; m++) {
+        unsigned __int128 most = std::max<uint64_t>(cfg_.max_step_cand, (uint64_t)kTile * shape_.items);
+        for (uint32_t i = 0; i < m; i++) most *= cfg_.max_degree;  // < 2^26 each
+        if (most >> 64) cfg_.big_tails |= 1u << m;
+    }
     cfg_.g = dg_->view;
     cfg_.ws = lane_.ws;
     grid_ = std::max<uint32_t>(ctx_.num_cus, 1) * std::max<uint32_t>(shape_.wgs_per_cu, 1);

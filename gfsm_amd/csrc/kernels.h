@@ -302,7 +302,7 @@ struct BatchCfg {
     uint32_t pool_words;
     uint32_t pad;
     uint64_t tile_room;           // tiles of one step (tail_sums)
-    uint32_t pad2;
+    uint32_t big_tails;           // bit m: the sums of a step of m leaves can pass 2^64
     uint32_t fill_tiles;          // tiles that fill the GPU (the step kernel's workgroups)
     uint64_t max_step_cand;       // upper bound of BatchCtl::step_cand (workspace size)
     uint64_t max_degree;          // of the data graph (scan value bound)

@@ -1729,21 +1729,12 @@ DEV uint64_t capped_chunk(const BatchSlot &B, uint32_t d, uint64_t n, uint64_t c
 // candidates fit the caps, and how many tiles those are.
 struct TailSums {
     uint64_t sum[2 * GFSM_MAXTAIL + 1], tiles;
-    uint32_t over;  // bit i: sum[i] passed 2^64
+    bool over;  // the count passed 2^64 - 1 (the other sums stay there)
 };
 
-// The sum of v (at most 2^62) over a wave; *over: it passed 2^64.
-DEV uint64_t wave_sum_over(uint64_t v, bool *over)
-{
-    *over = false;
-    if (!__any((v >> 57) != 0)) return wave_sum64(v);
-    const uint64_t lo = wave_sum64(v & 0xFFFFFFFFull), hi = wave_sum64(v >> 32) + (lo >> 32);
-    *over = hi >> 32;
-    return hi << 32 | (lo & 0xFFFFFFFFull);
-}
-
-// The sums of the tail step of slot B, by all 64 lanes of one wave.
-DEV TailSums wave_tail_sums(gptr_t<const uint64_t> sums, const BatchSlot &B)
+// The sums of the tail step of slot B, by all 64 lanes of one wave.  `big`: see
+// BatchCfg.
+DEV TailSums wave_tail_sums(gptr_t<const uint64_t> sums, const BatchSlot &B, uint32_t big)
 {
     const uint32_t lane = lane_id(), m = B.tail;
     const uint64_t n = B.io.ntiles;
@@ -1766,14 +1757,21 @@ DEV TailSums wave_tail_sums(gptr_t<const uint64_t> sums, const BatchSlot &B)
         if (B.max_cand) fit = fit && all <= B.max_cand - umin64(B.max_cand, B.cand_done);
         if (B.max_depth_cand || B.max_cand) fit = fit && all != ~0ull;  // (a saturated sum fits no cap)
         const uint64_t mask = __ballot(fit);
+        if (!((big >> m) & 1u)) {
 #pragma unroll
-        for (uint32_t i = 0; i < 2 * GFSM_MAXTAIL + 1; i++)
-            if (i < 2 * m + 1) {
-                bool over;
-                const uint64_t v = wave_sum_over(fit ? sums[kTailWords * t + i] : 0ull, &over);
-                r.sum[i] += v;
-                r.over |= (over || r.sum[i] < v) ? 1u << i : 0u;
+            for (uint32_t i = 0; i < 2 * GFSM_MAXTAIL + 1; i++)
+                if (i < 2 * m + 1) r.sum[i] += wave_sum64(fit ? sums[kTailWords * t + i] : 0ull);
+        } else {
+            // A tile's sum is under 2^62: two halves' sums over a wave fit.
+            for (uint32_t i = 0; i < 2 * m + 1; i++) {
+                const uint64_t x = fit ? sums[kTailWords * t + i] : 0ull;
+                const uint64_t lo = wave_sum64(x & 0xFFFFFFFFull), hi = wave_sum64(x >> 32) + (lo >> 32);
+                const uint64_t v = hi << 32 | (lo & 0xFFFFFFFFull), s = r.sum[i] + v;
+                const bool over = (hi >> 32) || s < v;
+                r.sum[i] = over ? ~0ull : s;
+                if (i == 2 * m) r.over = r.over || over;
             }
+        }
         r.tiles += (uint64_t)__popcll(mask);
         if (mask != ~0ull) break;  // the tiles that fit are the first ones
     }
@@ -1880,14 +1878,13 @@ DEV uint32_t schedule_slot(const BatchCfg &cfg, BatchSlot &B, Totals *tot, const
             B.level[d] += ts.sum[0];
             // Statistics past 2^64 stay at the largest number; a count there ends
             // the match.
-            const auto sum = [&](uint32_t i) { return (ts.over >> i) & 1u ? ~0ull : ts.sum[i]; };
             for (uint32_t i = 0; i < m; i++) {
-                B.cand[d + 1 + i] = add_sat(B.cand[d + 1 + i], sum(1 + 2 * i));
-                B.level[d + 1 + i] = add_sat(B.level[d + 1 + i], sum(2 + 2 * i));
-                B.cand_done = add_sat(B.cand_done, sum(1 + 2 * i));
+                B.cand[d + 1 + i] = add_sat(B.cand[d + 1 + i], ts.sum[1 + 2 * i]);
+                B.level[d + 1 + i] = add_sat(B.level[d + 1 + i], ts.sum[2 + 2 * i]);
+                B.cand_done = add_sat(B.cand_done, ts.sum[1 + 2 * i]);
             }
             B.count += ts.sum[2 * m];
-            if (((ts.over >> (2 * m)) & 1u) || B.count < ts.sum[2 * m]) {
+            if (ts.over || B.count < ts.sum[2 * m]) {
                 B.state = SLOT_OVER;
                 B.step = STEP_NONE;
                 return 0;
@@ -2088,7 +2085,7 @@ __global__ __launch_bounds__(kTile) void k_batch_schedule(BatchCfg cfg)
         uint32_t fin = 0;
         TailSums ts{};
         if (B.state == SLOT_RUN && B.step == EXPAND_TAIL)
-            ts = wave_tail_sums(gp((const uint64_t *)cfg.tail_sums) + kTailWords * B.tile0, B);
+            ts = wave_tail_sums(gp((const uint64_t *)cfg.tail_sums) + kTailWords * B.tile0, B, cfg.big_tails);
         if (lane == 0) {
             const uint32_t before = B.state;
             const uint32_t nt = schedule_slot(cfg, B, &cfg.slots[s].tot, ts);
