@@ -12,10 +12,11 @@ the deterministic per-depth candidate cap, and the fixed tail window, exact;
 embeddings counted on the device.  The data graph is resident in HBM before
 the timed region.  Reported beside it: rates per stratum, the share of the
 workload's roots and depth-1 candidates the sample covers, the roofline of
-the dominant kernel (the expand kernel: algorithmic bytes per launch / mean
-launch time, timed with HIP events on the matcher's stream inside the timed
-region), and the CPU oracle on complete windows of the same sample on this
-host's cores.
+the dominant kernel (the expand kernels: HBM bytes per launch, from recorded
+counters, over the mean launch time, timed with HIP events on the matcher's
+stream inside the timed region; and the same of the algorithmic bytes, an
+equivalent rate, since counted leaves are answered for without being read),
+and the CPU oracle on complete windows of the same sample on this host's cores.
 
 grid: the road-like workload (1400 x 1400 damaged grid; C4, C6, P7, 3x3
 patch over every root), per-query embeddings/s and the expand roofline.
@@ -69,19 +70,20 @@ def calibrate(mode):
     print(json.dumps({"calibrate": mode, "launches": 5, "read_bytes_per_launch": rd, "write_bytes_per_launch": wr}))
 
 
-def traffic_from_profiles():
-    """HBM bytes per expand launch of the timed sample, measured with rocprofv3
-    FETCH_SIZE/WRITE_SIZE and scaled by the gather calibration
-    (profiles/expand_config2_traffic.json), and where that figure comes from;
-    (None, None) when not recorded.  Counters need a profiler run of their
-    own, so the figure is not measured in the run that prints it."""
+def traffic_from_profiles(key="hbm_bytes_per_launch"):
+    """HBM bytes per expand launch of the timed sample (or, by its key, of the
+    grid section), measured with rocprofv3 FETCH_SIZE/WRITE_SIZE and scaled by
+    the gather calibration (profiles/expand_config2_traffic.json), and where
+    that figure comes from; (None, None) when not recorded.  Counters need a
+    profiler run of their own, so the figure is not measured in the run that
+    prints it."""
     path = os.path.join(ROOT, "profiles", "expand_config2_traffic.json")
     try:
         with open(path) as f:
             rec = json.load(f)
         src = (f"rocprofv3 FETCH_SIZE x {rec['fetch_factor']} + WRITE_SIZE x {rec['write_factor']} per expand "
                f"launch of this sample on commit {rec['commit']} ({rec['source']}); not measured in this run")
-        return float(rec["hbm_bytes_per_launch"]), src
+        return float(rec[key]), src
     except (OSError, KeyError, ValueError):
         return None, None
 
@@ -305,12 +307,32 @@ def serve_section(n):
     }
 
 
-def expand_roofline(alg, kms, launches):
-    """Algorithmic bytes per expand launch over the mean launch time."""
-    per_launch = alg / max(launches, 1)
-    mean_ms = kms / max(launches, 1)
-    achieved = per_launch / (mean_ms / 1e3) / 1e9 if mean_ms else 0.0
-    return achieved, mean_ms, per_launch
+def expand_rate(alg, kms, launches):
+    """Algorithmic GB/s of the expand launches (an equivalent rate where leaves are
+    counted without being read) and the mean launch time."""
+    return alg / (kms / 1e3) / 1e9 if kms else 0.0, kms / max(launches, 1)
+
+
+def expand_roofline(alg, kms, launches, steps, key="hbm_bytes_per_launch"):
+    equivalent, mean_ms = expand_rate(alg, kms, launches)
+    traffic, source = traffic_from_profiles(key)
+    achieved = traffic / (mean_ms / 1e3) / 1e9 if traffic and mean_ms else None
+    return {
+        "bound": "hbm",
+        "achieved": achieved,
+        "peak": HBM_PEAK_GBS,
+        "unit": "GB/s",
+        "frac": achieved / HBM_PEAK_GBS if achieved else None,
+        "equivalent": equivalent,
+        "equivalent_note": "algorithmic bytes over the same time; candidates of counted leaves are in them, "
+                           "though not read one by one",
+        "traffic": traffic,
+        "traffic_source": source,
+        "kernel": "gfsm::k_expand (inner depths) + gfsm::k_expand_tail (counted leaves) + "
+                  "gfsm::k_expand_bare (last depth)",
+        "launches": launches // steps,
+        "mean_launch_ms": mean_ms,
+    }
 
 
 def grid_section(steps):
@@ -340,22 +362,19 @@ def grid_section(steps):
             launches += st["expand_launches"]
             chunks = st["chunks"]
         wall = (time.perf_counter() - t0) / steps
-        ach, mean_ms, _ = expand_roofline(alg, kms, launches)
         out[name] = {"embeddings": emb, "candidates": cand, "ms": wall * 1e3, "embeddings_per_s": emb / wall,
                      "expand_launches": launches // steps, "chunked_launches": chunks,
-                     "expand_achieved_gbs": ach, "expand_frac": ach / HBM_PEAK_GBS}
+                     "expand_equivalent_gbs": expand_rate(alg, kms, launches)[0]}
         tot_alg += alg
         tot_kms += kms
         tot_l += launches
     ctx.close()
-    ach, mean_ms, _ = expand_roofline(tot_alg, tot_kms, tot_l)
     return {
         "workload": "road-like: 1400 x 1400 grid, 5% of edges deleted, 2% diagonals added, unlabeled; "
                     "C4, C6, P7, 3x3 patch, every root, count mode (chunked expansion)",
         "queries": out,
         "embeddings_per_s": sum(v["embeddings"] for v in out.values()) / sum(v["ms"] / 1e3 for v in out.values()),
-        "roofline": {"bound": "hbm", "achieved": ach, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": ach / HBM_PEAK_GBS, "launches": tot_l // steps, "mean_launch_ms": mean_ms},
+        "roofline": expand_roofline(tot_alg, tot_kms, tot_l, steps, "grid_hbm_bytes_per_launch"),
     }
 
 
@@ -416,7 +435,6 @@ def main():
     alg = sum(a["alg"] for a in acc.values())
     kms = sum(a["kms"] for a in acc.values())
     launches = sum(a["launches"] for a in acc.values())
-    achieved, mean_ms, _ = expand_roofline(alg, kms, launches)
     # coverage of the whole workload (every root of every query)
     roots_total = first_total = 0
     for q in queries:
@@ -425,11 +443,10 @@ def main():
         first_total += int(cand[1])
     per = {}
     for sname, a in acc.items():
-        ach, mms, _ = expand_roofline(a["alg"], a["kms"], a["launches"])
         per[sname] = {"embeddings_per_step": a["emb"] // K, "candidates_per_step": a["cand"] // K,
                       "ms_per_step": a["s"] * 1e3 / K, "embeddings_per_s": a["emb"] / a["s"] if a["s"] else 0.0,
                       "candidates_per_s": a["cand"] / a["s"] if a["s"] else 0.0,
-                      "expand_achieved_gbs": ach, "expand_frac": ach / HBM_PEAK_GBS,
+                      "expand_equivalent_gbs": expand_rate(a["alg"], a["kms"], a["launches"])[0],
                       "roots_tested": a["roots"] // K, "capped_windows": a["capped"] // K}
     roots_tested = sum(a["roots"] for a in acc.values()) // K
     first_tested = sum(a["first"] for a in acc.values()) // K
@@ -466,21 +483,9 @@ def main():
             "strata": per,
         },
         "queries_per_s": len(sample) * K / wall,
-        "roofline": {
-            "bound": "hbm",
-            "achieved": achieved,
-            "peak": HBM_PEAK_GBS,
-            "unit": "GB/s",
-            "frac": achieved / HBM_PEAK_GBS,
-            "traffic": None,
-            "kernel": "gfsm::k_expand (inner depths) + gfsm::k_expand_tail (counted leaves) + "
-                      "gfsm::k_expand_bare (last depth)",
-            "launches": launches // K,
-            "mean_launch_ms": mean_ms,
-        },
+        "roofline": expand_roofline(alg, kms, launches, K),
     }
     ctx.close()
-    line["roofline"]["traffic"], line["roofline"]["traffic_source"] = traffic_from_profiles()
     line["cpu_baseline"] = None if args.no_cpu else cpu_baseline(data, queries, sample, win_s)
     if "grid" in sections:
         line["grid"] = grid_section(max(1, min(K, 3)))
