@@ -38,15 +38,20 @@ static double now_ms()
         if (e_ != hipSuccess) return hip_status(e_, #expr);              \
     } while (0)
 
-Status CopyRing::init(size_t bytes)
+bool CopyRing::init(size_t bytes)
 {
-    if (bytes <= size) return Status::ok();
+    if (bytes <= size) return true;
     destroy();
-    HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&mem), bytes, hipHostMallocDefault));
-    size = bytes;
-    HIP_TRY(hipStreamCreateWithFlags(&second, hipStreamNonBlocking));
-    for (auto &e : ev) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    return Status::ok();
+    bool ok = hipHostMalloc(reinterpret_cast<void **>(&mem), bytes, hipHostMallocDefault) == hipSuccess &&
+              hipStreamCreateWithFlags(&second, hipStreamNonBlocking) == hipSuccess;
+    for (auto &e : ev) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+    if (ok) {
+        size = bytes;
+    } else {
+        destroy();
+        (void)hipGetLastError();
+    }
+    return ok;
 }
 
 void CopyRing::destroy()
@@ -68,8 +73,11 @@ Status CopyRing::to_host(hipStream_t s, void *dst, const void *src, size_t n)
         HIP_TRY(hipStreamSynchronize(s));
         return Status::ok();
     }
-    Status st = init(n <= kSmall ? kSmall : kSlots * kPiece);
-    if (!st.good()) return st;
+    if (!init(n <= kSmall ? kSmall : kSlots * kPiece)) {  // no pinned memory: the runtime's way
+        HIP_TRY(hipStreamSynchronize(s));
+        HIP_TRY(hipMemcpy(dst, src, n, hipMemcpyDeviceToHost));
+        return Status::ok();
+    }
     char *const to = static_cast<char *>(dst);
     const char *const from = static_cast<const char *>(src);
     if (n <= kMinPiece) {

@@ -105,7 +105,7 @@ struct CopyRing {
     size_t size = 0;
     hipStream_t second = nullptr;
     hipEvent_t ev[kSlots] = {};
-    Status init(size_t bytes);
+    bool init(size_t bytes);
     void destroy();
     // dst[0, n) = src on the device (whole words, on a 16-byte boundary), after the
     // work queued on `s`, which is idle on return.
