@@ -56,6 +56,7 @@ bool CopyRing::init(size_t bytes)
 
 void CopyRing::destroy()
 {
+    crew.stop();
     if (mem) (void)hipHostFree(mem);
     if (second) (void)hipStreamDestroy(second);
     for (auto &e : ev) {
@@ -65,6 +66,80 @@ void CopyRing::destroy()
     mem = nullptr;
     second = nullptr;
     size = 0;
+}
+
+// A table on its way out of the ring.  Pieces are taken in order, once they have
+// landed, by whoever is free; the calling thread waits for pieces, not for
+// threads, so one that wakes late finds nothing left.
+struct CopyJob {
+    char *to;
+    const char *mem;
+    size_t piece;
+    std::vector<size_t> at;  // the pieces' bounds in the table
+    std::atomic<size_t> ready{0}, next{0}, done{0};  // pieces landed; taken; copied
+    std::atomic<size_t> freed[CopyRing::kSlots];     // per slot, past its last copied piece
+    size_t pieces() const { return at.size() - 1; }
+
+    // Copies one landed piece that nobody has taken; false where there is none.
+    bool one()
+    {
+        size_t k = next.load(std::memory_order_relaxed);
+        if (k >= ready.load(std::memory_order_acquire) || !next.compare_exchange_strong(k, k + 1)) return false;
+        std::memcpy(to + at[k], mem + k % CopyRing::kSlots * piece, at[k + 1] - at[k]);
+        freed[k % CopyRing::kSlots].store(k + 1, std::memory_order_release);
+        done.fetch_add(1, std::memory_order_release);
+        return true;
+    }
+    void help()
+    {
+        for (uint32_t i = 1; next.load(std::memory_order_relaxed) < pieces(); i++) {
+            if (one()) continue;
+            __builtin_ia32_pause();
+            if ((i & 1023) == 0) std::this_thread::yield();
+        }
+    }
+};
+
+void CopyCrew::start(size_t n)
+{
+    try {
+        while (threads.size() < n)
+            threads.emplace_back([this] {
+                std::unique_lock<std::mutex> lk(mu);
+                for (uint64_t seen = 0;;) {
+                    cv.wait(lk, [&] { return quit || turn != seen; });
+                    if (quit) return;
+                    seen = turn;
+                    const std::shared_ptr<CopyJob> j = job;
+                    lk.unlock();
+                    if (j) j->help();
+                    lk.lock();
+                }
+            });
+    } catch (const std::exception &) {  // those there are, or the calling thread alone
+    }
+}
+
+void CopyCrew::post(const std::shared_ptr<CopyJob> &j)
+{
+    {
+        std::lock_guard<std::mutex> lk(mu);
+        job = j;
+        turn++;
+    }
+    if (j) cv.notify_all();
+}
+
+void CopyCrew::stop()
+{
+    {
+        std::lock_guard<std::mutex> lk(mu);
+        quit = true;
+    }
+    cv.notify_all();
+    for (auto &t : threads) t.join();
+    threads.clear();
+    quit = false;
 }
 
 Status CopyRing::to_host(hipStream_t s, void *dst, const void *src, size_t n)
@@ -86,44 +161,33 @@ Status CopyRing::to_host(hipStream_t s, void *dst, const void *src, size_t n)
         std::memcpy(to, mem, n);
         return Status::ok();
     }
-    // Up to kSmall bytes the calling thread empties the pieces of one stream; past
-    // them two streams and threads (their start costs 40 us, their end as much).
-    const bool small = n <= kSmall;
-    if (!small) HIP_TRY(hipStreamSynchronize(s));
-    size_t piece = kMinPiece;
+    const std::shared_ptr<CopyJob> job = std::make_shared<CopyJob>();
+    CopyJob &j = *job;
+    j.to = to;
+    j.mem = mem;
+    for (auto &f : j.freed) f.store(0, std::memory_order_relaxed);
+    size_t &piece = j.piece = kMinPiece;
     while (piece < kPiece && piece * kSlots < n) piece *= 2;
+    if (piece * kSlots > size) return Status::err(GFSM_ERR_DEVICE, "internal: copy ring shape check failed");
     // Pieces end at multiples of their size in the table's memory, give or take the
     // 16 bytes that the source is read by: large ones of two threads share no huge
     // page.
     size_t head = (piece - reinterpret_cast<uintptr_t>(to) % piece) & ~(size_t)15;
     if (!head) head = piece;
-    std::vector<size_t> at{0};
+    std::vector<size_t> &at = j.at;
+    at.push_back(0);
     for (size_t e = head; e < n; e += piece) at.push_back(e);
     // The last large one in quarters: nothing overlaps its way out of the ring.
     for (size_t e = at.back() + piece / 4; piece == kPiece && e < n; e += piece / 4) at.push_back(e);
     at.push_back(n);
-    const size_t np = at.size() - 1;
-    std::atomic<size_t> ready{0}, next{0}, freed[kSlots];  // pieces landed; taken; per slot, past its last piece done
-    std::atomic<bool> stop{false};
-    for (auto &f : freed) f.store(0, std::memory_order_relaxed);
-    const auto out = [&](size_t k) {
-        std::memcpy(to + at[k], mem + k % kSlots * piece, at[k + 1] - at[k]);
-        freed[k % kSlots].store(k + 1, std::memory_order_release);
-    };
-    const auto work = [&] {
-        for (size_t k; (k = next.fetch_add(1, std::memory_order_relaxed)) < np;) {
-            for (uint32_t i = 1; ready.load(std::memory_order_acquire) <= k; i++) {
-                if (stop.load(std::memory_order_relaxed)) return;
-                __builtin_ia32_pause();
-                if ((i & 1023) == 0) std::this_thread::yield();
-            }
-            out(k);
-        }
-    };
+    const size_t np = j.pieces();
+    // Past kSmall bytes a second stream and other threads take part.
+    const bool small = n <= kSmall;
+    if (!small) {
+        HIP_TRY(hipStreamSynchronize(s));
+        crew.start(kThreads);
+    }
     size_t issued = 0;
-    const auto slot_free = [&](size_t k) {
-        return k < kSlots || freed[k % kSlots].load(std::memory_order_acquire) == k - kSlots + 1;
-    };
     const auto issue = [&]() -> hipError_t {
         const size_t k = issued++, sl = k % kSlots;
         const hipStream_t q = k & 1 && !small ? second : s;
@@ -131,27 +195,25 @@ Status CopyRing::to_host(hipStream_t s, void *dst, const void *src, size_t n)
                                              reinterpret_cast<uint32_t *>(mem + sl * piece), (at[k + 1] - at[k]) / 4, q);
         return e == hipSuccess ? hipEventRecord(ev[sl], q) : e;
     };
-    hipError_t err = hipSuccess;
+    hipError_t err = issue();
+    if (!small) crew.post(job);
     while (err == hipSuccess && issued < np && issued < kSlots) err = issue();
-    std::vector<std::thread> th;
-    try {
-        th.reserve(kThreads);
-        while (!small && th.size() < kThreads) th.emplace_back(work);
-    } catch (const std::exception &) {  // no more threads: those there are, or this one
-    }
     for (size_t k = 0; k < np && err == hipSuccess; k++) {
         err = hipEventSynchronize(ev[k % kSlots]);
         if (err != hipSuccess) break;
-        ready.store(k + 1, std::memory_order_release);
-        if (th.empty()) out(k);
+        j.ready.store(k + 1, std::memory_order_release);
+        if (small) (void)j.one();
         while (err == hipSuccess && issued < np && issued <= k + kSlots) {
-            if (slot_free(issued)) err = issue();
+            if (j.freed[issued % kSlots].load(std::memory_order_acquire) == issued - kSlots + 1) err = issue();
             else if (issued > k + 1) break;  // others are on their way
-            else __builtin_ia32_pause();
+            else if (!j.one()) __builtin_ia32_pause();
         }
     }
-    if (err != hipSuccess) stop = true;
-    for (auto &t : th) t.join();
+    if (err == hipSuccess) j.help();
+    // Nothing is taken from here on; what was taken is waited for.
+    const size_t taken = std::min(j.next.exchange(np), np);
+    while (j.done.load(std::memory_order_acquire) < taken) __builtin_ia32_pause();
+    if (!small) crew.post(nullptr);
     if (err != hipSuccess) {
         (void)hipStreamSynchronize(s);
         (void)hipStreamSynchronize(second);

@@ -4,10 +4,12 @@
 #include <hip/hip_runtime_api.h>
 
 #include <atomic>
+#include <condition_variable>
 #include <cstdio>
 #include <memory>
 #include <mutex>
 #include <set>
+#include <thread>
 #include <unordered_map>
 
 #include "host.h"
@@ -98,6 +100,20 @@ struct Tuning {
 // huge page.  A call and the first read of its rows, results kept, against pinned
 // blocks: 0.26 MB 0.27 -> 0.11 ms, 2 MB 0.98 -> 0.24, 33 MB 12.9 -> 2.1; dropped 0.11 /
 // 0.11, 0.22 / 0.22, 1.6 / 1.7.)
+struct CopyJob;
+// Host threads that help one caller at a time to empty its ring, asleep between tables
+// (started for each table: 3 MB 258 against 232 us a call, 54 MB 1.46 against 1.42 ms).
+struct CopyCrew {
+    std::mutex mu;
+    std::condition_variable cv;
+    std::shared_ptr<CopyJob> job;
+    uint64_t turn = 0;
+    bool quit = false;
+    std::vector<std::thread> threads;
+    void start(size_t n);
+    void post(const std::shared_ptr<CopyJob> &j);  // null: no job
+    void stop();
+};
 struct CopyRing {
     static constexpr size_t kMinPiece = 256u << 10, kPiece = 2u << 20, kSlots = 8, kThreads = 4;
     static constexpr size_t kSmall = kSlots * kMinPiece;
@@ -105,6 +121,7 @@ struct CopyRing {
     size_t size = 0;
     hipStream_t second = nullptr;
     hipEvent_t ev[kSlots] = {};
+    CopyCrew crew;
     bool init(size_t bytes);
     void destroy();
     // dst[0, n) = src on the device (whole words, on a 16-byte boundary), after the
